@@ -137,6 +137,7 @@ struct KParams {
     uint32_t cap;         /* LDS walk capacity (steps per half ray) */
     uint32_t nslots;      /* number of 32-lane line slots = L * ceil(Q/32) */
     uint32_t slots_per_line;
+    uint32_t stage;       /* forward solve: entries a group of 32 lanes stages at a time */
     uint32_t j_lds;       /* forward solve: 1 = J accumulated in LDS, 0 = in the output row */
     uint32_t *status;     /* [0] error bits, [1] walk capacity needed, [2] adjoint segments needed */
 };
@@ -408,6 +409,20 @@ __device__ inline uint32_t n_interp_for_line(const KParams &kp, uint32_t l, uint
     return (k > 1) ? k : 1;
 }
 
+/* all-lines interpolation count (InterpHelper::get_n_interp, :10-46) */
+__device__ inline uint32_t n_interp_all(const KParams &kp, uint32_t c, uint32_t n)
+{
+    const uint32_t L = kp.m.nlines;
+    double mx = 0.0;
+    for (uint32_t l = 0; l < L; l++) {
+        const double d = (double)fabsf(mgx_ref_logf((float)(kp.m.interp_crit[(size_t)n * L + l] /
+                                                        kp.m.interp_crit[(size_t)c * L + l])));
+        if (l == 0 || mx < d) mx = d;
+    }
+    const uint32_t k = (uint32_t)ceil(mx / kp.log_max_interp);
+    return (k > 1) ? k : 1;
+}
+
 /* float transcendentals: in FP64 mode the reference's own (the C library's
    expf and powf, restated in mgx_fmath_ref.h), in mixed mode the hardware
    single-precision functions */
@@ -446,7 +461,7 @@ __device__ inline double interp_linear(double a, double b, double t)
    so that its registers do not count against the solve's loop (with the reference's
    double-internal powf inline, the FP64 forward kernel spilled 40 VGPRs) */
 template <int PREC>
-__device__ __attribute__((noinline)) double interp_log_pow(double a, double b, double t)
+__device__ __forceinline__ double interp_log_pow(double a, double b, double t)
 {
     return a * (double)f_pow<PREC>((float)(b / a), (float)t);
 }
@@ -554,9 +569,11 @@ struct OwnLine {
 __device__ inline OwnLine own_line(const mgx_model &m, uint32_t l)
 {
     OwnLine r;
-    uint32_t g = 0;
-    for (uint32_t s = 0; s < m.nlines; s++)
-        if (gld(&m.sorted_line_map[s]) == l) g = s;
+    /* lines given in ascending order sit at their own place */
+    uint32_t g = l;
+    if (gld(&m.sorted_line_map[l]) != l)
+        for (uint32_t s = 0; s < m.nlines; s++)
+            if (gld(&m.sorted_line_map[s]) == l) g = s;
     r.g = g;
     r.lidx = gld(&m.sorted_line_map[g]);
     r.f_own = gld(&m.line[r.lidx]);
@@ -860,34 +877,73 @@ __device__ inline double hi_advance(const KParams &kp, HalfIter &it, uint32_t l,
 /* ------------------------------------------------------------------------- */
 /* the forward-solve kernel                                                   */
 
-/* LDS layout of the walk buffers of both half rays plus the per-pass
-   interpolation-count tables (2 lines x 2 halves x cap u16) */
+#include "mgx_staged.h"
+
+/* LDS layout of the walk buffers of both half rays (point, length, shift per step)
+   plus 16 bytes a step for interpolation counts: four tables (2 lines x 2 halves)
+   of u16 in the tracing, imaging and adjoint kernels, two tables of u32 prefix sums
+   in the solves */
 __host__ __device__ inline size_t walk_lds_bytes(uint32_t cap)
 {
     return 8 * ((2 * (size_t)cap * 4 + 7) / 8) + 4 * (size_t)cap * 8 + 4 * (size_t)cap * 2;
 }
 
-/* dynamic LDS of the solve kernel: walk buffers, the Lambda (L) accumulator and, when
-   j_lds, the J (F) accumulator */
-__host__ __device__ inline size_t solve_lds_bytes(uint32_t cap, uint32_t F, uint32_t L, bool j_lds)
+/* where the staged entries of a solve start (16-byte aligned) and how long they are */
+__host__ __device__ inline size_t stage_lds_offset(uint32_t cap)
 {
-    return ((walk_lds_bytes(cap) + 7) / 8) * 8 + 8 * (size_t)L + (j_lds ? 8 * (size_t)F : 0);
+    return (walk_lds_bytes(cap) + 15) / 16 * 16;
 }
+
+__host__ __device__ inline size_t group_lds_offset(uint32_t cap, uint32_t stage)
+{
+    return stage_lds_offset(cap) + 2 * (size_t)stage * sizeof(StagedEntry);
+}
+
+__host__ __device__ inline size_t lines_lds_offset(uint32_t cap, uint32_t stage)
+{
+    return group_lds_offset(cap, stage) + 2 * sizeof(GroupRay);
+}
+
+/* lines a group takes side by side for windows with several lines */
+__host__ __device__ inline uint32_t window_lines(uint32_t stage) { return stage < kStage ? 1 : kWindowLines; }
+
+__host__ __device__ inline size_t acc_lds_offset(uint32_t cap, uint32_t stage)
+{
+    return lines_lds_offset(cap, stage) + 2 * (size_t)window_lines(stage) * sizeof(WindowLine);
+}
+
+/* dynamic LDS of the solve kernel: walk buffers, staged entries (stage of each of two
+   groups) and their half rays, the Lambda (L) accumulator and, when j_lds, the J (F) accumulator */
+__host__ __device__ inline size_t solve_lds_bytes(uint32_t cap, uint32_t stage, uint32_t F, uint32_t L,
+                                                  bool j_lds)
+{
+    return acc_lds_offset(cap, stage) + 8 * (size_t)L + (j_lds ? 8 * (size_t)F : 0);
+}
+
+/* LDS kept beside the walk buffers when the longest walk that fits is worked out: the
+   static LDS of a kernel (the float functions' tables, MGX_REF_LDS_TABLE_BYTES, and a
+   few words) and the smallest chunk of staged entries */
+constexpr uint32_t kStageMin = 6;
+constexpr size_t kStaticLds = MGX_REF_LDS_TABLE_BYTES + 64;
+constexpr size_t kReservedLds = 2048;
+static_assert(kStaticLds + 2 * (kStageMin * sizeof(StagedEntry) + sizeof(GroupRay) + sizeof(WindowLine)) + 16 <= kReservedLds, "reserved LDS");
 
 /* J stays in LDS while the whole LDS of a workgroup fits the share of a CU's
    160 KiB that the register-limited occupancy (MGX_SOLVE_WAVES_PER_SIMD waves on
    each of 4 SIMDs) leaves it; beyond that (many lines, F ~ 10^3) LDS would lower
    the occupancy, and J is accumulated in the origin's row of the output instead
    (only that origin's wave writes it) */
-/* room for the static LDS of a kernel: the float functions' tables
-   (MGX_REF_LDS_TABLE_BYTES) and a few words */
-constexpr size_t kStaticLds = 2048;
-static_assert(MGX_REF_LDS_TABLE_BYTES + 64 <= kStaticLds, "static LDS estimate");
-
-inline bool j_in_lds(uint32_t cap, uint32_t F, uint32_t L)
+inline bool j_in_lds(uint32_t cap, uint32_t stage, uint32_t F, uint32_t L)
 {
     const size_t share = (160 * 1024) / (4 * MGX_SOLVE_WAVES_PER_SIMD);
-    return solve_lds_bytes(cap, F, L, true) + kStaticLds <= share;
+    return solve_lds_bytes(cap, stage, F, L, true) + kStaticLds <= share;
+}
+
+/* entries a group stages at a time: as many as its lanes can stage side by side; few
+   where the walk buffers of very long rays need the room */
+inline uint32_t stage_entries(uint32_t cap, uint32_t L)
+{
+    return solve_lds_bytes(cap, kStage, 0, L, false) + kStaticLds <= 80 * 1024 ? kStage : kStageMin;
 }
 
 /* J(o, f) += c for one ray pair: the first ray pair of a full pass stores (the sum
@@ -900,6 +956,9 @@ __device__ inline void j_add(double *Jrow, uint32_t f, double c, bool first, boo
     else
         Jrow[f] = first ? c : Jrow[f] + c;
 }
+
+/* which formal solution solve_origin runs */
+enum { METHOD_FEAUTRIER = 0, METHOD_SHORTCHAR = 1, METHOD_UV = 2 };
 
 /*
  * One half ray of the two-sided elimination.  Walking from the boundary end
@@ -939,7 +998,7 @@ struct BandRing {
 };
 
 template <int NB>
-__device__ inline void ring_push(BandRing<NB> &r, double h, double g, const Entry &e)
+__device__ inline void ring_push(BandRing<NB> &r, double h, double g, uint32_t nr, double shift)
 {
 #pragma unroll
     for (int i = NB - 1; i > 0; i--) {
@@ -950,122 +1009,135 @@ __device__ inline void ring_push(BandRing<NB> &r, double h, double g, const Entr
     }
     r.h[0] = h;
     r.g[0] = g;
-    r.sh[0] = e.shift;
-    r.nr[0] = e.nr;
+    r.sh[0] = shift;
+    r.nr[0] = nr;
     r.n = (r.n < (uint32_t)NB) ? r.n + 1 : (uint32_t)NB;
 }
 
-template <int APPROX, int PREC, int NB = 0>
-__device__ inline void sweep_half(const KParams &kp, const double *s_erf, const OwnLine &ol,
-                                  bool backward, uint32_t S, uint32_t o, double shift0,
-                                  const uint32_t *s_nxt, const double *s_dZ, const double *s_sh,
-                                  const uint16_t *mtab, uint32_t l, double freq, Sweep &sw,
-                                  PointEC &ec_centre, BandRing<NB> *ring = nullptr)
+/*
+ * The bins of a group sweep their half ray from its outer end to the origin, over
+ * entries staged chunk by chunk.  backward (per group) marks the antipod half.
+ * With METHOD_SHORTCHAR it is one direction of the order-0 short-characteristics
+ * solve instead (solve_shortchar_order_0_ray_forward / _backward,
+ * solver.tpp:1565-1757): I <- e^-dt I + expm1(-dt)/dt (S_c - S_n (1 + dt)) + S_c - S_n
+ * per segment, from the outer entry (current) to the inner one (next) on both halves,
+ * with dt = max(min_dtau, dtau) and the reference's float expf / expm1f; sw.Y carries
+ * I and sw.prev_dtau the last dt.
+ */
+template <int APPROX, int PREC, int METHOD, int NB>
+__device__ __forceinline__ void staged_sweep(const KParams &kp, unsigned char *smem, const GroupRay *g,
+                                             bool backward, double freq, bool active, StagedEntry *chunk,
+                                             double min_dtau, Sweep &sw, BandRing<NB> &ring)
 {
-    HalfIter it;
-    it.s = (int)S - 1;
-    hi_load_step(kp, it, l, o, shift0, s_nxt, s_dZ, s_sh, mtab);
-    Entry outer = hi_entry(it, o);
+    const uint32_t count = kp.stage;
+    const uint32_t n = active ? g->n : 0;
+    const uint32_t nA = (uint32_t)__builtin_amdgcn_readlane((int)n, 0);
+    const uint32_t nB = (uint32_t)__builtin_amdgcn_readlane((int)n, 32);
+    const BinLine bin = {freq, g->ol.a_g};
+    WindowLine *lines = reinterpret_cast<WindowLine *>(smem + lines_lds_offset(kp.cap, count)) +
+                        ((threadIdx.x & (MGX_WAVE - 1)) >> 5) * window_lines(count);
+    const uint32_t nmax = nA > nB ? nA : nB;
+    OuterEnd out = {0.0, 0.0, 0.0, 0.0};
     PointEC ec_out = {0.0, 0.0, false};
+    double I_b = 0.0;
     sw.started = false;
-    for (;;) {
-        const double dz = hi_advance(kp, it, l, o, shift0, s_nxt, s_dZ, s_sh, mtab);
-        Entry inner = hi_entry(it, o);
-        PointEC ec_in = (it.s < 0) ? ec_centre : PointEC{0.0, 0.0, false};
-        /* the segment runs from the rr-side entry to the antipod-side entry */
-        const Entry &cu = backward ? inner : outer;
-        const Entry &nx = backward ? outer : inner;
-        PointEC &ec_cu = backward ? ec_in : ec_out;
-        PointEC &ec_nx = backward ? ec_out : ec_in;
-        double dtau, S_cu, S_nx;
-        sw.last_trap =
-            segment<APPROX, PREC>(kp, s_erf, ol, cu, nx, dz, freq, l, ec_cu, ec_nx, dtau, S_cu, S_nx);
-        sw.chi_outer = ec_out.chi;
-        sw.dz_last = dz;
-        const double S_out = backward ? S_nx : S_cu; /* row "outer" from this segment */
-        const double S_in = backward ? S_cu : S_nx;
-        /* row "outer": the boundary row first, then interior rows; the backward
-           half's interior row takes its source from the segment beyond it */
-        const double S_row = backward ? (sw.started ? sw.S_prev_row : S_out) : S_out;
-        if (!sw.started) {
-            const double I_b = boundary_intensity(kp, outer.nr, freq * outer.shift);
-            const double idt = rcp(dtau);
-            const double B_min = fma(2.0, idt, 1.0);
-            const double B = fma(2.0 * idt, idt, B_min);
-            const double iB = rcp(B);
-            sw.Y = fma(2.0 * I_b, idt, S_row) * iB;
-            sw.X = 0.5 * B_min * dtau * dtau;
-            sw.XI = rcp(1.0 + sw.X);
-            sw.started = true;
-            if constexpr (NB > 0) ring_push<NB>(*ring, iB, 0.0, outer);
-        } else {
-            const double avg = 0.5 * (sw.prev_dtau + dtau);
-            const double q_out = avg * sw.prev_dtau;
-            const double q_in = avg * dtau;
-            const double r = rcp(q_out);
-            sw.X = fma(r * sw.X, sw.XI, 1.0) * q_in;
-            sw.XI = rcp(1.0 + sw.X);
-            sw.Y = fma(r, sw.Y, S_row) * sw.XI * q_in;
-            if constexpr (NB > 0) {
-                const double hq = sw.XI * q_in;
-                ring_push<NB>(*ring, hq, r * hq, outer);
-            }
+    sw.last_trap = false;
+    sw.X = sw.XI = sw.Y = sw.prev_dtau = sw.S_prev_row = sw.chi_outer = sw.dz_last = 0.0;
+    for (uint32_t k0 = 0; k0 < nmax; k0 += count - 1) {
+        stage_chunk<APPROX, PREC>(kp, smem, g, k0, count, chunk);
+        if (k0 == 0 && n > 0) {
+            const double s = chunk->shift;
+            out.iw = chunk->iw;
+            out.kap = chunk->kap;
+            out.src = chunk->src;
+            out.f = freq * s;
+            I_b = boundary_intensity(kp, chunk->nr, out.f);
         }
-        sw.prev_dtau = dtau;
-        sw.S_inner = S_in;
-        sw.S_prev_row = S_in;
-        outer = inner;
-        ec_out = ec_in;
-        if (it.s < 0) break;
+        const uint32_t left = nmax - k0, jmax = left < count - 1 ? left : count - 1;
+        for (uint32_t j = 1; j <= jmax; j++) {
+            const StagedEntry *eo = chunk + j - 1, *ei = chunk + j;
+            PointEC ec_in = {0.0, 0.0, false};
+            double dtau, S_out, S_in;
+            const bool on = k0 + j <= n;
+            staged_segment<APPROX, PREC>(kp, g, lines, window_lines(count), bin, eo, ei, on, out, ec_out, ec_in, dtau,
+                                         S_out, S_in);
+            if (!on) continue;
+            if constexpr (METHOD == METHOD_SHORTCHAR) {
+                if (!sw.started) sw.Y = I_b;
+                sw.started = true;
+                const double dt = (min_dtau < dtau) ? dtau : min_dtau; /* std::max(min_dtau, dtau) */
+                const float mdt = (float)(-dt);
+                sw.Y = (double)mgx_ref_expf(mdt) * sw.Y +
+                       (double)mgx_ref_expm1f(mdt) / dt * (S_out - S_in * (1.0 + dt)) + S_out - S_in;
+                sw.prev_dtau = dt;
+                ec_out = ec_in;
+                continue;
+            }
+            if constexpr (METHOD == METHOD_UV) {
+                const uint32_t kind = ei->kind;
+                sw.last_trap = (kind & SEG_IS_TRAP) != 0;
+                sw.chi_outer = (kind & SEG_MASK) == SEG_EMPTY ? kp.op.min_opacity : ec_out.chi;
+                sw.dz_last = ei->dz;
+            }
+            /* row "outer": the boundary row first, then interior rows; the backward
+               half's interior row takes its source from the segment beyond it */
+            if (!sw.started) {
+                const double idt = rcp(dtau);
+                const double B_min = fma(2.0, idt, 1.0);
+                const double B = fma(2.0 * idt, idt, B_min);
+                const double iB = rcp(B);
+                sw.Y = fma(2.0 * I_b, idt, S_out) * iB;
+                sw.X = 0.5 * B_min * dtau * dtau;
+                sw.XI = rcp(1.0 + sw.X);
+                sw.started = true;
+                if constexpr (NB > 0) ring_push<NB>(ring, iB, 0.0, eo->nr, eo->shift);
+            } else {
+                const double S_row = backward ? sw.S_prev_row : S_out;
+                const double avg = 0.5 * (sw.prev_dtau + dtau);
+                const double q_out = avg * sw.prev_dtau;
+                const double q_in = avg * dtau;
+                const double r = rcp(q_out);
+                sw.X = fma(r * sw.X, sw.XI, 1.0) * q_in;
+                sw.XI = rcp(1.0 + sw.X);
+                sw.Y = fma(r, sw.Y, S_row) * sw.XI * q_in;
+                if constexpr (NB > 0) {
+                    const double hq = sw.XI * q_in;
+                    ring_push<NB>(ring, hq, r * hq, eo->nr, eo->shift);
+                }
+            }
+            sw.prev_dtau = dtau;
+            sw.S_prev_row = S_in;
+            ec_out = ec_in;
+        }
     }
-    ec_centre = ec_out;
+    sw.S_inner = sw.S_prev_row;
 }
 
-/*
- * One direction of the order-0 short-characteristics solve
- * (solve_shortchar_order_0_ray_forward / _backward, solver.tpp:1565-1757): from
- * the outer end of a half ray to the origin, I <- e^-dt I + expm1(-dt)/dt
- * (S_c - S_n (1 + dt)) + S_c - S_n per segment with dt = max(min_dtau, dtau)
- * and the reference's float expf / expm1f.  Segments run from the outer entry
- * (current) to the inner one (next) on both halves, as the reference calls
- * compute_source_dtau.  dt_last receives the last segment's dt (0 when the half
- * has no segment: I is then the boundary intensity at the origin).
- */
-template <int APPROX, int PREC>
-__device__ inline double shortchar_half(const KParams &kp, const double *s_erf, const OwnLine &ol,
-                                        uint32_t S, uint32_t o, double shift0,
-                                        const uint32_t *s_nxt, const double *s_dZ,
-                                        const double *s_sh, const uint16_t *mtab, uint32_t l,
-                                        double freq, double min_dtau, double &dt_last,
-                                        PointEC &ec_centre)
+/* the lane's sweep of the other half ray, held by the other group of the wave */
+template <int METHOD, int NB>
+__device__ inline void exchange_halves(Sweep &sw, BandRing<NB> &ring)
 {
-    dt_last = 0.0;
-    if (S == 0) return boundary_intensity(kp, o, freq);
-    HalfIter it;
-    it.s = (int)S - 1;
-    hi_load_step(kp, it, l, o, shift0, s_nxt, s_dZ, s_sh, mtab);
-    Entry outer = hi_entry(it, o);
-    PointEC ec_out = {0.0, 0.0, false};
-    double I = boundary_intensity(kp, outer.nr, freq * outer.shift);
-    double dt = 0.0;
-    for (;;) {
-        const double dz = hi_advance(kp, it, l, o, shift0, s_nxt, s_dZ, s_sh, mtab);
-        Entry inner = hi_entry(it, o);
-        PointEC ec_in = (it.s < 0) ? ec_centre : PointEC{0.0, 0.0, false};
-        double dtau, S_c, S_n;
-        segment<APPROX, PREC>(kp, s_erf, ol, outer, inner, dz, freq, l, ec_out, ec_in, dtau, S_c,
-                              S_n);
-        dt = (min_dtau < dtau) ? dtau : min_dtau; /* std::max(min_dtau, dtau) */
-        const float mdt = (float)(-dt);
-        I = (double)mgx_ref_expf(mdt) * I + (double)mgx_ref_expm1f(mdt) / dt * (S_c - S_n * (1.0 + dt)) +
-            S_c - S_n;
-        outer = inner;
-        ec_out = ec_in;
-        if (it.s < 0) break;
+    const auto x = [](double v) { return __shfl_xor(v, 32, MGX_WAVE); };
+    sw.X = x(sw.X);
+    sw.XI = x(sw.XI);
+    sw.Y = x(sw.Y);
+    sw.prev_dtau = x(sw.prev_dtau);
+    sw.S_inner = x(sw.S_inner);
+    if constexpr (METHOD == METHOD_UV) {
+        sw.chi_outer = x(sw.chi_outer);
+        sw.dz_last = x(sw.dz_last);
+        sw.last_trap = __shfl_xor((int)sw.last_trap, 32, MGX_WAVE) != 0;
     }
-    ec_centre = ec_out;
-    dt_last = dt;
-    return I;
+    if constexpr (NB > 0) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            ring.h[i] = x(ring.h[i]);
+            ring.g[i] = x(ring.g[i]);
+            ring.sh[i] = x(ring.sh[i]);
+            ring.nr[i] = __shfl_xor(ring.nr[i], 32, MGX_WAVE);
+        }
+        ring.n = __shfl_xor(ring.n, 32, MGX_WAVE);
+    }
 }
 
 /* The factors of a Lambda element at the origin that do not depend on the
@@ -1100,9 +1172,6 @@ __device__ inline LamPoint lambda_point(const KParams &kp, const OwnLine &ol, ui
     r.phi = inverse_width * MGX_INVERSE_SQRT_PI * (double)f_exp<PREC>((float)(-ex));
     return r;
 }
-
-/* which formal solution solve_origin runs */
-enum { METHOD_FEAUTRIER = 0, METHOD_SHORTCHAR = 1, METHOD_UV = 2 };
 
 /* extra outputs of the short-characteristics and u/v solves */
 struct ShortcharOut {
@@ -1174,7 +1243,9 @@ __device__ __forceinline__ int solve_origin(const KParams &kp, uint32_t o, uint3
     double *s_dZ1 = s_dZ0 + cap;
     double *s_sh0 = s_dZ1 + cap;
     double *s_sh1 = s_sh0 + cap;
-    uint16_t *s_m = reinterpret_cast<uint16_t *>(s_sh1 + cap); /* [line j][half h][step] */
+    uint32_t *s_pre = reinterpret_cast<uint32_t *>(s_sh1 + cap); /* [group][step] */
+    const uint32_t grp = lane >> 5;
+    StagedEntry *chunk = reinterpret_cast<StagedEntry *>(smem + stage_lds_offset(cap)) + grp * kp.stage;
     const size_t PF = (size_t)P * F;
 
     for (uint32_t rr = rr0; rr < rr1; rr++) {
@@ -1192,29 +1263,16 @@ __device__ __forceinline__ int solve_origin(const KParams &kp, uint32_t o, uint3
         }
         __syncthreads();
         const double w = ray_weight(m, o, rr);
-        const uint32_t Sall = S0 + S1;
 
         for (uint32_t slot0 = 0; slot0 < kp.nslots; slot0 += 2) {
-            /* interpolation counts of this pass's two lines, one per (line, step) */
-            const uint32_t lA = slot0 / kp.slots_per_line;
-            const uint32_t lB = (slot0 + 1 < kp.nslots) ? (slot0 + 1) / kp.slots_per_line : lA;
-            for (uint32_t i = lane; i < 2 * Sall; i += MGX_WAVE) {
-                const uint32_t j = i / Sall, r = i % Sall;
-                const uint32_t h = (r < S0) ? 0 : 1;
-                const uint32_t st = h ? r - S0 : r;
-                const uint32_t *nx = h ? s_nxt1 : s_nxt0;
-                const uint32_t crt = (st == 0) ? o : nx[st - 1];
-                const uint32_t mm = n_interp_for_line(kp, j ? lB : lA, crt, nx[st]);
-                if (mm > 0xffffu) atomicOr(&kp.status[0], (uint32_t)ERR_INTERP);
-                s_m[(j * 2 + h) * cap + st] = (uint16_t)(mm > 0xffffu ? 0xffffu : mm);
-            }
-            __syncthreads();
-
-            const uint32_t jj = lane >> 5;
-            const uint32_t slot = slot0 + jj;
-            const uint32_t l = jj ? lB : lA;
+            /* two line slots at a time, one per group, each half ray in turn; the last
+               slot of an odd number is left alone: then each group takes one of its
+               half rays, and both meet at the origin */
+            const bool alone = slot0 + 1 == kp.nslots;
+            const uint32_t slot = alone ? slot0 : slot0 + grp;
+            const uint32_t l = slot / kp.slots_per_line;
             const uint32_t z = (slot % kp.slots_per_line) * 32 + (lane & 31);
-            const bool active = (slot < kp.nslots) && (z < Q);
+            const bool active = z < Q;
             double Lval = 0.0;
             /* band elements of this lane, rr side (lo) and antipod side (up), j = 0 .. NB-1 */
             double Llo[NB > 0 ? NB : 1], Lup[NB > 0 ? NB : 1];
@@ -1226,11 +1284,51 @@ __device__ __forceinline__ int solve_origin(const KParams &kp, uint32_t o, uint3
                 Llo[j] = Lup[j] = 0.0;
                 qlo[j] = qup[j] = 0;
             }
-            if (active) {
+            const uint32_t f = l * Q + (active ? z : Q - 1);
+            const size_t of = (size_t)o * F + f;
+            const double freq = gld(&m.nu[of]);
+            Sweep fw, bw;
+            BandRing<NB> ring_f, ring_b;
+            if constexpr (NB > 0) ring_f = ring_b = BandRing<NB>{};
+            {
+                GroupRay *g = reinterpret_cast<GroupRay *>(smem + group_lds_offset(cap, kp.stage)) + grp;
+                const double fmin = group32(freq, [](double a, double b) { return a < b ? a : b; });
+                const double fmax = group32(freq, [](double a, double b) { return a < b ? b : a; });
+#pragma unroll 1
+                for (uint32_t pass = 0; pass < (alone ? 1u : 2u); pass++) {
+                    const bool back = alone ? grp == 1 : pass == 0;
+                    if ((lane & 31) == 0) {
+                        GroupRay r;
+                        r.o = o;
+                        r.line = l;
+                        r.S = back ? S1 : S0;
+                        r.list = back ? 1 : 0;
+                        r.shift0 = back ? sh01 : sh00;
+                        r.shift_c = 1.0;
+                        r.fmin = fmin;
+                        r.fmax = fmax;
+                        r.ol = own_line(m, l);
+                        *g = r;
+                    }
+                    __syncthreads();
+                    if (pass == 1) {
+                        bw = fw;
+                        if constexpr (NB > 0) ring_b = ring_f;
+                        if constexpr (NB > 0) ring_f = BandRing<NB>{};
+                    }
+                    count_entries<false>(kp, smem, g);
+                    staged_sweep<APPROX, PREC, METHOD, NB>(kp, smem, g, back, freq, active, chunk, sc.min_dtau,
+                                                           fw, ring_f);
+                }
+                if (alone) {
+                    /* group 0 swept the rr side: it takes the antipod side's state from group 1 */
+                    bw = fw;
+                    if constexpr (NB > 0) ring_b = ring_f;
+                    exchange_halves<METHOD, NB>(bw, ring_b);
+                }
+            }
+            if (active && !(alone && grp == 1)) {
                 const OwnLine ol = own_line(m, l);
-                const uint32_t f = l * Q + z;
-                const size_t of = (size_t)o * F + f;
-                const double freq = gld(&m.nu[of]);
                 if constexpr (METHOD == METHOD_SHORTCHAR) {
                     /* solve_shortchar_order_0 (solver.tpp:186-224): both directions,
                        u, v, J and a Lambda element per direction */
@@ -1239,14 +1337,10 @@ __device__ __forceinline__ int solve_origin(const KParams &kp, uint32_t o, uint3
                         If = Ib = uc = boundary_intensity(kp, o, freq);
                         vc = 0.0;
                     } else {
-                        PointEC ec_cent = {0.0, 0.0, false};
-                        double dtf, dtb;
-                        If = shortchar_half<APPROX, PREC>(kp, s_erf, ol, S0, o, sh00, s_nxt0, s_dZ0,
-                                                          s_sh0, s_m + (jj * 2 + 0) * cap, l, freq,
-                                                          sc.min_dtau, dtf, ec_cent);
-                        Ib = shortchar_half<APPROX, PREC>(kp, s_erf, ol, S1, o, sh01, s_nxt1, s_dZ1,
-                                                          s_sh1, s_m + (jj * 2 + 1) * cap, l, freq,
-                                                          sc.min_dtau, dtb, ec_cent);
+                        /* a half without a segment is its boundary intensity */
+                        const double dtf = fw.prev_dtau, dtb = bw.prev_dtau;
+                        If = S0 > 0 ? fw.Y : boundary_intensity(kp, o, freq);
+                        Ib = S1 > 0 ? bw.Y : boundary_intensity(kp, o, freq);
                         uc = 0.5 * (If + Ib);
                         vc = 0.5 * (If - Ib);
                         if (with_lam) {
@@ -1286,19 +1380,6 @@ __device__ __forceinline__ int solve_origin(const KParams &kp, uint32_t o, uint3
                             j_add(Jrow, f, 2.0 * w * uc, rr == rr0, j_atomic);
                     }
                 } else {
-                    PointEC ec_cent = {0.0, 0.0, false};
-                    Sweep bw, fw;
-                    bw.started = fw.started = false;
-                    BandRing<NB> ring_b, ring_f;
-                    ring_b.n = ring_f.n = 0;
-                    if (S1 > 0)
-                        sweep_half<APPROX, PREC, NB>(kp, s_erf, ol, true, S1, o, sh01, s_nxt1,
-                                                     s_dZ1, s_sh1, s_m + (jj * 2 + 1) * cap, l,
-                                                     freq, bw, ec_cent, &ring_b);
-                    if (S0 > 0)
-                        sweep_half<APPROX, PREC, NB>(kp, s_erf, ol, false, S0, o, sh00, s_nxt0,
-                                                     s_dZ0, s_sh0, s_m + (jj * 2 + 0) * cap, l,
-                                                     freq, fw, ec_cent, &ring_f);
                     double Lc;
                     double du_fw = 0.0, du_bw = 0.0; /* du_c / dY of each half's last row */
                     if (S1 > 0) {
@@ -1516,7 +1597,7 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void feautrier_
             __hip_atomic_load(&kp.status[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) &
         ERR_CAP)
         return;
-    double *s_L = reinterpret_cast<double *>(smem + ((walk_lds_bytes(kp.cap) + 7) / 8) * 8);
+    double *s_L = reinterpret_cast<double *>(smem + acc_lds_offset(kp.cap, kp.stage));
     double *s_J = kp.j_lds ? s_L + L : nullptr;
     for (uint32_t i = lane; i < L + (s_J ? F : 0); i += MGX_WAVE) s_L[i] = 0.0;
     if (solve_origin<APPROX, PREC>(kp, o, 0, m.hnrays, smem, s_erf, u, lam != nullptr, s_J,
@@ -1560,7 +1641,7 @@ __global__ __launch_bounds__(MGX_WAVE, 2) void feautrier_bands_kernel(
             __hip_atomic_load(&kp.status[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) &
         ERR_CAP)
         return;
-    double *s_L = reinterpret_cast<double *>(smem + ((walk_lds_bytes(kp.cap) + 7) / 8) * 8);
+    double *s_L = reinterpret_cast<double *>(smem + acc_lds_offset(kp.cap, kp.stage));
     double *s_J = kp.j_lds ? s_L + L : nullptr;
     for (uint32_t i = lane; i < L + (s_J ? F : 0); i += MGX_WAVE) s_L[i] = 0.0;
     if (lane == 0)
@@ -1592,7 +1673,7 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void shortchar_
             __hip_atomic_load(&kp.status[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) &
         ERR_CAP)
         return;
-    double *s_L = reinterpret_cast<double *>(smem + ((walk_lds_bytes(kp.cap) + 7) / 8) * 8);
+    double *s_L = reinterpret_cast<double *>(smem + acc_lds_offset(kp.cap, kp.stage));
     double *s_J = kp.j_lds ? s_L + L : nullptr;
     for (uint32_t i = lane; i < L + (s_J ? F : 0); i += MGX_WAVE) s_L[i] = 0.0;
     if (solve_origin<APPROX, PREC, METHOD_SHORTCHAR>(kp, o, 0, m.hnrays, smem, s_erf, u,
@@ -1616,7 +1697,7 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void feautrier_
     extern __shared__ unsigned char smem[];
     const double *s_erf = nullptr; /* erf needs no table */
     const uint32_t o = blockIdx.x;
-    double *s_L = reinterpret_cast<double *>(smem + ((walk_lds_bytes(kp.cap) + 7) / 8) * 8);
+    double *s_L = reinterpret_cast<double *>(smem + acc_lds_offset(kp.cap, kp.stage));
     ShortcharOut sc{nullptr, v, 0.0};
     solve_origin<APPROX, PREC, METHOD_UV>(kp, o, 0, kp.m.hnrays, smem, s_erf, u, false, nullptr,
                                           nullptr, false, s_L, sc);
@@ -1658,7 +1739,7 @@ __global__ __launch_bounds__(MGX_WAVE, WPS) void feautrier_batch_kernel(
         const BatchItem it = items[w];
         const KParams &kp = kps[it.model];
         const uint32_t F = kp.m.nfreqs, L = kp.m.nlines;
-        double *s_L = reinterpret_cast<double *>(smem + ((walk_lds_bytes(kp.cap) + 7) / 8) * 8);
+        double *s_L = reinterpret_cast<double *>(smem + acc_lds_offset(kp.cap, kp.stage));
         double *s_J = kp.j_lds ? s_L + L : nullptr;
         for (uint32_t i = lane; i < L + (s_J ? F : 0); i += MGX_WAVE) s_L[i] = 0.0;
         double *Jm = J[it.model];
@@ -2149,20 +2230,6 @@ __device__ inline double fe_last(const FwdElim &fe, double S_last, double I_l)
     const double denominator = rcp(fma(Bl, fe.FF, Bl_min_Al));
     const double Sl = fma(2.0 * I_l, idt, S_last);
     return fma(A_l, fe.Su, Sl) * (1.0 + fe.FF) * denominator;
-}
-
-/* all-lines interpolation count (InterpHelper::get_n_interp, :10-46) */
-__device__ inline uint32_t n_interp_all(const KParams &kp, uint32_t c, uint32_t n)
-{
-    const uint32_t L = kp.m.nlines;
-    double mx = 0.0;
-    for (uint32_t l = 0; l < L; l++) {
-        const double d = (double)fabsf(mgx_ref_logf((float)(kp.m.interp_crit[(size_t)n * L + l] /
-                                                        kp.m.interp_crit[(size_t)c * L + l])));
-        if (l == 0 || mx < d) mx = d;
-    }
-    const uint32_t k = (uint32_t)ceil(mx / kp.log_max_interp);
-    return (k > 1) ? k : 1;
 }
 
 /* The projection-surface imager, one pixel at a time (the pixel loop bodies of
@@ -4159,7 +4226,7 @@ int read_status(hipStream_t st, const DevBuffers &b, uint32_t *need, uint32_t *n
 }
 
 /* LDS per workgroup available to dynamic allocations: the device's limit (160 KiB
-   on gfx950) less the static LDS, queried once per device */
+   on gfx950) less what is kept beside the walk buffers, queried once per device */
 size_t lds_budget()
 {
     static size_t cached[64] = {};
@@ -4170,7 +4237,7 @@ size_t lds_budget()
         if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
             v <= 0)
             v = 65536;
-        cached[dev] = (size_t)v - kStaticLds;
+        cached[dev] = (size_t)v - kReservedLds;
     }
     return cached[dev];
 }
@@ -4298,7 +4365,8 @@ int launch_with_capacity(hipStream_t st, DevBuffers &b, KParams &kp, Launch laun
     }
     for (;;) {
         kp.cap = cap;
-        kp.j_lds = j_in_lds(cap, kp.m.nfreqs, kp.m.nlines) ? 1 : 0;
+        kp.stage = stage_entries(cap, kp.m.nlines);
+        kp.j_lds = j_in_lds(cap, kp.stage, kp.m.nfreqs, kp.m.nlines) ? 1 : 0;
         HIP_TRY(hipMemsetAsync(b.status, 0, 4 * sizeof(uint32_t), st));
         HIP_TRY(hipMemcpyAsync(b.kp_dev, &kp, sizeof(KParams), hipMemcpyHostToDevice, st));
         g_last_kernel_ms = 0.0;
@@ -4595,11 +4663,13 @@ uint32_t batch_grid(uint32_t wps, size_t lds)
     return persistent_waves(feautrier_batch_kernel<A, PR, 3>, lds, 0xffffffffu);
 }
 
-bool batch_j_lds(const mgx_batch &B) { return j_in_lds(B.cap, B.maxF, B.maxL); }
+uint32_t batch_stage(const mgx_batch &B) { return stage_entries(B.cap, B.maxL); }
+
+bool batch_j_lds(const mgx_batch &B) { return j_in_lds(B.cap, batch_stage(B), B.maxF, B.maxL); }
 
 size_t batch_lds(const mgx_batch &B)
 {
-    return walk_lds_bytes(B.cap) + 8 + 8 * (size_t)B.maxL + (batch_j_lds(B) ? 8 * (size_t)B.maxF : 0);
+    return solve_lds_bytes(B.cap, batch_stage(B), B.maxF, B.maxL, batch_j_lds(B));
 }
 
 /* persistent grid of the current configuration (resident waves, at most n_items) */
@@ -4723,6 +4793,7 @@ int batch_upload(mgx_batch &B, hipStream_t st)
                            hipMemcpyHostToDevice, st));
     for (auto &k : B.kps) {
         k.cap = B.cap;
+        k.stage = batch_stage(B);
         k.j_lds = batch_j_lds(B) ? 1 : 0;
     }
     HIP_TRY(hipMemcpyAsync(B.kps_dev, B.kps.data(), B.kps.size() * sizeof(KParams),
@@ -4897,7 +4968,7 @@ int forward_launch(const mgx_model *model, const mgx_options *opts, double *u, d
             J = *J_scratch;
         }
         const dim3 grid(model->npoints), block(MGX_WAVE);
-        const size_t lds = solve_lds_bytes(kp.cap, model->nfreqs, model->nlines, kp.j_lds != 0);
+        const size_t lds = solve_lds_bytes(kp.cap, kp.stage, model->nfreqs, model->nlines, kp.j_lds != 0);
         timed(st, [&] {
             const bool fp64 = opts->precision == MGX_PREC_FP64;
             switch (opts->approx) {
@@ -5052,7 +5123,7 @@ int mgx_feautrier_forward_lambda_device(const mgx_model *model, const mgx_option
     const LamBands lb{lam_count, lam_nr, lam_val, cap, opts->n_off_diag};
     return launch_with_capacity(st, b, kp, [&](size_t) {
         const dim3 grid(model->npoints), block(MGX_WAVE);
-        const size_t lds = solve_lds_bytes(kp.cap, model->nfreqs, model->nlines, kp.j_lds != 0);
+        const size_t lds = solve_lds_bytes(kp.cap, kp.stage, model->nfreqs, model->nlines, kp.j_lds != 0);
         timed(st, [&] {
             const bool fp64 = op.precision == MGX_PREC_FP64;
             switch (op.approx) {
@@ -5099,7 +5170,7 @@ int mgx_shortchar_order_0_device(const mgx_model *model, const mgx_options *opts
     const ShortcharOut sc{I, v, min_dtau};
     return launch_with_capacity(st, b, kp, [&](size_t) {
         const dim3 grid(model->npoints), block(MGX_WAVE);
-        const size_t lds = solve_lds_bytes(kp.cap, model->nfreqs, model->nlines, kp.j_lds != 0);
+        const size_t lds = solve_lds_bytes(kp.cap, kp.stage, model->nfreqs, model->nlines, kp.j_lds != 0);
         timed(st, [&] {
             const bool fp64 = opts->precision == MGX_PREC_FP64;
             switch (opts->approx) {
@@ -5143,7 +5214,7 @@ int mgx_feautrier_order_2_uv_device(const mgx_model *model, const mgx_options *o
     if (int e = prepare(model, opts, st, b, kp)) return e;
     return launch_with_capacity(st, b, kp, [&](size_t) {
         const dim3 grid(model->npoints), block(MGX_WAVE);
-        const size_t lds = solve_lds_bytes(kp.cap, model->nfreqs, model->nlines, false);
+        const size_t lds = solve_lds_bytes(kp.cap, kp.stage, model->nfreqs, model->nlines, false);
         timed(st, [&] {
             const bool fp64 = opts->precision == MGX_PREC_FP64;
             switch (opts->approx) {
