@@ -85,6 +85,7 @@ MGX_FM_CONST uint64_t MGX_REF_EXP2_TAB[32] = {
 #if defined(__HIP_DEVICE_COMPILE__)
 static __shared__ uint64_t mgx_ref_lds_exp2[32];
 static __shared__ double mgx_ref_lds_log[16][3];
+static __shared__ float4 mgx_ref_lds_erf[4][4];
 #define MGX_REF_EXP2_AT(i) mgx_ref_lds_exp2[(i)]
 #define MGX_REF_LOG_AT(i, j) mgx_ref_lds_log[(i)][(j)]
 #else
@@ -92,7 +93,7 @@ static __shared__ double mgx_ref_lds_log[16][3];
 #define MGX_REF_LOG_AT(i, j) MGX_REF_LOG_TAB[(i)][(j)]
 #endif
 /* LDS the tables take in each workgroup of a kernel that uses them */
-#define MGX_REF_LDS_TABLE_BYTES (32 * 8 + 16 * 3 * 8)
+#define MGX_REF_LDS_TABLE_BYTES (32 * 8 + 16 * 3 * 8 + 4 * 64)
 
 /* Cubic for 2^(r/32), r in [-1/2, 1/2]: coefficients of r^3, r^2, r (the
  * minimax fit of optimized-routines' exp2f, scaled by 1/32^3, 1/32^2, 1/32). */
@@ -255,6 +256,99 @@ MGX_FM_HD float mgx_ref_fdiv(float a, float b)
 #endif
 }
 
+/*
+ * erff on the device, the same bits by one path for every range: fdlibm's rational
+ * functions of the four ranges of |x| (below 0.84375 in x^2, below 1.25 in |x| - 1,
+ * below 1/0.35 and beyond in 1/x^2) are evaluated by one pair of Horner chains of
+ * degree 7 and 8, whose coefficients each lane reads from its range's row in LDS
+ * (64-byte rows: the four rows lie in different banks).  A shorter polynomial is
+ * padded with zeros in front: 0 s + c is c exactly, so the operations that count are
+ * fdlibm's own, in their order.  The bins of a line spread over all four ranges, so
+ * branches per range made a wave run each range's polynomials in turn: ~200
+ * instructions per call against ~110 here.  The tail's exponentials take
+ * the fused form of the expf above; that this leaves every erff result alone was checked
+ * on all floats in [1.25, 6), and erff as a whole on all 2^32 arguments
+ * (mgx_fmath_digest).  From MGX_REF_ERF_ONE on the result is 1 (checked up to 6, where
+ * fdlibm returns 1 too).
+ */
+#define MGX_REF_ERF_ONE 0x407ad445u /* 3.9192059 */
+
+/* coefficients by range: numerator s^7 .. s^0, denominator s^8 .. s^1 */
+MGX_FM_CONST float MGX_REF_ERF_TAB[4][16] = {
+    {0.0f, 0.0f, 0.0f, -2.3763017452e-05f, -5.7702702470e-03f, -2.8481749818e-02f, -3.2504209876e-01f,
+     1.2837916613e-01f, 0.0f, 0.0f, 0.0f, -3.9602282413e-06f, 1.3249473704e-04f, 5.0813062117e-03f,
+     6.5022252500e-02f, 3.9791721106e-01f},
+    {0.0f, -2.1663755178e-03f, 3.5478305072e-02f, -1.1089469492e-01f, 3.1834661961e-01f, -3.7220788002e-01f,
+     4.1485610604e-01f, -2.3621185683e-03f, 0.0f, 0.0f, 1.1984500103e-02f, 1.3637083583e-02f,
+     1.2617121637e-01f, 7.1828655899e-02f, 5.4039794207e-01f, 1.0642088205e-01f},
+    {-9.8143291473e+00f, -8.1287437439e+01f, -1.8460508728e+02f, -1.6239666748e+02f, -6.2375331879e+01f,
+     -1.0558626175e+01f, -6.9385856390e-01f, -9.8649440333e-03f, -6.0424413532e-02f, 6.5702495575e+00f,
+     1.0863500214e+02f, 4.2900814819e+02f, 6.4538726807e+02f, 4.3456588745e+02f, 1.3765776062e+02f,
+     1.9651271820e+01f},
+    {0.0f, -4.8351919556e+02f, -1.0250950928e+03f, -6.3756646729e+02f, -1.6063638306e+02f,
+     -1.7757955551e+01f, -7.9928326607e-01f, -9.8649431020e-03f, 0.0f, -2.2440952301e+01f,
+     4.7452853394e+02f, 2.5530502930e+03f, 3.1998581543e+03f, 1.5367296143e+03f, 3.2579251099e+02f,
+     3.0338060379e+01f}};
+
+#if defined(__HIP_DEVICE_COMPILE__)
+/* expf for arguments in (-88, 88): the fused form without the range checks */
+__device__ static inline float mgx_ref_expf_inner(float x)
+{
+    const double xd = (double)x;
+    double kd = MGX_FMA(MGX_REF_EXPF_INVLN2N, xd, MGX_REF_EXPF_SHIFT);
+    const uint64_t ki = mgx_fm_bits(kd);
+    kd -= MGX_REF_EXPF_SHIFT;
+    const double r = MGX_FMA(MGX_REF_EXPF_INVLN2N, xd, -kd);
+    const double s = mgx_fm_from_bits(mgx_ref_lds_exp2[ki % 32] + (ki << 47));
+    const double z = MGX_FMA(MGX_REF_EXPF_C0, r, MGX_REF_EXPF_C1);
+    const double y = MGX_FMA(z, r * r, MGX_FMA(MGX_REF_EXPF_C2, r, 1.0));
+    return (float)(y * s);
+}
+
+__device__ static inline float mgx_ref_erff(float x)
+{
+    const float ax = fabsf(x);
+    const uint32_t ix = mgx_rf_asuint(ax);
+    float e = 1.0f;
+    if (ix < MGX_REF_ERF_ONE) {
+        const uint32_t cls = (uint32_t)(ix >= 0x3f580000u) + (uint32_t)(ix >= 0x3fa00000u) +
+                             (uint32_t)(ix >= 0x4036db6eu);
+        const float xx = x * x;
+        float s = cls == 0 ? xx : ax - 1.0f;
+        if (cls >= 2) s = mgx_ref_fdiv(1.0f, xx);
+        const float4 n0 = mgx_ref_lds_erf[cls][0], n1 = mgx_ref_lds_erf[cls][1];
+        const float4 d0 = mgx_ref_lds_erf[cls][2], d1 = mgx_ref_lds_erf[cls][3];
+        float p = n0.y + s * n0.x;
+        p = n0.z + s * p;
+        p = n0.w + s * p;
+        p = n1.x + s * p;
+        p = n1.y + s * p;
+        p = n1.z + s * p;
+        p = n1.w + s * p;
+        float q = d0.y + s * d0.x;
+        q = d0.z + s * q;
+        q = d0.w + s * q;
+        q = d1.x + s * q;
+        q = d1.y + s * q;
+        q = d1.z + s * q;
+        q = d1.w + s * q;
+        q = 1.0f + s * q;
+        const float y = mgx_ref_fdiv(p, q);
+        e = cls == 0 ? ax + ax * y : 8.4506291151e-01f + y;
+        if (cls >= 2) {
+            const float z = mgx_rf_asfloat(ix & 0xfffff000u);
+            const float r = mgx_ref_expf_inner(-z * z - 0.5625f) * mgx_ref_expf_inner((z - ax) * (z + ax) + y);
+            e = 1.0f - mgx_ref_fdiv(r, ax);
+        }
+        if (ix < 0x31800000u) { /* |x| < 2^-28 */
+            const float efx = 1.2837916613e-01f;
+            e = ix < 0x04000000u ? 0.0625f * (16.0f * ax + (16.0f * efx) * ax) : ax + efx * ax;
+        }
+    }
+    if (ix > 0x7f800000u) e = x;
+    return mgx_rf_asfloat((mgx_rf_asuint(e) & 0x7fffffffu) | (mgx_rf_asuint(x) & 0x80000000u));
+}
+#else
 /* fdlibm s_erff.c */
 MGX_FM_HD float mgx_ref_erff(float x)
 {
@@ -329,6 +423,8 @@ MGX_FM_HD float mgx_ref_erff(float x)
     return rx - one;
 }
 
+#endif
+
 /* {1/c, log(c), log2(c)} for the 16 subintervals of [0x1.66p-1, 0x1.66p0). */
 MGX_FM_CONST double MGX_REF_LOG_TAB[16][3] = {
     {0x1.661ec79f8f3bep+0, -0x1.57bf7808caadep-2, -0x1.efec65b963019p-2},
@@ -358,6 +454,10 @@ __device__ static inline void mgx_ref_tables_init()
     for (uint32_t k = threadIdx.x; k < 32; k += blockDim.x) mgx_ref_lds_exp2[k] = MGX_REF_EXP2_TAB[k];
     for (uint32_t k = threadIdx.x; k < 48; k += blockDim.x)
         mgx_ref_lds_log[k / 3][k % 3] = MGX_REF_LOG_TAB[k / 3][k % 3];
+    for (uint32_t k = threadIdx.x; k < 16; k += blockDim.x) {
+        const float *c = &MGX_REF_ERF_TAB[k / 4][4 * (k % 4)];
+        mgx_ref_lds_erf[k / 4][k % 4] = make_float4(c[0], c[1], c[2], c[3]);
+    }
     __syncthreads();
 #endif
 }

@@ -923,7 +923,7 @@ __host__ __device__ inline size_t solve_lds_bytes(uint32_t cap, uint32_t stage, 
 /* LDS kept beside the walk buffers when the longest walk that fits is worked out: the
    static LDS of a kernel (the float functions' tables, MGX_REF_LDS_TABLE_BYTES, and a
    few words) and the smallest chunk of staged entries */
-constexpr uint32_t kStageMin = 6;
+constexpr uint32_t kStageMin = 4;
 constexpr size_t kStaticLds = MGX_REF_LDS_TABLE_BYTES + 64;
 constexpr size_t kReservedLds = 2048;
 static_assert(kStaticLds + 2 * (kStageMin * sizeof(StagedEntry) + sizeof(GroupRay) + sizeof(WindowLine)) + 16 <= kReservedLds, "reserved LDS");
