@@ -1575,13 +1575,26 @@ __device__ __forceinline__ int solve_origin(const KParams &kp, uint32_t o, uint3
     return 0;
 }
 
-/* One origin per wave.  With Jline set (the sparse solve) the origin's J stays in
-   LDS (or in its row of J, a scratch) and only its line integrals are written:
-   Jline(o, l) = sum_z w_z J(o, l Q + z) with the quadrature weights of line l's
-   species (lspec.J of Solver::solve_feautrier_order_2_sparse, solver.tpp:340-357). */
+/* line integrals of the sparse solve: Jline(o, l) = sum_z w_z J(o, l Q + z) with the
+   quadrature weights of line l's species (lspec.J of
+   Solver::solve_feautrier_order_2_sparse, solver.tpp:340-357) */
+__device__ inline double line_integral(const mgx_model &m, const double *Jo, uint32_t l)
+{
+    const uint32_t Q = m.nquads;
+    const double *w = &m.quad_weights[(size_t)m.line_species[l] * Q];
+    double acc = 0.0;
+    for (uint32_t z = 0; z < Q; z++) acc += w[z] * Jo[(size_t)l * Q + z];
+    return acc;
+}
+
+/* One origin and one group of per ray pairs per wave: block (o, g) takes ray pairs
+   g per .. g per + per - 1.  With several groups J and lam are their parts, (groups, P, F)
+   and (groups, P, L), which sum_parts_kernel adds up.  With Jline set (the sparse solve, one
+   group) the origin's J stays in LDS (or in its row of J, a scratch) and only its line
+   integrals are written. */
 template <int APPROX, int PREC>
 __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void feautrier_kernel(
-    const KParams *__restrict__ kpp, double *u, double *J, double *lam, double *Jline = nullptr)
+    const KParams *__restrict__ kpp, double *u, double *J, double *lam, double *Jline, uint32_t per)
 {
     mgx_ref_tables_init();
     const KParams &kp = *kpp;
@@ -1600,24 +1613,47 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void feautrier_
     double *s_L = reinterpret_cast<double *>(smem + acc_lds_offset(kp.cap, kp.stage));
     double *s_J = kp.j_lds ? s_L + L : nullptr;
     for (uint32_t i = lane; i < L + (s_J ? F : 0); i += MGX_WAVE) s_L[i] = 0.0;
-    if (solve_origin<APPROX, PREC>(kp, o, 0, m.hnrays, smem, s_erf, u, lam != nullptr, s_J,
-                                   s_J ? nullptr : J + (size_t)o * F, false, s_L))
+    const uint32_t rr0 = blockIdx.y * per, rr1 = rr0 + per < m.hnrays ? rr0 + per : m.hnrays;
+    const size_t row = (size_t)blockIdx.y * m.npoints + o;
+    if (solve_origin<APPROX, PREC>(kp, o, rr0, rr1, smem, s_erf, u, lam != nullptr, s_J,
+                                   s_J ? nullptr : J + row * F, false, s_L))
         return;
     if (Jline) {
         __syncthreads();
-        const double *Jo = s_J ? s_J : J + (size_t)o * F;
-        const uint32_t Q = m.nquads;
-        for (uint32_t l = lane; l < L; l += MGX_WAVE) {
-            const double *w = &m.quad_weights[(size_t)m.line_species[l] * Q];
-            double acc = 0.0;
-            for (uint32_t z = 0; z < Q; z++) acc += w[z] * Jo[(size_t)l * Q + z];
-            Jline[(size_t)o * L + l] = acc;
-        }
+        const double *Jo = s_J ? s_J : J + row * F;
+        for (uint32_t l = lane; l < L; l += MGX_WAVE) Jline[(size_t)o * L + l] = line_integral(m, Jo, l);
     } else if (s_J) {
-        for (uint32_t i = lane; i < F; i += MGX_WAVE) J[(size_t)o * F + i] = s_J[i];
+        for (uint32_t i = lane; i < F; i += MGX_WAVE) J[row * F + i] = s_J[i];
     }
     if (lam)
-        for (uint32_t i = lane; i < L; i += MGX_WAVE) lam[(size_t)o * L + i] = s_L[i];
+        for (uint32_t i = lane; i < L; i += MGX_WAVE) lam[row * L + i] = s_L[i];
+}
+
+/* Adds up the groups' parts of J (n_J = P F values each) and of the Lambda diagonal (n_L,
+   0 without it), group by group, into J and lam. */
+__global__ __launch_bounds__(256) void sum_parts_kernel(const double *Jp,
+                                                        const double *Lp, size_t n_J,
+                                                        size_t n_L, uint32_t groups, double *J, double *lam)
+{
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n_J + n_L) return;
+    const bool isJ = i < n_J;
+    const size_t n = isJ ? n_J : n_L, k = isJ ? i : i - n_J;
+    const double *p = isJ ? Jp : Lp;
+    double v = p[k];
+    for (uint32_t g = 1; g < groups; g++) v += p[g * n + k];
+    (isJ ? J : lam)[k] = v;
+}
+
+/* the sparse solve's line integrals from J (P, F) */
+__global__ __launch_bounds__(256) void line_integral_kernel(const KParams *__restrict__ kpp, const double *J,
+                                                            double *Jline)
+{
+    const mgx_model &m = kpp->m;
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (size_t)m.npoints * m.nlines) return;
+    const size_t o = i / m.nlines;
+    Jline[i] = line_integral(m, J + o * m.nfreqs, (uint32_t)(i % m.nlines));
 }
 
 /* The forward solve with the general Lambda operator: the bands of up to MGX_MAX_OFF_DIAG
@@ -1654,10 +1690,10 @@ __global__ __launch_bounds__(MGX_WAVE, 2) void feautrier_bands_kernel(
 }
 
 /* Order-0 short characteristics (Solver::solve_shortchar_order_0, solver.tpp:151-235):
-   the same grid, walk and segments as feautrier_kernel */
+   the same grid, walk, segments and parts as feautrier_kernel */
 template <int APPROX, int PREC>
 __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void shortchar_kernel(
-    const KParams *__restrict__ kpp, ShortcharOut sc, double *u, double *J, double *lam)
+    const KParams *__restrict__ kpp, ShortcharOut sc, double *u, double *J, double *lam, uint32_t per)
 {
     mgx_ref_tables_init();
     const KParams &kp = *kpp;
@@ -1676,21 +1712,23 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void shortchar_
     double *s_L = reinterpret_cast<double *>(smem + acc_lds_offset(kp.cap, kp.stage));
     double *s_J = kp.j_lds ? s_L + L : nullptr;
     for (uint32_t i = lane; i < L + (s_J ? F : 0); i += MGX_WAVE) s_L[i] = 0.0;
-    if (solve_origin<APPROX, PREC, METHOD_SHORTCHAR>(kp, o, 0, m.hnrays, smem, s_erf, u,
-                                                     lam != nullptr, s_J, J + (size_t)o * F,
+    const uint32_t rr0 = blockIdx.y * per, rr1 = rr0 + per < m.hnrays ? rr0 + per : m.hnrays;
+    const size_t row = (size_t)blockIdx.y * m.npoints + o;
+    if (solve_origin<APPROX, PREC, METHOD_SHORTCHAR>(kp, o, rr0, rr1, smem, s_erf, u,
+                                                     lam != nullptr, s_J, J + row * F,
                                                      false, s_L, sc))
         return;
     if (s_J)
-        for (uint32_t i = lane; i < F; i += MGX_WAVE) J[(size_t)o * F + i] = s_J[i];
+        for (uint32_t i = lane; i < F; i += MGX_WAVE) J[row * F + i] = s_J[i];
     if (lam)
-        for (uint32_t i = lane; i < L; i += MGX_WAVE) lam[(size_t)o * L + i] = s_L[i];
+        for (uint32_t i = lane; i < L; i += MGX_WAVE) lam[row * L + i] = s_L[i];
 }
 
 /* Feautrier order 2 with v (Solver::solve_feautrier_order_2_uv, solver.tpp:238-295,
    2767-2921): u and v only */
 template <int APPROX, int PREC>
 __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void feautrier_uv_kernel(
-    const KParams *__restrict__ kpp, double *u, double *v)
+    const KParams *__restrict__ kpp, double *u, double *v, uint32_t per)
 {
     mgx_ref_tables_init();
     const KParams &kp = *kpp;
@@ -1699,7 +1737,8 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void feautrier_
     const uint32_t o = blockIdx.x;
     double *s_L = reinterpret_cast<double *>(smem + acc_lds_offset(kp.cap, kp.stage));
     ShortcharOut sc{nullptr, v, 0.0};
-    solve_origin<APPROX, PREC, METHOD_UV>(kp, o, 0, kp.m.hnrays, smem, s_erf, u, false, nullptr,
+    const uint32_t rr0 = blockIdx.y * per, rr1 = rr0 + per < kp.m.hnrays ? rr0 + per : kp.m.hnrays;
+    solve_origin<APPROX, PREC, METHOD_UV>(kp, o, rr0, rr1, smem, s_erf, u, false, nullptr,
                                           nullptr, false, s_L, sc);
 }
 
@@ -3995,6 +4034,7 @@ struct DevBuffers {
     uint32_t *status = nullptr;
     KParams *kp_dev = nullptr; /* device copy of the launch parameters */
     ImageFrame *frame = nullptr; /* the imager's frame (carved with the rest) */
+    double *parts = nullptr;     /* the ray-pair groups' parts of J and Lambda (carved) */
     bool owned = true;         /* false: carved out of a shared buffer */
     std::unique_lock<std::mutex> ws_lock; /* held while carved from the call workspace */
     ~DevBuffers()
@@ -4128,7 +4168,7 @@ namespace {
 /* the tables of model m in b: from the call workspace, or (persistent, for objects
    that keep them, such as a batch) in allocations of their own */
 int prepare(const mgx_model *m, const mgx_options *op, hipStream_t st, DevBuffers &b, KParams &kp,
-            bool persistent = false)
+            bool persistent = false, size_t parts_bytes = 0)
 {
     const size_t P = m->npoints, PL = (size_t)m->npoints * m->nlines;
     if (persistent) {
@@ -4142,7 +4182,7 @@ int prepare(const mgx_model *m, const mgx_options *op, hipStream_t st, DevBuffer
     const auto rnd = [](size_t n) { return (n + 255) & ~(size_t)255; };
     const size_t need = rnd(PL * sizeof(double4)) + rnd(P * sizeof(PointRec)) +
                         rnd(P * sizeof(PointIdx)) + rnd(4 * sizeof(uint32_t)) +
-                        rnd(sizeof(KParams)) + rnd(sizeof(ImageFrame));
+                        rnd(sizeof(KParams)) + rnd(sizeof(ImageFrame)) + rnd(parts_bytes);
     b.ws_lock = std::unique_lock<std::mutex>(g_prep_mutex);
     int dev = 0;
     HIP_TRY(hipGetDevice(&dev));
@@ -4168,6 +4208,8 @@ int prepare(const mgx_model *m, const mgx_options *op, hipStream_t st, DevBuffer
     b.kp_dev = reinterpret_cast<KParams *>(q);
     q += rnd(sizeof(KParams));
     b.frame = reinterpret_cast<ImageFrame *>(q);
+    q += rnd(sizeof(ImageFrame));
+    b.parts = reinterpret_cast<double *>(q);
     return prepare_tables(m, op, st, b, kp);
 }
 
@@ -4948,16 +4990,74 @@ const char *mgx_version(void) { return "magritte_amd 0.1.0 (gfx950)"; }
 
 namespace {
 
+/*
+ * How a solve splits the ray pairs of an origin over waves.  One wave per origin
+ * leaves the GPU idle when there are few origins (3072 waves are resident at once) and
+ * ends with a long tail when there are not many more; kSplitWaves waves fill it about
+ * five times over.  Splitting costs a pass over the parts of J and Lambda, and memory for
+ * them, so the groups are as few as reach that count, and their parts have to fit the
+ * no-allocation solve's scratch beside its tables (both entry points then add up in the
+ * same order and give the same bits).  Measured: 250 shells, 100 ray pairs
+ * 39.8 -> 9.2 ms; 20^3 wind (3 groups), short
+ * characteristics, 3.12 -> 2.92 ms; from
+ * 16384 origins on nothing is split.
+ */
+constexpr uint32_t kSplitWaves = 16384;
+
+struct RaySplit {
+    uint32_t per, groups; /* ray pairs per group, groups */
+    size_t bytes;         /* parts of J and Lambda (0: none) */
+};
+
+size_t noalloc_scratch_bytes(const mgx_model *model)
+{
+    const size_t P = model->npoints, PL = (size_t)model->npoints * model->nlines;
+    const auto rnd = [](size_t n) { return (n + 255) & ~(size_t)255; };
+    return rnd(4 * sizeof(uint32_t)) + rnd(sizeof(KParams)) + rnd(P * sizeof(PointRec)) +
+           rnd(P * sizeof(PointIdx)) + rnd(PL * sizeof(double4));
+}
+
+RaySplit ray_split(const mgx_model &m)
+{
+    RaySplit r{m.hnrays, 1, 0};
+    const uint64_t P = m.npoints;
+    uint64_t g = (kSplitWaves + P - 1) / P;
+    if (g > m.hnrays) g = m.hnrays;
+    const size_t part = (size_t)P * ((size_t)m.nfreqs + m.nlines) * sizeof(double);
+    const size_t used = noalloc_scratch_bytes(&m) + 256;
+    const size_t room = used < (size_t)MGX_NOALLOC_SCRATCH_BYTES ? (size_t)MGX_NOALLOC_SCRATCH_BYTES - used : 0;
+    if (g > room / part) g = room / part;
+    if (g < 2) return r;
+    r.per = (uint32_t)((m.hnrays + g - 1) / g);
+    r.groups = (m.hnrays + r.per - 1) / r.per;
+    if (r.groups > 1) r.bytes = r.groups * part;
+    return r;
+}
+
+/* adds the groups' parts at b.parts up into J and lam */
+void sum_parts(const mgx_model &m, const RaySplit &sp, const DevBuffers &b, double *J, double *lam,
+               hipStream_t st)
+{
+    const size_t nJ = (size_t)m.npoints * m.nfreqs, nL = lam ? (size_t)m.npoints * m.nlines : 0;
+    hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((nJ + nL + 255) / 256)), dim3(256), 0, st, b.parts,
+                       b.parts + sp.groups * nJ, nJ, nL, sp.groups, J, lam);
+}
+
 /* the plain-method solve on prepared buffers (shared by the allocating and the
    no-allocation entry points) */
 int forward_launch(const mgx_model *model, const mgx_options *opts, double *u, double *J_out,
-                   double *lambda_diag, hipStream_t st, DevBuffers &b, KParams &kp,
-                   double *Jline = nullptr, double **J_scratch = nullptr)
+                   double *lambda_out, hipStream_t st, DevBuffers &b, KParams &kp,
+                   const RaySplit &sp, double *Jline_out = nullptr, double **J_scratch = nullptr)
 {
     bool scratch_failed = false;
     const int e = launch_with_capacity(st, b, kp, [&](size_t) {
         /* the line-integrated solve keeps J in LDS, or else in a scratch J (P, F) */
-        double *J = J_out;
+        double *J = J_out, *lambda_diag = lambda_out, *Jline = Jline_out;
+        if (sp.groups > 1) {
+            J = b.parts;
+            lambda_diag = lambda_out ? b.parts + (size_t)sp.groups * model->npoints * model->nfreqs : nullptr;
+            Jline = nullptr; /* from the sum of the parts */
+        }
         if (Jline && !kp.j_lds) {
             if (!*J_scratch &&
                 hipMalloc(J_scratch, (size_t)model->npoints * model->nfreqs * sizeof(double)) !=
@@ -4967,7 +5067,7 @@ int forward_launch(const mgx_model *model, const mgx_options *opts, double *u, d
             }
             J = *J_scratch;
         }
-        const dim3 grid(model->npoints), block(MGX_WAVE);
+        const dim3 grid(model->npoints, sp.groups), block(MGX_WAVE);
         const size_t lds = solve_lds_bytes(kp.cap, kp.stage, model->nfreqs, model->nlines, kp.j_lds != 0);
         timed(st, [&] {
             const bool fp64 = opts->precision == MGX_PREC_FP64;
@@ -4975,26 +5075,34 @@ int forward_launch(const mgx_model *model, const mgx_options *opts, double *u, d
             case MGX_APPROX_NONE:
                 if (fp64)
                     hipLaunchKernelGGL((feautrier_kernel<MGX_APPROX_NONE, MGX_PREC_FP64>), grid,
-                                       block, lds, st, b.kp_dev, u, J, lambda_diag, Jline);
+                                       block, lds, st, b.kp_dev, u, J, lambda_diag, Jline, sp.per);
                 else
                     hipLaunchKernelGGL((feautrier_kernel<MGX_APPROX_NONE, MGX_PREC_MIXED>), grid,
-                                       block, lds, st, b.kp_dev, u, J, lambda_diag, Jline);
+                                       block, lds, st, b.kp_dev, u, J, lambda_diag, Jline, sp.per);
                 break;
             case MGX_APPROX_ONE_LINE:
                 if (fp64)
                     hipLaunchKernelGGL((feautrier_kernel<MGX_APPROX_ONE_LINE, MGX_PREC_FP64>), grid,
-                                       block, lds, st, b.kp_dev, u, J, lambda_diag, Jline);
+                                       block, lds, st, b.kp_dev, u, J, lambda_diag, Jline, sp.per);
                 else
                     hipLaunchKernelGGL((feautrier_kernel<MGX_APPROX_ONE_LINE, MGX_PREC_MIXED>),
-                                       grid, block, lds, st, b.kp_dev, u, J, lambda_diag, Jline);
+                                       grid, block, lds, st, b.kp_dev, u, J, lambda_diag, Jline, sp.per);
                 break;
             default:
                 if (fp64)
                     hipLaunchKernelGGL((feautrier_kernel<MGX_APPROX_CLOSE_LINES, MGX_PREC_FP64>),
-                                       grid, block, lds, st, b.kp_dev, u, J, lambda_diag, Jline);
+                                       grid, block, lds, st, b.kp_dev, u, J, lambda_diag, Jline, sp.per);
                 else
                     hipLaunchKernelGGL((feautrier_kernel<MGX_APPROX_CLOSE_LINES, MGX_PREC_MIXED>),
-                                       grid, block, lds, st, b.kp_dev, u, J, lambda_diag, Jline);
+                                       grid, block, lds, st, b.kp_dev, u, J, lambda_diag, Jline, sp.per);
+            }
+            if (sp.groups > 1) {
+                /* the sparse solve's J goes into the first group's part */
+                sum_parts(*model, sp, b, Jline_out ? b.parts : J_out, lambda_out, st);
+                if (Jline_out)
+                    hipLaunchKernelGGL(line_integral_kernel,
+                                       dim3((unsigned)(((size_t)model->npoints * model->nlines + 255) / 256)),
+                                       dim3(256), 0, st, b.kp_dev, b.parts, Jline_out);
             }
         });
     }, 8 * (size_t)model->nlines, true);
@@ -5014,8 +5122,9 @@ int mgx_feautrier_forward_device(const mgx_model *model, const mgx_options *opts
     hipStream_t st = (hipStream_t)stream;
     DevBuffers b;
     KParams kp;
-    if (int e = prepare(model, opts, st, b, kp)) return e;
-    return forward_launch(model, opts, u, J, lambda_diag, st, b, kp);
+    const RaySplit sp = ray_split(*model);
+    if (int e = prepare(model, opts, st, b, kp, false, sp.bytes)) return e;
+    return forward_launch(model, opts, u, J, lambda_diag, st, b, kp, sp);
 }
 
 int mgx_feautrier_sparse_device(const mgx_model *model, const mgx_options *opts, double *J_line,
@@ -5043,7 +5152,8 @@ int mgx_feautrier_sparse_device(const mgx_model *model, const mgx_options *opts,
     }
     DevBuffers b;
     KParams kp;
-    if (int e = prepare(model, opts, st, b, kp)) return e;
+    const RaySplit sp = ray_split(*model);
+    if (int e = prepare(model, opts, st, b, kp, false, sp.bytes)) return e;
     /* J of an origin stays in LDS; when it does not fit (long walks), its row of a
        scratch J, allocated by the launch that needs it */
     double *Jtmp = nullptr;
@@ -5051,16 +5161,7 @@ int mgx_feautrier_sparse_device(const mgx_model *model, const mgx_options *opts,
         double *&p;
         ~Free() { if (p) (void)hipFree(p); }
     } free_tmp{Jtmp};
-    return forward_launch(model, opts, nullptr, nullptr, lambda_diag, st, b, kp, J_line, &Jtmp);
-}
-
-static size_t noalloc_scratch_bytes(const mgx_model *model)
-{
-    if (!model) return 0;
-    const size_t P = model->npoints, PL = (size_t)model->npoints * model->nlines;
-    const auto rnd = [](size_t n) { return (n + 255) & ~(size_t)255; };
-    return rnd(4 * sizeof(uint32_t)) + rnd(sizeof(KParams)) + rnd(P * sizeof(PointRec)) +
-           rnd(P * sizeof(PointIdx)) + rnd(PL * sizeof(double4));
+    return forward_launch(model, opts, nullptr, nullptr, lambda_diag, st, b, kp, sp, J_line, &Jtmp);
 }
 
 int mgx_feautrier_forward_noalloc(const mgx_model *model, const mgx_options *opts, double *u,
@@ -5093,6 +5194,8 @@ int mgx_feautrier_forward_noalloc(const mgx_model *model, const mgx_options *opt
     b.pts = reinterpret_cast<PointRec *>(take(P * sizeof(PointRec)));
     b.pidx = reinterpret_cast<PointIdx *>(take(P * sizeof(PointIdx)));
     b.lpack = reinterpret_cast<double4 *>(take(PL * sizeof(double4)));
+    const RaySplit sp = ray_split(*model);
+    b.parts = reinterpret_cast<double *>(take(sp.bytes));
     struct NoEvents {
         NoEvents() { t_no_events = true; }
         ~NoEvents() { t_no_events = false; }
@@ -5100,7 +5203,7 @@ int mgx_feautrier_forward_noalloc(const mgx_model *model, const mgx_options *opt
     hipStream_t st = (hipStream_t)stream;
     KParams kp;
     if (int e = prepare_tables(model, opts, st, b, kp)) return e;
-    return forward_launch(model, opts, u, J, lambda_diag, st, b, kp);
+    return forward_launch(model, opts, u, J, lambda_diag, st, b, kp, sp);
 }
 
 int mgx_feautrier_forward_lambda_device(const mgx_model *model, const mgx_options *opts,
@@ -5166,10 +5269,14 @@ int mgx_shortchar_order_0_device(const mgx_model *model, const mgx_options *opts
     hipStream_t st = (hipStream_t)stream;
     DevBuffers b;
     KParams kp;
-    if (int e = prepare(model, opts, st, b, kp)) return e;
+    const RaySplit sp = ray_split(*model);
+    if (int e = prepare(model, opts, st, b, kp, false, sp.bytes)) return e;
     const ShortcharOut sc{I, v, min_dtau};
     return launch_with_capacity(st, b, kp, [&](size_t) {
-        const dim3 grid(model->npoints), block(MGX_WAVE);
+        const dim3 grid(model->npoints, sp.groups), block(MGX_WAVE);
+        double *Jp = sp.groups > 1 ? b.parts : J;
+        double *Lp = sp.groups > 1 && lambda_diag ? b.parts + (size_t)sp.groups * model->npoints * model->nfreqs
+                                                  : lambda_diag;
         const size_t lds = solve_lds_bytes(kp.cap, kp.stage, model->nfreqs, model->nlines, kp.j_lds != 0);
         timed(st, [&] {
             const bool fp64 = opts->precision == MGX_PREC_FP64;
@@ -5177,27 +5284,28 @@ int mgx_shortchar_order_0_device(const mgx_model *model, const mgx_options *opts
             case MGX_APPROX_NONE:
                 if (fp64)
                     hipLaunchKernelGGL((shortchar_kernel<MGX_APPROX_NONE, MGX_PREC_FP64>), grid,
-                                       block, lds, st, b.kp_dev, sc, u, J, lambda_diag);
+                                       block, lds, st, b.kp_dev, sc, u, Jp, Lp, sp.per);
                 else
                     hipLaunchKernelGGL((shortchar_kernel<MGX_APPROX_NONE, MGX_PREC_MIXED>), grid,
-                                       block, lds, st, b.kp_dev, sc, u, J, lambda_diag);
+                                       block, lds, st, b.kp_dev, sc, u, Jp, Lp, sp.per);
                 break;
             case MGX_APPROX_ONE_LINE:
                 if (fp64)
                     hipLaunchKernelGGL((shortchar_kernel<MGX_APPROX_ONE_LINE, MGX_PREC_FP64>), grid,
-                                       block, lds, st, b.kp_dev, sc, u, J, lambda_diag);
+                                       block, lds, st, b.kp_dev, sc, u, Jp, Lp, sp.per);
                 else
                     hipLaunchKernelGGL((shortchar_kernel<MGX_APPROX_ONE_LINE, MGX_PREC_MIXED>),
-                                       grid, block, lds, st, b.kp_dev, sc, u, J, lambda_diag);
+                                       grid, block, lds, st, b.kp_dev, sc, u, Jp, Lp, sp.per);
                 break;
             default:
                 if (fp64)
                     hipLaunchKernelGGL((shortchar_kernel<MGX_APPROX_CLOSE_LINES, MGX_PREC_FP64>),
-                                       grid, block, lds, st, b.kp_dev, sc, u, J, lambda_diag);
+                                       grid, block, lds, st, b.kp_dev, sc, u, Jp, Lp, sp.per);
                 else
                     hipLaunchKernelGGL((shortchar_kernel<MGX_APPROX_CLOSE_LINES, MGX_PREC_MIXED>),
-                                       grid, block, lds, st, b.kp_dev, sc, u, J, lambda_diag);
+                                       grid, block, lds, st, b.kp_dev, sc, u, Jp, Lp, sp.per);
             }
+            if (sp.groups > 1) sum_parts(*model, sp, b, J, lambda_diag, st);
         });
     }, 8 * (size_t)model->nlines, true);
 }
@@ -5212,8 +5320,9 @@ int mgx_feautrier_order_2_uv_device(const mgx_model *model, const mgx_options *o
     DevBuffers b;
     KParams kp;
     if (int e = prepare(model, opts, st, b, kp)) return e;
+    const RaySplit sp = ray_split(*model); /* no parts: u and v are per ray pair */
     return launch_with_capacity(st, b, kp, [&](size_t) {
-        const dim3 grid(model->npoints), block(MGX_WAVE);
+        const dim3 grid(model->npoints, sp.groups), block(MGX_WAVE);
         const size_t lds = solve_lds_bytes(kp.cap, kp.stage, model->nfreqs, model->nlines, false);
         timed(st, [&] {
             const bool fp64 = opts->precision == MGX_PREC_FP64;
@@ -5221,26 +5330,26 @@ int mgx_feautrier_order_2_uv_device(const mgx_model *model, const mgx_options *o
             case MGX_APPROX_NONE:
                 if (fp64)
                     hipLaunchKernelGGL((feautrier_uv_kernel<MGX_APPROX_NONE, MGX_PREC_FP64>), grid,
-                                       block, lds, st, b.kp_dev, u, v);
+                                       block, lds, st, b.kp_dev, u, v, sp.per);
                 else
                     hipLaunchKernelGGL((feautrier_uv_kernel<MGX_APPROX_NONE, MGX_PREC_MIXED>), grid,
-                                       block, lds, st, b.kp_dev, u, v);
+                                       block, lds, st, b.kp_dev, u, v, sp.per);
                 break;
             case MGX_APPROX_ONE_LINE:
                 if (fp64)
                     hipLaunchKernelGGL((feautrier_uv_kernel<MGX_APPROX_ONE_LINE, MGX_PREC_FP64>),
-                                       grid, block, lds, st, b.kp_dev, u, v);
+                                       grid, block, lds, st, b.kp_dev, u, v, sp.per);
                 else
                     hipLaunchKernelGGL((feautrier_uv_kernel<MGX_APPROX_ONE_LINE, MGX_PREC_MIXED>),
-                                       grid, block, lds, st, b.kp_dev, u, v);
+                                       grid, block, lds, st, b.kp_dev, u, v, sp.per);
                 break;
             default:
                 if (fp64)
                     hipLaunchKernelGGL((feautrier_uv_kernel<MGX_APPROX_CLOSE_LINES, MGX_PREC_FP64>),
-                                       grid, block, lds, st, b.kp_dev, u, v);
+                                       grid, block, lds, st, b.kp_dev, u, v, sp.per);
                 else
                     hipLaunchKernelGGL((feautrier_uv_kernel<MGX_APPROX_CLOSE_LINES, MGX_PREC_MIXED>),
-                                       grid, block, lds, st, b.kp_dev, u, v);
+                                       grid, block, lds, st, b.kp_dev, u, v, sp.per);
             }
         });
     }, 8 * (size_t)model->nlines, true);
