@@ -396,6 +396,134 @@ __device__ int walk_half(const KParams &kp, uint32_t o, uint32_t r, uint32_t *s_
     return 0;
 }
 
+/* A value of the even and of the odd row of 16 of each half of the wave, in every lane of
+   that half (v_permlane16_swap: the odd rows of the first operand change places with the
+   even rows of the second). */
+template <typename T>
+__device__ __forceinline__ void half_rows(T v, T &even, T &odd)
+{
+    static_assert(sizeof(T) == 4 || sizeof(T) == 8, "one or two words");
+    constexpr int n = sizeof(T) / 4;
+    uint32_t w[n], e[n], o[n];
+    __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+    for (int i = 0; i < n; i++) {
+        const auto r = __builtin_amdgcn_permlane16_swap(w[i], w[i], false, false);
+        e[i] = r[0];
+        o[i] = r[1];
+    }
+    __builtin_memcpy(&even, e, sizeof(T));
+    __builtin_memcpy(&odd, o, sizeof(T));
+}
+
+/* a neighbour on its way through the arg-min of a half-wave: smaller d2 wins, ties go to
+   the smaller list index */
+struct NextPoint {
+    double d2, zn;
+    uint32_t idx, n;
+};
+
+__device__ __forceinline__ void next_take(NextPoint &a, const NextPoint &b)
+{
+    if (b.d2 < a.d2 || (b.d2 == a.d2 && b.idx < a.idx)) a = b;
+}
+
+template <int CTRL>
+__device__ __forceinline__ void next_dpp(NextPoint &a)
+{
+    next_take(a, NextPoint{dpp_get<CTRL>(a.d2), dpp_get<CTRL>(a.zn), dpp_get<CTRL>(a.idx), dpp_get<CTRL>(a.n)});
+}
+
+/*
+ * Both half rays of a ray pair at once: lanes 0-31 walk from o along ray rr into the first
+ * list, lanes 32-63 along its antipod ar into the second (walk_half's steps, lists and
+ * error codes).  A walk is a chain of dependent gathers (the list, its points, the next
+ * point's list) and a point has some 15 neighbours, so a whole wave per half ray left
+ * three quarters of its lanes idle through twice as many of them (32^3 wind, mixed,
+ * 14.5 -> 13.4 ms; 250 shells 9.2 -> 7.0 ms).  S and shift0 are those of the lane's half
+ * ray.
+ */
+__device__ int walk_pair(const KParams &kp, uint32_t o, uint32_t rr, uint32_t ar, unsigned char *smem,
+                         uint32_t &S, double &shift0)
+{
+    const mgx_model &m = kp.m;
+    const uint32_t q = threadIdx.x & 31, half = (threadIdx.x & (MGX_WAVE - 1)) >> 5;
+    const uint32_t r = half ? ar : rr;
+    uint32_t *s_nxt = reinterpret_cast<uint32_t *>(smem) + half * kp.cap;
+    double *s_dZ = reinterpret_cast<double *>(smem + 8 * ((2 * kp.cap * 4 + 7) / 8)) + half * kp.cap;
+    double *s_sh = s_dZ + 2 * kp.cap;
+    const PointRec po = gld(&kp.pts[o]);
+    const double origin[3] = {po.x, po.y, po.z};
+    const double ovel[3] = {po.vx, po.vy, po.vz};
+    const double *dp = ray_dir(m, o, r);
+    const double dir[3] = {gld(&dp[0]), gld(&dp[1]), gld(&dp[2])};
+    double Z = 0.0, dZ = 0.0;
+    uint32_t crt = o;
+    S = 0;
+    shift0 = shift_comoving(kp, origin, ovel, dir, o, 0.0);
+    PointIdx pc = gld(&kp.pidx[o]);
+    int err = 0;
+    bool go = true;
+    while (go) {
+        uint32_t nxt;
+        if (m.spherical_symmetry) {
+            nxt = next_spherical(kp, origin, dir, crt, Z, dZ);
+        } else {
+            /* get_next_general_geometry<Defaulttracer> (geometry.tpp:14-44) */
+            NextPoint best = {__builtin_inf(), 0.0, 0xffffffffu, m.npoints};
+            for (uint32_t i = q; i < pc.n_nbs; i += 32) {
+                const uint32_t n = gld(&m.neighbors[pc.cum + i]);
+                const PointPos pn = gld(reinterpret_cast<const PointPos *>(&kp.pts[n]));
+                double R[3];
+                R[0] = pn.x - origin[0];
+                R[1] = pn.y - origin[1];
+                R[2] = pn.z - origin[2];
+                const double Z_new = dot3(R, dir);
+                if (Z_new > Z) {
+                    const double d2 = dot3(R, R) - Z_new * Z_new;
+                    if (d2 < DBL_MAX && d2 < best.d2) best = NextPoint{d2, Z_new, i, n};
+                }
+            }
+            next_dpp<0xb1>(best);
+            next_dpp<0x4e>(best);
+            next_dpp<0x141>(best);
+            next_dpp<0x140>(best);
+            NextPoint odd;
+            half_rows(best.d2, best.d2, odd.d2);
+            half_rows(best.zn, best.zn, odd.zn);
+            half_rows(best.idx, best.idx, odd.idx);
+            half_rows(best.n, best.n, odd.n);
+            next_take(best, odd);
+            nxt = best.n;
+            if (best.idx != 0xffffffffu) {
+                dZ = best.zn - Z;
+                Z += dZ;
+            }
+        }
+        if (nxt >= m.npoints) {
+            if (S != 0) err = ERR_NO_NEXT; /* else nothing in this direction */
+            go = false;
+        } else if (S >= kp.cap) {
+            err = ERR_CAP;
+            go = false;
+        } else {
+            /* the next point's record serves the boundary test and the next step */
+            pc = gld(&kp.pidx[nxt]);
+            const double sh = shift_comoving(kp, origin, ovel, dir, nxt, Z);
+            if (q == 0) {
+                s_nxt[S] = nxt;
+                s_dZ[S] = dZ;
+                s_sh[S] = sh;
+            }
+            S++;
+            crt = nxt;
+            go = pc.p2b == m.npoints; /* until the boundary */
+        }
+    }
+    const int e0 = __builtin_amdgcn_readlane(err, 0), e1 = __builtin_amdgcn_readlane(err, 32);
+    return e0 ? e0 : e1;
+}
+
 /* ------------------------------------------------------------------------- */
 /* per-line interpolation count (InterpHelper::get_n_interp_for_line, :55-75)  */
 
@@ -1237,23 +1365,15 @@ __device__ __forceinline__ int solve_origin(const KParams &kp, uint32_t o, uint3
     const uint32_t lane = threadIdx.x;
     const uint32_t cap = kp.cap;
     const uint32_t P = m.npoints, F = m.nfreqs, Q = m.nquads;
-    uint32_t *s_nxt0 = reinterpret_cast<uint32_t *>(smem);
-    uint32_t *s_nxt1 = s_nxt0 + cap;
-    double *s_dZ0 = reinterpret_cast<double *>(smem + 8 * ((2 * cap * 4 + 7) / 8));
-    double *s_dZ1 = s_dZ0 + cap;
-    double *s_sh0 = s_dZ1 + cap;
-    double *s_sh1 = s_sh0 + cap;
-    uint32_t *s_pre = reinterpret_cast<uint32_t *>(s_sh1 + cap); /* [group][step] */
     const uint32_t grp = lane >> 5;
     StagedEntry *chunk = reinterpret_cast<StagedEntry *>(smem + stage_lds_offset(cap)) + grp * kp.stage;
     const size_t PF = (size_t)P * F;
 
     for (uint32_t rr = rr0; rr < rr1; rr++) {
         const uint32_t ar = gld(&m.antipod[rr]);
-        uint32_t S0, S1;
-        double sh00, sh01;
-        int e = walk_half(kp, o, rr, s_nxt0, s_dZ0, s_sh0, S0, sh00);
-        if (!e) e = walk_half(kp, o, ar, s_nxt1, s_dZ1, s_sh1, S1, sh01);
+        uint32_t S;
+        double shift0;
+        const int e = walk_pair(kp, o, rr, ar, smem, S, shift0);
         if (e) {
             if (lane == 0) {
                 atomicOr(&kp.status[0], (uint32_t)e);
@@ -1262,6 +1382,9 @@ __device__ __forceinline__ int solve_origin(const KParams &kp, uint32_t o, uint3
             return e;
         }
         __syncthreads();
+        const uint32_t S0 = (uint32_t)__builtin_amdgcn_readlane((int)S, 0);
+        const uint32_t S1 = (uint32_t)__builtin_amdgcn_readlane((int)S, 32);
+        const double sh00 = read_lane(shift0, 0), sh01 = read_lane(shift0, 32);
         const double w = ray_weight(m, o, rr);
 
         for (uint32_t slot0 = 0; slot0 < kp.nslots; slot0 += 2) {
@@ -1631,8 +1754,7 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void feautrier_
 
 /* Adds up the groups' parts of J (n_J = P F values each) and of the Lambda diagonal (n_L,
    0 without it), group by group, into J and lam. */
-__global__ __launch_bounds__(256) void sum_parts_kernel(const double *Jp,
-                                                        const double *Lp, size_t n_J,
+__global__ __launch_bounds__(256) void sum_parts_kernel(const double *Jp, const double *Lp, size_t n_J,
                                                         size_t n_L, uint32_t groups, double *J, double *lam)
 {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;

@@ -83,7 +83,9 @@ __device__ __forceinline__ double group32(double v, Op op)
     v = op(v, dpp_get<0x4e>(v));
     v = op(v, dpp_get<0x141>(v));
     v = op(v, dpp_get<0x140>(v));
-    return op(v, __shfl_xor(v, 16, MGX_WAVE));
+    double even, odd;
+    half_rows(v, even, odd);
+    return op(even, odd);
 }
 
 /* Interpolation counts of the groups' half rays (o, line, S and list of *g are set):

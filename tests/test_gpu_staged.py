@@ -1,0 +1,54 @@
+"""The staged sweeps of the formal solves at their edges, against the oracle: rays whose
+entries end on, one before and one after a chunk of staged entries, quadratures around a
+half-wave's 32 lanes, an odd and an even number of lines, windows with more lines than a
+group takes side by side, interpolated entries across chunks, and ray pairs split over
+waves or not.  FP64 mode differs from the oracle by a few roundings per row (1e-10
+relative, as the other parity tests)."""
+import numpy as np
+import pytest
+
+from magritte_amd import _abi, models
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(m, op):
+    from magritte_amd import solver
+    from oracle import oracle
+
+    out = solver.feautrier_forward(solver.DeviceModel(m), op)
+    u, J, lam = (out[k].cpu().numpy() for k in ("u", "J", "lambda_diag"))
+    for name, a, b in zip(("u", "J", "lambda"), (u, J, lam), oracle.solve(m, op)):
+        assert np.all(np.isfinite(a)), name
+        err = float(np.max(np.abs(a - b) / np.maximum(np.abs(b), 1e-300)))
+        assert err < 1e-10, f"{name}: {err:.2e}"
+
+
+@pytest.mark.parametrize("npoints", [2, 3, 31, 32, 33, 34, 63, 64, 95])
+@pytest.mark.parametrize("nquads", [1, 31, 32, 33, 65])
+def test_chunk_and_half_wave_edges(npoints, nquads):
+    print(f"[staged] line {npoints} points {nquads} bins", flush=True)
+    m = models.model_line_1d(npoints=npoints, nquads=nquads)
+    _check(m, m.options())
+
+
+@pytest.mark.parametrize("approx", [_abi.APPROX_NONE, _abi.APPROX_ONE_LINE, _abi.APPROX_CLOSE_LINES])
+@pytest.mark.parametrize("nlines", [1, 2, 5, 17])
+def test_blended_windows(approx, nlines):
+    """lines a width or two apart: more than 16 of them go through two rounds of a window"""
+    print(f"[staged] {nlines} blended lines approx {approx}", flush=True)
+    clumps = np.exp(0.5 * np.random.Generator(np.random.PCG64(5)).standard_normal(5**3))
+    m = models.model_wind(n_edge=5, nrays=12, nquads=7, clumps=clumps, v_out=1.5e3)
+    ld = models.linedata_blended(115.0e9, [1.5e-6 * (k + 1) for k in range(nlines - 1)], A=1.0e-7)
+    m.set_lines([ld], 7)
+    m.finalize()
+    _check(m, m.options(approx=approx))
+
+
+def test_interpolated_entries_across_chunks():
+    """a clumpy wind with many interpolated entries: several chunks per half ray"""
+    clumps = np.exp(2.0 * np.random.Generator(np.random.PCG64(6)).standard_normal(7**3))
+    m = models.model_wind(n_edge=7, nrays=12, nquads=9, nlev=4, clumps=clumps)
+    m.params["max_interpolation_diff"] = 1.02
+    print("[staged] interpolated chunks", flush=True)
+    _check(m, m.options())
