@@ -155,7 +155,8 @@ int mgx_feautrier_sparse_device(const mgx_model *model_dev, const mgx_options *o
  * capture, tight serving loops, harnesses that forbid hipMalloc.
  * Its scratch (status words, launch parameters and the packed point and line
  * tables: 256-byte-aligned pieces of 16 B, the parameter block, 80 B per point
- * and 32 B per (point, line)) lives in a static device array of
+ * and 32 B per (point, line); where they fit beside them, the ray pairs' parts
+ * of J and Lambda of a model small enough to be split) lives in a static device array of
  * MGX_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends; a model
  * needing more fails with MGX_E_ARG (e.g. 64 MiB holds the 32^3 wind with 9
  * lines, 12 MB).  The caller passes the inputs and outputs as for

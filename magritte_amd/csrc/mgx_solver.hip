@@ -1079,6 +1079,7 @@ inline uint32_t stage_entries(uint32_t cap, uint32_t L)
    several waves add atomically into a cleared row */
 __device__ inline void j_add(double *Jrow, uint32_t f, double c, bool first, bool atomic)
 {
+    if (!Jrow) return; /* the sum is taken from u */
     if (atomic)
         unsafeAtomicAdd(&Jrow[f], c);
     else
@@ -1387,6 +1388,10 @@ __device__ __forceinline__ int solve_origin(const KParams &kp, uint32_t o, uint3
         const double sh00 = read_lane(shift0, 0), sh01 = read_lane(shift0, 32);
         const double w = ray_weight(m, o, rr);
 
+        /* the ray pair's sum of the line whose slots are passing (a line's slots follow one
+           another), added to the line's total when the next line comes */
+        uint32_t lam_line = 0;
+        double lam_sum = 0.0;
         for (uint32_t slot0 = 0; slot0 < kp.nslots; slot0 += 2) {
             /* two line slots at a time, one per group, each half ray in turn; the last
                slot of an odd number is left alone: then each group takes one of its
@@ -1626,19 +1631,24 @@ __device__ __forceinline__ int solve_origin(const KParams &kp, uint32_t o, uint3
                 if (METHOD == METHOD_UV && sc.v) sc.v[(size_t)rr * PF + of] = vc;
                 }
             }
-            /* per-line sum of the Lambda contributions over the 32 lanes of a slot;
-               lane 0 then adds both slots of the pass in order (they may share a line) */
+            /* per-line sum of the Lambda contributions over the 32 lanes of a slot, both
+               slots of the pass in order (they may share a line) */
             if (with_lam) {
                 double v = Lval;
 #pragma unroll
                 for (int off = 16; off >= 1; off >>= 1) v += __shfl_xor(v, off, MGX_WAVE);
                 const double v_hi = __shfl(v, 32, MGX_WAVE);
-                if (lane == 0) {
-                    for (uint32_t h = 0; h < 2; h++) {
-                        const uint32_t slot_h = slot0 + h;
-                        if (slot_h >= kp.nslots) break;
-                        const uint32_t ll = slot_h / kp.slots_per_line;
-                        s_L[ll] = s_L[ll] + (h ? v_hi : v);
+                for (uint32_t h = 0; h < 2; h++) {
+                    const uint32_t slot_h = slot0 + h;
+                    if (slot_h >= kp.nslots) break;
+                    const uint32_t ll = slot_h / kp.slots_per_line;
+                    const double vh = h ? v_hi : v;
+                    if (ll != lam_line) {
+                        if (lane == 0) s_L[lam_line] = s_L[lam_line] + lam_sum;
+                        lam_line = ll;
+                        lam_sum = vh;
+                    } else {
+                        lam_sum = lam_sum + vh;
                     }
                 }
                 /* band elements: the same sums, then lane 0 merges them into the lists of
@@ -1694,6 +1704,8 @@ __device__ __forceinline__ int solve_origin(const KParams &kp, uint32_t o, uint3
             }
             __syncthreads();
         }
+        if (with_lam && lane == 0) s_L[lam_line] = s_L[lam_line] + lam_sum;
+        __syncthreads();
     }
     return 0;
 }
@@ -1710,9 +1722,11 @@ __device__ inline double line_integral(const mgx_model &m, const double *Jo, uin
     return acc;
 }
 
-/* One origin and one group of per ray pairs per wave: block (o, g) takes ray pairs
-   g per .. g per + per - 1.  With several groups J and lam are their parts, (groups, P, F)
-   and (groups, P, L), which sum_parts_kernel adds up.  With Jline set (the sparse solve, one
+/* Block (o, g) takes ray pairs g per .. g per + per - 1 of origin o.  With one group the
+   wave adds J and the Lambda diagonal up itself.  With several, every ray pair's
+   contributions are kept apart -- the Lambda part (hnrays, P, L) in lam, J's (hnrays, P, F)
+   in J, or nowhere when u is stored, whose values they are a multiple of -- and
+   sum_parts_kernel adds them up in the same order.  With Jline set (the sparse solve, one
    group) the origin's J stays in LDS (or in its row of J, a scratch) and only its line
    integrals are written. */
 template <int APPROX, int PREC>
@@ -1734,37 +1748,52 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void feautrier_
         ERR_CAP)
         return;
     double *s_L = reinterpret_cast<double *>(smem + acc_lds_offset(kp.cap, kp.stage));
-    double *s_J = kp.j_lds ? s_L + L : nullptr;
-    for (uint32_t i = lane; i < L + (s_J ? F : 0); i += MGX_WAVE) s_L[i] = 0.0;
+    const bool split = gridDim.y > 1;
+    double *s_J = kp.j_lds && !split ? s_L + L : nullptr;
     const uint32_t rr0 = blockIdx.y * per, rr1 = rr0 + per < m.hnrays ? rr0 + per : m.hnrays;
-    const size_t row = (size_t)blockIdx.y * m.npoints + o;
-    if (solve_origin<APPROX, PREC>(kp, o, rr0, rr1, smem, s_erf, u, lam != nullptr, s_J,
-                                   s_J ? nullptr : J + row * F, false, s_L))
-        return;
-    if (Jline) {
+    const uint32_t step = split ? 1 : rr1 - rr0;
+#pragma unroll 1
+    for (uint32_t rr = rr0; rr < rr1; rr += step) {
+        const size_t row = split ? (size_t)rr * m.npoints + o : o;
+        for (uint32_t i = lane; i < L + (s_J ? F : 0); i += MGX_WAVE) s_L[i] = 0.0;
+        if (solve_origin<APPROX, PREC>(kp, o, rr, rr + step, smem, s_erf, u, lam != nullptr, s_J,
+                                       s_J || !J ? nullptr : J + row * F, false, s_L))
+            return;
+        if (Jline) {
+            const double *Jo = s_J ? s_J : J + row * F;
+            for (uint32_t l = lane; l < L; l += MGX_WAVE) Jline[(size_t)o * L + l] = line_integral(m, Jo, l);
+        } else if (s_J) {
+            for (uint32_t i = lane; i < F; i += MGX_WAVE) J[row * F + i] = s_J[i];
+        }
+        if (lam)
+            for (uint32_t i = lane; i < L; i += MGX_WAVE) lam[row * L + i] = s_L[i];
         __syncthreads();
-        const double *Jo = s_J ? s_J : J + row * F;
-        for (uint32_t l = lane; l < L; l += MGX_WAVE) Jline[(size_t)o * L + l] = line_integral(m, Jo, l);
-    } else if (s_J) {
-        for (uint32_t i = lane; i < F; i += MGX_WAVE) J[row * F + i] = s_J[i];
     }
-    if (lam)
-        for (uint32_t i = lane; i < L; i += MGX_WAVE) lam[row * L + i] = s_L[i];
 }
 
-/* Adds up the groups' parts of J (n_J = P F values each) and of the Lambda diagonal (n_L,
-   0 without it), group by group, into J and lam. */
-__global__ __launch_bounds__(256) void sum_parts_kernel(const double *Jp, const double *Lp, size_t n_J,
-                                                        size_t n_L, uint32_t groups, double *J, double *lam)
+/* Adds up the ray pairs' contributions, in their order, to J (P F values; Jp their parts
+   (hnrays, P, F), or NULL: 2 w u) and to the Lambda diagonal (P L, lam may be NULL). */
+__global__ __launch_bounds__(256) void sum_parts_kernel(const KParams *__restrict__ kpp, const double *u,
+                                                        const double *Jp, const double *Lp, double *J,
+                                                        double *lam)
 {
+    const mgx_model &m = kpp->m;
+    const size_t n_J = (size_t)m.npoints * m.nfreqs, n_L = lam ? (size_t)m.npoints * m.nlines : 0;
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n_J + n_L) return;
-    const bool isJ = i < n_J;
-    const size_t n = isJ ? n_J : n_L, k = isJ ? i : i - n_J;
-    const double *p = isJ ? Jp : Lp;
-    double v = p[k];
-    for (uint32_t g = 1; g < groups; g++) v += p[g * n + k];
-    (isJ ? J : lam)[k] = v;
+    double v = 0.0;
+    if (i < n_J && !Jp) {
+        const uint32_t o = (uint32_t)(i / m.nfreqs);
+        for (uint32_t rr = 0; rr < m.hnrays; rr++) v = v + u[rr * n_J + i] * 2.0 * ray_weight(m, o, rr);
+        J[i] = v;
+    } else if (i < n_J) {
+        for (uint32_t rr = 0; rr < m.hnrays; rr++) v = v + Jp[rr * n_J + i];
+        J[i] = v;
+    } else {
+        const size_t k = i - n_J;
+        for (uint32_t rr = 0; rr < m.hnrays; rr++) v = v + Lp[rr * n_L + k];
+        lam[k] = v;
+    }
 }
 
 /* the sparse solve's line integrals from J (P, F) */
@@ -1832,18 +1861,24 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void shortchar_
         ERR_CAP)
         return;
     double *s_L = reinterpret_cast<double *>(smem + acc_lds_offset(kp.cap, kp.stage));
-    double *s_J = kp.j_lds ? s_L + L : nullptr;
-    for (uint32_t i = lane; i < L + (s_J ? F : 0); i += MGX_WAVE) s_L[i] = 0.0;
+    const bool split = gridDim.y > 1;
+    double *s_J = kp.j_lds && !split ? s_L + L : nullptr;
     const uint32_t rr0 = blockIdx.y * per, rr1 = rr0 + per < m.hnrays ? rr0 + per : m.hnrays;
-    const size_t row = (size_t)blockIdx.y * m.npoints + o;
-    if (solve_origin<APPROX, PREC, METHOD_SHORTCHAR>(kp, o, rr0, rr1, smem, s_erf, u,
-                                                     lam != nullptr, s_J, J + row * F,
-                                                     false, s_L, sc))
-        return;
-    if (s_J)
-        for (uint32_t i = lane; i < F; i += MGX_WAVE) J[row * F + i] = s_J[i];
-    if (lam)
-        for (uint32_t i = lane; i < L; i += MGX_WAVE) lam[row * L + i] = s_L[i];
+    const uint32_t step = split ? 1 : rr1 - rr0;
+#pragma unroll 1
+    for (uint32_t rr = rr0; rr < rr1; rr += step) {
+        const size_t row = split ? (size_t)rr * m.npoints + o : o;
+        for (uint32_t i = lane; i < L + (s_J ? F : 0); i += MGX_WAVE) s_L[i] = 0.0;
+        if (solve_origin<APPROX, PREC, METHOD_SHORTCHAR>(kp, o, rr, rr + step, smem, s_erf, u, lam != nullptr,
+                                                         s_J, s_J || !J ? nullptr : J + row * F, false, s_L,
+                                                         sc))
+            return;
+        if (s_J)
+            for (uint32_t i = lane; i < F; i += MGX_WAVE) J[row * F + i] = s_J[i];
+        if (lam)
+            for (uint32_t i = lane; i < L; i += MGX_WAVE) lam[row * L + i] = s_L[i];
+        __syncthreads();
+    }
 }
 
 /* Feautrier order 2 with v (Solver::solve_feautrier_order_2_uv, solver.tpp:238-295,
@@ -5116,19 +5151,18 @@ namespace {
  * How a solve splits the ray pairs of an origin over waves.  One wave per origin
  * leaves the GPU idle when there are few origins (3072 waves are resident at once) and
  * ends with a long tail when there are not many more; kSplitWaves waves fill it about
- * five times over.  Splitting costs a pass over the parts of J and Lambda, and memory for
- * them, so the groups are as few as reach that count, and their parts have to fit the
- * no-allocation solve's scratch beside its tables (both entry points then add up in the
- * same order and give the same bits).  Measured: 250 shells, 100 ray pairs
- * 39.8 -> 9.2 ms; 20^3 wind (3 groups), short
- * characteristics, 3.12 -> 2.92 ms; from
- * 16384 origins on nothing is split.
+ * five times over.  Splitting costs the ray pairs' contributions of J (unless u is
+ * stored) and Lambda a trip through memory of their own, at most kSplitBytes; the sums
+ * are the same to the last bit.  Measured: 250 shells, 100 ray pairs 39.8 -> 9.2 ms;
+ * 10^3 wind, 6 pairs, three solves 2.2 -> 0.9 ms; from 16384 origins on nothing is split.
  */
 constexpr uint32_t kSplitWaves = 16384;
+constexpr size_t kSplitBytes = (size_t)256 << 20;
 
 struct RaySplit {
     uint32_t per, groups; /* ray pairs per group, groups */
-    size_t bytes;         /* parts of J and Lambda (0: none) */
+    size_t J_bytes;       /* the ray pairs' parts of J (0: from u) and of Lambda */
+    size_t bytes;         /* all parts (0: not split) */
 };
 
 size_t noalloc_scratch_bytes(const mgx_model *model)
@@ -5139,30 +5173,36 @@ size_t noalloc_scratch_bytes(const mgx_model *model)
            rnd(P * sizeof(PointIdx)) + rnd(PL * sizeof(double4));
 }
 
-RaySplit ray_split(const mgx_model &m)
+RaySplit ray_split(const mgx_model &m, bool with_J, bool with_u, bool with_lam, size_t room)
 {
-    RaySplit r{m.hnrays, 1, 0};
+    RaySplit r{m.hnrays, 1, 0, 0};
     const uint64_t P = m.npoints;
-    uint64_t g = (kSplitWaves + P - 1) / P;
-    if (g > m.hnrays) g = m.hnrays;
-    const size_t part = (size_t)P * ((size_t)m.nfreqs + m.nlines) * sizeof(double);
-    const size_t used = noalloc_scratch_bytes(&m) + 256;
-    const size_t room = used < (size_t)MGX_NOALLOC_SCRATCH_BYTES ? (size_t)MGX_NOALLOC_SCRATCH_BYTES - used : 0;
-    if (g > room / part) g = room / part;
-    if (g < 2) return r;
-    r.per = (uint32_t)((m.hnrays + g - 1) / g);
+    const uint64_t g = (kSplitWaves + P - 1) / P;
+    if (g < 2 || m.hnrays < 2) return r;
+    const size_t PR = (size_t)P * m.hnrays * sizeof(double);
+    const size_t J_bytes = with_J && !with_u ? PR * m.nfreqs : 0;
+    const size_t bytes = J_bytes + (with_lam ? PR * m.nlines : 0);
+    if (bytes > room) return r;
+    r.per = g >= m.hnrays ? 1 : (uint32_t)((m.hnrays + g - 1) / g);
     r.groups = (m.hnrays + r.per - 1) / r.per;
-    if (r.groups > 1) r.bytes = r.groups * part;
+    if (r.groups > 1) {
+        r.J_bytes = J_bytes;
+        r.bytes = bytes;
+    }
     return r;
 }
 
-/* adds the groups' parts at b.parts up into J and lam */
-void sum_parts(const mgx_model &m, const RaySplit &sp, const DevBuffers &b, double *J, double *lam,
-               hipStream_t st)
+double *J_parts(const RaySplit &sp, const DevBuffers &b) { return sp.J_bytes ? b.parts : nullptr; }
+
+double *lam_parts(const RaySplit &sp, const DevBuffers &b) { return b.parts + sp.J_bytes / sizeof(double); }
+
+/* adds the ray pairs' contributions up into J and lam */
+void sum_parts(const mgx_model &m, const RaySplit &sp, const DevBuffers &b, const double *u, double *J,
+               double *lam, hipStream_t st)
 {
-    const size_t nJ = (size_t)m.npoints * m.nfreqs, nL = lam ? (size_t)m.npoints * m.nlines : 0;
-    hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((nJ + nL + 255) / 256)), dim3(256), 0, st, b.parts,
-                       b.parts + sp.groups * nJ, nJ, nL, sp.groups, J, lam);
+    const size_t n = (size_t)m.npoints * ((size_t)m.nfreqs + (lam ? m.nlines : 0));
+    hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, b.kp_dev, u,
+                       J_parts(sp, b), lam_parts(sp, b), J, lam);
 }
 
 /* the plain-method solve on prepared buffers (shared by the allocating and the
@@ -5176,8 +5216,8 @@ int forward_launch(const mgx_model *model, const mgx_options *opts, double *u, d
         /* the line-integrated solve keeps J in LDS, or else in a scratch J (P, F) */
         double *J = J_out, *lambda_diag = lambda_out, *Jline = Jline_out;
         if (sp.groups > 1) {
-            J = b.parts;
-            lambda_diag = lambda_out ? b.parts + (size_t)sp.groups * model->npoints * model->nfreqs : nullptr;
+            J = J_parts(sp, b);
+            lambda_diag = lambda_out ? lam_parts(sp, b) : nullptr;
             Jline = nullptr; /* from the sum of the parts */
         }
         if (Jline && !kp.j_lds) {
@@ -5219,8 +5259,8 @@ int forward_launch(const mgx_model *model, const mgx_options *opts, double *u, d
                                        grid, block, lds, st, b.kp_dev, u, J, lambda_diag, Jline, sp.per);
             }
             if (sp.groups > 1) {
-                /* the sparse solve's J goes into the first group's part */
-                sum_parts(*model, sp, b, Jline_out ? b.parts : J_out, lambda_out, st);
+                /* the sparse solve's J goes into the first ray pair's part */
+                sum_parts(*model, sp, b, u, Jline_out ? b.parts : J_out, lambda_out, st);
                 if (Jline_out)
                     hipLaunchKernelGGL(line_integral_kernel,
                                        dim3((unsigned)(((size_t)model->npoints * model->nlines + 255) / 256)),
@@ -5244,7 +5284,7 @@ int mgx_feautrier_forward_device(const mgx_model *model, const mgx_options *opts
     hipStream_t st = (hipStream_t)stream;
     DevBuffers b;
     KParams kp;
-    const RaySplit sp = ray_split(*model);
+    const RaySplit sp = ray_split(*model, true, u != nullptr, lambda_diag != nullptr, kSplitBytes);
     if (int e = prepare(model, opts, st, b, kp, false, sp.bytes)) return e;
     return forward_launch(model, opts, u, J, lambda_diag, st, b, kp, sp);
 }
@@ -5274,7 +5314,7 @@ int mgx_feautrier_sparse_device(const mgx_model *model, const mgx_options *opts,
     }
     DevBuffers b;
     KParams kp;
-    const RaySplit sp = ray_split(*model);
+    const RaySplit sp = ray_split(*model, true, false, lambda_diag != nullptr, kSplitBytes);
     if (int e = prepare(model, opts, st, b, kp, false, sp.bytes)) return e;
     /* J of an origin stays in LDS; when it does not fit (long walks), its row of a
        scratch J, allocated by the launch that needs it */
@@ -5316,7 +5356,8 @@ int mgx_feautrier_forward_noalloc(const mgx_model *model, const mgx_options *opt
     b.pts = reinterpret_cast<PointRec *>(take(P * sizeof(PointRec)));
     b.pidx = reinterpret_cast<PointIdx *>(take(P * sizeof(PointIdx)));
     b.lpack = reinterpret_cast<double4 *>(take(PL * sizeof(double4)));
-    const RaySplit sp = ray_split(*model);
+    const RaySplit sp = ray_split(*model, true, u != nullptr, lambda_diag != nullptr,
+                                  (size_t)MGX_NOALLOC_SCRATCH_BYTES - off);
     b.parts = reinterpret_cast<double *>(take(sp.bytes));
     struct NoEvents {
         NoEvents() { t_no_events = true; }
@@ -5391,14 +5432,13 @@ int mgx_shortchar_order_0_device(const mgx_model *model, const mgx_options *opts
     hipStream_t st = (hipStream_t)stream;
     DevBuffers b;
     KParams kp;
-    const RaySplit sp = ray_split(*model);
+    const RaySplit sp = ray_split(*model, true, u != nullptr, lambda_diag != nullptr, kSplitBytes);
     if (int e = prepare(model, opts, st, b, kp, false, sp.bytes)) return e;
     const ShortcharOut sc{I, v, min_dtau};
     return launch_with_capacity(st, b, kp, [&](size_t) {
         const dim3 grid(model->npoints, sp.groups), block(MGX_WAVE);
-        double *Jp = sp.groups > 1 ? b.parts : J;
-        double *Lp = sp.groups > 1 && lambda_diag ? b.parts + (size_t)sp.groups * model->npoints * model->nfreqs
-                                                  : lambda_diag;
+        double *Jp = sp.groups > 1 ? J_parts(sp, b) : J;
+        double *Lp = sp.groups > 1 && lambda_diag ? lam_parts(sp, b) : lambda_diag;
         const size_t lds = solve_lds_bytes(kp.cap, kp.stage, model->nfreqs, model->nlines, kp.j_lds != 0);
         timed(st, [&] {
             const bool fp64 = opts->precision == MGX_PREC_FP64;
@@ -5427,7 +5467,7 @@ int mgx_shortchar_order_0_device(const mgx_model *model, const mgx_options *opts
                     hipLaunchKernelGGL((shortchar_kernel<MGX_APPROX_CLOSE_LINES, MGX_PREC_MIXED>),
                                        grid, block, lds, st, b.kp_dev, sc, u, Jp, Lp, sp.per);
             }
-            if (sp.groups > 1) sum_parts(*model, sp, b, J, lambda_diag, st);
+            if (sp.groups > 1) sum_parts(*model, sp, b, u, J, lambda_diag, st);
         });
     }, 8 * (size_t)model->nlines, true);
 }
@@ -5442,7 +5482,7 @@ int mgx_feautrier_order_2_uv_device(const mgx_model *model, const mgx_options *o
     DevBuffers b;
     KParams kp;
     if (int e = prepare(model, opts, st, b, kp)) return e;
-    const RaySplit sp = ray_split(*model); /* no parts: u and v are per ray pair */
+    const RaySplit sp = ray_split(*model, false, true, false, 0); /* u and v are per ray pair */
     return launch_with_capacity(st, b, kp, [&](size_t) {
         const dim3 grid(model->npoints, sp.groups), block(MGX_WAVE);
         const size_t lds = solve_lds_bytes(kp.cap, kp.stage, model->nfreqs, model->nlines, false);
