@@ -53,9 +53,15 @@
 #ifndef MGX_SOLVE_WAVES_PER_SIMD
 #define MGX_SOLVE_WAVES_PER_SIMD 3
 #endif
-/* the same for the adjoint kernels */
-#ifndef MGX_ADJ_WAVES_PER_SIMD
-#define MGX_ADJ_WAVES_PER_SIMD 2
+/* the same for the adjoint kernels: three waves hide more of the tape's and the walk's
+   latency in the J adjoint than their spills cost (24^3 wind, FP64, with its forward: 21.0 ms
+   at two, 20.1 at three); the image adjoint has fewer waves to fill and the wider state of the
+   inverse widths (128^2 clumpy image gradient 2.79 ms at two, 3.15 at three) */
+#ifndef MGX_J_ADJOINT_WAVES_PER_SIMD
+#define MGX_J_ADJOINT_WAVES_PER_SIMD 3
+#endif
+#ifndef MGX_IMAGE_ADJOINT_WAVES_PER_SIMD
+#define MGX_IMAGE_ADJOINT_WAVES_PER_SIMD 2
 #endif
 
 namespace {
@@ -434,6 +440,46 @@ __device__ __forceinline__ void next_dpp(NextPoint &a)
     next_take(a, NextPoint{dpp_get<CTRL>(a.d2), dpp_get<CTRL>(a.zn), dpp_get<CTRL>(a.idx), dpp_get<CTRL>(a.n)});
 }
 
+/* the arg-min of a half-wave, in its lanes */
+__device__ __forceinline__ void next_min(NextPoint &best)
+{
+    next_dpp<0xb1>(best);
+    next_dpp<0x4e>(best);
+    next_dpp<0x141>(best);
+    next_dpp<0x140>(best);
+    NextPoint odd;
+    half_rows(best.d2, best.d2, odd.d2);
+    half_rows(best.zn, best.zn, odd.zn);
+    half_rows(best.idx, best.idx, odd.idx);
+    half_rows(best.n, best.n, odd.n);
+    next_take(best, odd);
+}
+
+/* get_next_general_geometry<Defaulttracer> (geometry.tpp:14-44) by a half-wave */
+__device__ inline uint32_t next_half(const KParams &kp, const double *origin, const double *dir,
+                                     const PointIdx &pc, double &Z, double &dZ)
+{
+    NextPoint best = {__builtin_inf(), 0.0, 0xffffffffu, kp.m.npoints};
+    for (uint32_t i = threadIdx.x & 31; i < pc.n_nbs; i += 32) {
+        const uint32_t n = gld(&kp.m.neighbors[pc.cum + i]);
+        const PointPos pn = gld(reinterpret_cast<const PointPos *>(&kp.pts[n]));
+        double R[3];
+        R[0] = pn.x - origin[0];
+        R[1] = pn.y - origin[1];
+        R[2] = pn.z - origin[2];
+        const double Z_new = dot3(R, dir);
+        if (Z_new > Z) {
+            const double d2 = dot3(R, R) - Z_new * Z_new;
+            if (d2 < DBL_MAX && d2 < best.d2) best = NextPoint{d2, Z_new, i, n};
+        }
+    }
+    next_min(best);
+    if (best.idx == 0xffffffffu) return kp.m.npoints;
+    dZ = best.zn - Z;
+    Z += dZ;
+    return best.n;
+}
+
 /*
  * Both half rays of a ray pair at once: lanes 0-31 walk from o along ray rr into the first
  * list, lanes 32-63 along its antipod ar into the second (walk_half's steps, lists and
@@ -469,36 +515,7 @@ __device__ int walk_pair(const KParams &kp, uint32_t o, uint32_t rr, uint32_t ar
         if (m.spherical_symmetry) {
             nxt = next_spherical(kp, origin, dir, crt, Z, dZ);
         } else {
-            /* get_next_general_geometry<Defaulttracer> (geometry.tpp:14-44) */
-            NextPoint best = {__builtin_inf(), 0.0, 0xffffffffu, m.npoints};
-            for (uint32_t i = q; i < pc.n_nbs; i += 32) {
-                const uint32_t n = gld(&m.neighbors[pc.cum + i]);
-                const PointPos pn = gld(reinterpret_cast<const PointPos *>(&kp.pts[n]));
-                double R[3];
-                R[0] = pn.x - origin[0];
-                R[1] = pn.y - origin[1];
-                R[2] = pn.z - origin[2];
-                const double Z_new = dot3(R, dir);
-                if (Z_new > Z) {
-                    const double d2 = dot3(R, R) - Z_new * Z_new;
-                    if (d2 < DBL_MAX && d2 < best.d2) best = NextPoint{d2, Z_new, i, n};
-                }
-            }
-            next_dpp<0xb1>(best);
-            next_dpp<0x4e>(best);
-            next_dpp<0x141>(best);
-            next_dpp<0x140>(best);
-            NextPoint odd;
-            half_rows(best.d2, best.d2, odd.d2);
-            half_rows(best.zn, best.zn, odd.zn);
-            half_rows(best.idx, best.idx, odd.idx);
-            half_rows(best.n, best.n, odd.n);
-            next_take(best, odd);
-            nxt = best.n;
-            if (best.idx != 0xffffffffu) {
-                dZ = best.zn - Z;
-                Z += dZ;
-            }
+            nxt = next_half(kp, origin, dir, pc, Z, dZ);
         }
         if (nxt >= m.npoints) {
             if (S != 0) err = ERR_NO_NEXT; /* else nothing in this direction */
@@ -543,8 +560,8 @@ __device__ inline uint32_t n_interp_all(const KParams &kp, uint32_t c, uint32_t 
     const uint32_t L = kp.m.nlines;
     double mx = 0.0;
     for (uint32_t l = 0; l < L; l++) {
-        const double d = (double)fabsf(mgx_ref_logf((float)(kp.m.interp_crit[(size_t)n * L + l] /
-                                                        kp.m.interp_crit[(size_t)c * L + l])));
+        const double d = (double)fabsf(mgx_ref_logf((float)(gld(&kp.m.interp_crit[(size_t)n * L + l]) /
+                                                    gld(&kp.m.interp_crit[(size_t)c * L + l]))));
         if (l == 0 || mx < d) mx = d;
     }
     const uint32_t k = (uint32_t)ceil(mx / kp.log_max_interp);
@@ -680,19 +697,7 @@ struct OwnLine {
     uint32_t g;
     uint32_t lidx;   /* sorted_line_map[g]: the line at position g */
     double a_lo, a_g, a_hi;
-    double f_own;    /* line[lidx] */
 };
-
-/* Whether the line-integrated segments take the own line's frequency from OwnLine
-   (a register) or read line[lidx] (a load that needs no other load first).  The
-   adjoint unit, at 256 VGPRs, keeps it in a register; the solve unit, at 168,
-   reads it: measured on the 32^3 wind, the register cost the forward 4-6% in
-   spills, the load cost the adjoint 8%. */
-#ifdef MGX_ADJOINT_TU
-#define MGX_OWN_FREQ_IN_REGS 1
-#else
-#define MGX_OWN_FREQ_IN_REGS 0
-#endif
 
 __device__ inline OwnLine own_line(const mgx_model &m, uint32_t l)
 {
@@ -704,7 +709,6 @@ __device__ inline OwnLine own_line(const mgx_model &m, uint32_t l)
             if (gld(&m.sorted_line_map[s]) == l) g = s;
     r.g = g;
     r.lidx = gld(&m.sorted_line_map[g]);
-    r.f_own = gld(&m.line[r.lidx]);
     r.a_g = gld(&m.sorted_line[g]);
     r.a_lo = (g > 0) ? gld(&m.sorted_line[g - 1]) : -__builtin_inf();
     r.a_hi = (g + 1 < m.nlines) ? gld(&m.sorted_line[g + 1]) : __builtin_inf();
@@ -832,17 +836,16 @@ __device__ void S_dtau_line_integrated(const KParams &kp, const double *erf_tab,
         line_window(m, ol, left_freq - W, right_freq + W, lo, hi);
     }
     for (uint32_t s = lo; s < hi; s++) {
-        /* the own line's index and frequency come from OwnLine, so the usual
-           one-line window waits on no table load before its gathers */
+        /* the own line's index comes from OwnLine, so the usual one-line window waits
+           on no table load before its gathers */
         uint32_t l = s;
         double linefreq;
         if (APPROX == MGX_APPROX_CLOSE_LINES && s == ol.g) {
             l = ol.lidx;
-            linefreq = MGX_OWN_FREQ_IN_REGS ? ol.f_own : gld(&m.line[l]);
-        } else {
-            if (APPROX == MGX_APPROX_CLOSE_LINES) l = gld(&m.sorted_line_map[s]);
-            linefreq = gld(&m.line[l]);
+        } else if (APPROX == MGX_APPROX_CLOSE_LINES) {
+            l = gld(&m.sorted_line_map[s]);
         }
+        linefreq = gld(&m.line[l]);
         const double4 c = lp(kp, cp, l), cI = lp(kp, cpi, l);
         const double4 n = lp(kp, np, l), nI = lp(kp, npi, l);
         const double line_dtau = dtau_single_line<PREC>(kp, erf_tab, c, cI, n, nI, linefreq,
@@ -1040,6 +1043,14 @@ __host__ __device__ inline size_t acc_lds_offset(uint32_t cap, uint32_t stage)
     return lines_lds_offset(cap, stage) + 2 * (size_t)window_lines(stage) * sizeof(WindowLine);
 }
 
+#include "mgx_staged_adjoint.h"
+
+/* dynamic LDS of the adjoint kernels: as the solve's, and the staged entries' sums */
+__host__ __device__ inline size_t adjoint_lds_bytes(uint32_t cap, uint32_t stage)
+{
+    return acc_lds_offset(cap, stage) + 2 * (size_t)stage * sizeof(EntryGrad);
+}
+
 /* dynamic LDS of the solve kernel: walk buffers, staged entries (stage of each of two
    groups) and their half rays, the Lambda (L) accumulator and, when j_lds, the J (F) accumulator */
 __host__ __device__ inline size_t solve_lds_bytes(uint32_t cap, uint32_t stage, uint32_t F, uint32_t L,
@@ -1051,10 +1062,11 @@ __host__ __device__ inline size_t solve_lds_bytes(uint32_t cap, uint32_t stage, 
 /* LDS kept beside the walk buffers when the longest walk that fits is worked out: the
    static LDS of a kernel (the float functions' tables, MGX_REF_LDS_TABLE_BYTES, and a
    few words) and the smallest chunk of staged entries */
-constexpr uint32_t kStageMin = 4;
+constexpr uint32_t kStageMin = 3;
 constexpr size_t kStaticLds = MGX_REF_LDS_TABLE_BYTES + 64;
 constexpr size_t kReservedLds = 2048;
-static_assert(kStaticLds + 2 * (kStageMin * sizeof(StagedEntry) + sizeof(GroupRay) + sizeof(WindowLine)) + 16 <= kReservedLds, "reserved LDS");
+static_assert(kStaticLds + 2 * (kStageMin * (sizeof(StagedEntry) + sizeof(EntryGrad)) + sizeof(GroupRay) + sizeof(WindowLine)) +
+                      16 <= kReservedLds, "reserved LDS");
 
 /* J stays in LDS while the whole LDS of a workgroup fits the share of a CU's
    160 KiB that the register-limited occupancy (MGX_SOLVE_WAVES_PER_SIMD waves on
@@ -1086,8 +1098,8 @@ __device__ inline void j_add(double *Jrow, uint32_t f, double c, bool first, boo
         Jrow[f] = first ? c : Jrow[f] + c;
 }
 
-/* which formal solution solve_origin runs */
-enum { METHOD_FEAUTRIER = 0, METHOD_SHORTCHAR = 1, METHOD_UV = 2 };
+/* what a sweep computes (METHOD_TAU: the optical depth along the half ray, in Y) */
+enum { METHOD_FEAUTRIER = 0, METHOD_SHORTCHAR = 1, METHOD_UV = 2, METHOD_TAU = 3 };
 
 /*
  * One half ray of the two-sided elimination.  Walking from the boundary end
@@ -1153,10 +1165,11 @@ __device__ inline void ring_push(BandRing<NB> &r, double h, double g, uint32_t n
  * with dt = max(min_dtau, dtau) and the reference's float expf / expm1f; sw.Y carries
  * I and sw.prev_dtau the last dt.
  */
-template <int APPROX, int PREC, int METHOD, int NB>
+template <int APPROX, int PREC, int METHOD, int NB, bool TAPE = false>
 __device__ __forceinline__ void staged_sweep(const KParams &kp, unsigned char *smem, const GroupRay *g,
                                              bool backward, double freq, bool active, StagedEntry *chunk,
-                                             double min_dtau, Sweep &sw, BandRing<NB> &ring)
+                                             double min_dtau, Sweep &sw, BandRing<NB> &ring,
+                                             const Tape *tape = nullptr, double *I_outer = nullptr)
 {
     const uint32_t count = kp.stage;
     const uint32_t n = active ? g->n : 0;
@@ -1180,17 +1193,24 @@ __device__ __forceinline__ void staged_sweep(const KParams &kp, unsigned char *s
             out.kap = chunk->kap;
             out.src = chunk->src;
             out.f = freq * s;
-            I_b = boundary_intensity(kp, chunk->nr, out.f);
+            if constexpr (METHOD != METHOD_TAU) I_b = boundary_intensity(kp, chunk->nr, out.f);
+            if constexpr (TAPE) *I_outer = I_b;
         }
         const uint32_t left = nmax - k0, jmax = left < count - 1 ? left : count - 1;
         for (uint32_t j = 1; j <= jmax; j++) {
             const StagedEntry *eo = chunk + j - 1, *ei = chunk + j;
             PointEC ec_in = {0.0, 0.0, false};
-            double dtau, S_out, S_in;
+            double dtau, S_out, S_in, dop;
             const bool on = k0 + j <= n;
             staged_segment<APPROX, PREC>(kp, g, lines, window_lines(count), bin, eo, ei, on, out, ec_out, ec_in, dtau,
-                                         S_out, S_in);
+                                         S_out, S_in, dop);
             if (!on) continue;
+            if constexpr (METHOD == METHOD_TAU) {
+                sw.Y += dtau;
+                sw.started = true;
+                ec_out = ec_in;
+                continue;
+            }
             if constexpr (METHOD == METHOD_SHORTCHAR) {
                 if (!sw.started) sw.Y = I_b;
                 sw.started = true;
@@ -1237,6 +1257,15 @@ __device__ __forceinline__ void staged_sweep(const KParams &kp, unsigned char *s
             sw.prev_dtau = dtau;
             sw.S_prev_row = S_in;
             ec_out = ec_in;
+            if constexpr (TAPE) {
+                const uint32_t k = k0 + j - 1;
+                *tape->at(k, 0) = sw.Y;
+                *tape->at(k, 1) = sw.X;
+                if ((ei->kind & SEG_MASK) != SEG_EMPTY) {
+                    *tape->at(k, 2) = dtau;
+                    *tape->at(k, 3) = dop;
+                }
+            }
         }
     }
     sw.S_inner = sw.S_prev_row;
@@ -2338,47 +2367,44 @@ __global__ __launch_bounds__(256) void image_frame_kernel(mgx_model m, ImageFram
     }
 }
 
-/* get_boundary_point_closer_to_custom_ray (geometry.tpp:310-341), wave-cooperative */
+/* get_boundary_point_closer_to_custom_ray (geometry.tpp:310-341) by the lanes of a
+   half-wave, each with its own ray */
 __device__ inline uint32_t bdy_closer(const mgx_model &m, const double *origin, const double *rd,
                                       uint32_t crt)
 {
-    const uint32_t lane = threadIdx.x & (MGX_WAVE - 1);
-    const uint32_t n_nbs = m.n_neighbors[crt];
-    const uint32_t cum = m.cum_n_neighbors[crt];
+    const uint32_t q = threadIdx.x & 31;
+    const uint32_t n_nbs = gld(&m.n_neighbors[crt]);
+    const uint32_t cum = gld(&m.cum_n_neighbors[crt]);
     double Rc[3];
-    for (int i = 0; i < 3; i++) Rc[i] = m.position[3 * (size_t)crt + i] - origin[i];
+    for (int i = 0; i < 3; i++) Rc[i] = gld(&m.position[3 * (size_t)crt + i]) - origin[i];
     const double Zc = dot3(Rc, rd);
     /* the current point is the candidate to beat (key 0); neighbour i has key i + 1 */
-    double best = (lane == 0) ? dot3(Rc, Rc) - Zc * Zc : __builtin_inf();
-    uint32_t key = (lane == 0) ? 0u : 0xffffffffu;
-    double dummy = 0.0;
-    for (uint32_t i = lane; i < n_nbs; i += MGX_WAVE) {
-        const uint32_t n = m.neighbors[cum + i];
-        if (m.point2boundary[n] != m.npoints) {
+    NextPoint best = {dot3(Rc, Rc) - Zc * Zc, 0.0, 0u, crt};
+    if (q != 0) best = NextPoint{__builtin_inf(), 0.0, 0xffffffffu, crt};
+    for (uint32_t i = q; i < n_nbs; i += 32) {
+        const uint32_t n = gld(&m.neighbors[cum + i]);
+        if (gld(&m.point2boundary[n]) != m.npoints) {
             double R[3];
-            for (int j = 0; j < 3; j++) R[j] = m.position[3 * (size_t)n + j] - origin[j];
+            for (int j = 0; j < 3; j++) R[j] = gld(&m.position[3 * (size_t)n + j]) - origin[j];
             const double Zn = dot3(R, rd);
-            const double d2 = dot3(R, R) - Zn * Zn;
-            if (lex_less(d2, i + 1, best, key)) {
-                best = d2;
-                key = i + 1;
-            }
+            next_take(best, NextPoint{dot3(R, R) - Zn * Zn, 0.0, i + 1, n});
         }
     }
-    wave_argmin(best, key, dummy, n_nbs);
-    return (key == 0 || key == 0xffffffffu) ? crt : m.neighbors[cum + key - 1];
+    next_min(best);
+    return best.n;
 }
 
-__device__ inline double shift_rest(const mgx_model &m, const double *origin, const double *rd,
+__device__ inline double shift_rest(const KParams &kp, const double *origin, const double *rd,
                                     uint32_t c, double Z)
 {
-    if (m.spherical_symmetry) {
-        const double *pc = &m.position[3 * (size_t)c];
-        if (pc[0] == 0.0) return 1.0;
+    const PointRec pc = gld(&kp.pts[c]);
+    if (kp.m.spherical_symmetry) {
+        if (pc.x == 0.0) return 1.0;
         const double Rcos_plus_Z = dot3(origin, rd) + Z;
-        return 1.0 + m.velocity[3 * (size_t)c] * Rcos_plus_Z / pc[0];
+        return 1.0 + pc.vx * Rcos_plus_Z / pc.x;
     }
-    return 1.0 + dot3(&m.velocity[3 * (size_t)c], rd);
+    const double v[3] = {pc.vx, pc.vy, pc.vz};
+    return 1.0 + dot3(v, rd);
 }
 
 /* image kinds: the intensity (2 Su[last] - I_bdy) or the optical depth along the ray */
@@ -2428,54 +2454,34 @@ __device__ inline double fe_last(const FwdElim &fe, double S_last, double I_l)
     return fma(A_l, fe.Su, Sl) * (1.0 + fe.FF) * denominator;
 }
 
-/* The projection-surface imager, one pixel at a time (the pixel loop bodies of
+/* The projection-surface imager (the pixel loop bodies of
    Solver::image_feautrier_order_2_new_imager and image_optical_depth_new_imager,
-   solver.tpp:590-620, 701-729), in two parts: image_walk, where the whole wave
-   walks the pixel's ray into its lists in the LDS walk buffer, and image_freqs,
-   where lanes take the pixel's frequencies.  The walk buffer of capacity cap
-   (walk_lds_bytes(cap) bytes) holds two pixels' lists of up to cap steps each:
-   slot 0 and slot 1. */
+   solver.tpp:590-620, 701-729): each half-wave walks a pixel's ray into its own list and
+   its lanes take frequencies, over staged entries.  Two walks side by side and staged
+   line data took the 256^2 x 31 image of the 32^3 wind, mixed, from 3.1 to 1.8 ms. */
 struct PixelWalk {
-    uint32_t *nxt;
-    double *dZ, *sh;
-    uint16_t *m;
     uint32_t ip, S;
     double shift0, shift_centre;
 };
 
-__device__ inline PixelWalk pixel_slot(unsigned char *smem, uint32_t cap, uint32_t slot)
-{
-    PixelWalk w;
-    double *dZ = reinterpret_cast<double *>(smem + 8 * ((2 * cap * 4 + 7) / 8));
-    w.nxt = reinterpret_cast<uint32_t *>(smem) + slot * cap;
-    w.dZ = dZ + slot * cap;
-    w.sh = dZ + 2 * cap + slot * cap;
-    w.m = reinterpret_cast<uint16_t *>(dZ + 4 * cap) + slot * cap;
-    w.ip = 0;
-    w.S = 0;
-    w.shift0 = w.shift_centre = 0.0;
-    return w;
-}
-
-/* Walks pixel pix's ray into w's lists (the whole wave; lane 0 writes ImX, ImY and
-   the lists).  Returns false when the walk needs more than kp.cap steps (the status
-   words then hold ERR_CAP and the capacity needed). */
-__device__ bool image_walk(const KParams &kp, const ImageFrame &fr, uint32_t pix, PixelWalk &w,
-                           double *ImX, double *ImY)
+/* Walks pixel pix's ray into list of the half-wave (its first lane writes ImX, ImY and the
+   list).  Returns false when the walk needs more than kp.cap steps (the status words then
+   hold ERR_CAP and the capacity needed). */
+__device__ bool image_walk(const KParams &kp, const ImageFrame &fr, uint32_t pix, unsigned char *smem,
+                           PixelWalk &w, double *ImX, double *ImY)
 {
     const mgx_model &m = kp.m;
-    const uint32_t lane = threadIdx.x & (MGX_WAVE - 1);
+    const uint32_t q = threadIdx.x & 31, list = (threadIdx.x & (MGX_WAVE - 1)) >> 5;
     const uint32_t cap = kp.cap;
-    uint32_t *s_nxt = w.nxt;
-    double *s_dZ = w.dZ;
-    double *s_sh = w.sh;
-    uint16_t *s_m = w.m;
+    uint32_t *s_nxt = reinterpret_cast<uint32_t *>(smem) + list * cap;
+    double *s_dZ = reinterpret_cast<double *>(smem + 8 * ((2 * cap * 4 + 7) / 8)) + list * cap;
+    double *s_sh = s_dZ + 2 * cap;
 
     /* pixel position on the projection surface and its 3D origin */
     const uint32_t x_idx = pix / fr.ny, y_idx = pix % fr.ny;
     const double xloc = fr.min_x + fr.deltax / 2.0 + x_idx * fr.deltax;
     const double yloc = fr.min_y + fr.deltay / 2.0 + y_idx * fr.deltay;
-    if (lane == 0 && ImX) {
+    if (q == 0 && ImX) {
         ImX[pix] = xloc;
         ImY[pix] = yloc;
     }
@@ -2512,7 +2518,7 @@ __device__ bool image_walk(const KParams &kp, const ImageFrame &fr, uint32_t pix
             Z = (h2 > 0) ? (-sqrt(h2) - Rcos) : -Rcos;
         }
     }
-    const double shift_centre = shift_rest(m, origin, rd, ip, Z);
+    const double shift_centre = shift_rest(kp, origin, rd, ip, Z);
 
     /* trace_ray_imaging<Rest> (solver.tpp:842-897): walk into LDS */
     uint32_t S = 0;
@@ -2521,27 +2527,27 @@ __device__ bool image_walk(const KParams &kp, const ImageFrame &fr, uint32_t pix
         double dZ = 0.0;
         uint32_t crt = ip;
         uint32_t nxt = m.spherical_symmetry ? next_spherical(kp, origin, rd, crt, Z, dZ)
-                                            : next_general(kp, origin, rd, gld(&kp.pidx[crt]), Z, dZ);
+                                            : next_half(kp, origin, rd, gld(&kp.pidx[crt]), Z, dZ);
         bool accessed_non_boundary = false;
         if (nxt < m.npoints) {
-            shift0 = shift_rest(m, origin, rd, crt, Z - dZ);
-            double shift_nxt = shift_rest(m, origin, rd, nxt, Z);
+            shift0 = shift_rest(kp, origin, rd, crt, Z - dZ);
+            double shift_nxt = shift_rest(kp, origin, rd, nxt, Z);
             for (;;) {
                 /* past the buffer the walk goes on uncounted in LDS, so that the
                    relaunch gets the ray's exact length; a chord crosses every point
                    at most twice (each shell, under spherical symmetry) */
                 if (S > 2 * m.npoints + 2) {
-                    if (lane == 0) atomicOr(&kp.status[0], (uint32_t)ERR_NO_NEXT);
+                    if (q == 0) atomicOr(&kp.status[0], (uint32_t)ERR_NO_NEXT);
                     return false;
                 }
-                if (S < cap && lane == 0) {
+                if (S < cap && q == 0) {
                     s_nxt[S] = nxt;
                     s_dZ[S] = dZ;
                     s_sh[S] = shift_nxt;
                 }
                 S++;
-                double rel[3];
-                for (int i = 0; i < 3; i++) rel[i] = m.position[3 * (size_t)nxt + i] - m.center[i];
+                const PointPos pr = gld(reinterpret_cast<const PointPos *>(&kp.pts[nxt]));
+                const double rel[3] = {pr.x - m.center[0], pr.y - m.center[1], pr.z - m.center[2]};
                 /* the record of nxt serves the boundary test and the next step */
                 const PointIdx pn = gld(&kp.pidx[nxt]);
                 const bool interior = pn.p2b == m.npoints;
@@ -2549,28 +2555,20 @@ __device__ bool image_walk(const KParams &kp, const ImageFrame &fr, uint32_t pix
                 crt = nxt;
                 if (interior) accessed_non_boundary = true;
                 nxt = m.spherical_symmetry ? next_spherical(kp, origin, rd, crt, Z, dZ)
-                                           : next_general(kp, origin, rd, pn, Z, dZ);
+                                           : next_half(kp, origin, rd, pn, Z, dZ);
                 if (nxt >= m.npoints) break;
-                shift_nxt = shift_rest(m, origin, rd, nxt, Z);
+                shift_nxt = shift_rest(kp, origin, rd, nxt, Z);
             }
         }
         if (!accessed_non_boundary && !m.spherical_symmetry) S = 0;
     }
     if (S > cap) {
-        if (lane == 0) {
+        if (q == 0) {
             atomicOr(&kp.status[0], (uint32_t)ERR_CAP);
             atomicMax(&kp.status[1], S);
         }
         return false;
     }
-    __syncthreads();
-    for (uint32_t i = lane; i < S; i += MGX_WAVE) {
-        const uint32_t crt = (i == 0) ? ip : s_nxt[i - 1];
-        const uint32_t mm = n_interp_all(kp, crt, s_nxt[i]);
-        if (mm > 0xffffu) atomicOr(&kp.status[0], (uint32_t)ERR_INTERP);
-        s_m[i] = (uint16_t)(mm > 0xffffu ? 0xffffu : mm);
-    }
-    __syncthreads();
     w.ip = ip;
     w.S = S;
     w.shift0 = shift0;
@@ -2578,95 +2576,80 @@ __device__ bool image_walk(const KParams &kp, const ImageFrame &fr, uint32_t pix
     return true;
 }
 
-/* The frequencies f0, f0 + fstep, ... of the walked pixel pix. */
-template <int APPROX, int PREC, int KIND>
-__device__ void image_freqs(const KParams &kp, const PixelWalk &w, uint32_t pix, uint32_t f0,
-                            uint32_t fstep, double *I)
+/* The lane's bin of the walked pixel: its frequency, and the group's half ray in LDS with
+   the line nearest below the middle frequency as the own line (windows that hold other lines
+   or none say so themselves).  f is the lane's frequency index, past the last one for idle
+   lanes.  All lanes of the wave call this together. */
+__device__ inline double image_group(const KParams &kp, unsigned char *smem, const PixelWalk &w, uint32_t f,
+                                     GroupRay *g)
 {
-    const double *s_erf = nullptr; /* erf needs no table */
     const mgx_model &m = kp.m;
-    const uint32_t F = m.nfreqs;
-    const uint32_t ip = w.ip, S = w.S;
-    const double shift0 = w.shift0, shift_centre = w.shift_centre;
-    const uint32_t *s_nxt = w.nxt;
-    const double *s_dZ = w.dZ, *s_sh = w.sh;
-    const uint16_t *s_m = w.m;
-
-    for (uint32_t f = f0; f < F; f += fstep) {
-        const double nu_ip = m.nu[(size_t)ip * F + f];
-        double Ival;
-        if (S == 0) {
-            /* n_tot = 1: the boundary intensity, or no optical depth
-               (image_optical_depth_new_imager, solver.tpp:703-729) */
-            Ival = (KIND == IMG_OPTICAL_DEPTH) ? 0.0 : boundary_intensity(kp, ip, nu_ip);
-        } else {
-            const double freq = nu_ip;
-            const uint32_t line = m.f_line[f];
-            const uint32_t ub_idx = upper_bound_d(m.sorted_line, m.nlines, freq);
-            const uint32_t own_l = m.sorted_line_map[ub_idx > 0 ? ub_idx - 1 : 0];
-            const OwnLine ol = own_line(m, own_l);
-            HalfIter it;
-            it.s = (int)S - 1;
-            hi_load_step(kp, it, line, ip, shift0, s_nxt, s_dZ, s_sh, s_m);
-            Entry outer = hi_entry(it, ip);
-            PointEC ec_out = {0.0, 0.0, false};
-            FwdElim fe;
-            fe.started = false;
-            double prev_Snext = 0.0, tau = 0.0;
-            for (;;) {
-                const double dz = hi_advance(kp, it, line, ip, shift0, s_nxt, s_dZ, s_sh, s_m);
-                Entry inner = hi_entry(it, ip);
-                if (it.s < 0) inner.shift = shift_centre;
-                PointEC ec_in = {0.0, 0.0, false};
-                double dtau, S_out, S_in;
-                segment<APPROX, PREC>(kp, s_erf, ol, outer, inner, dz, freq, line, ec_out, ec_in,
-                                      dtau, S_out, S_in);
-                if constexpr (KIND == IMG_OPTICAL_DEPTH)
-                    tau += dtau; /* image_optical_depth (solver.tpp:2718-2758) */
-                else
-                    fe_row(kp, fe, dtau, S_out, outer, freq);
-                prev_Snext = S_in;
-                outer = inner;
-                ec_out = ec_in;
-                if (it.s < 0) break;
-            }
-            if constexpr (KIND == IMG_OPTICAL_DEPTH) {
-                Ival = tau;
-            } else {
-                /* last row at the start point (image_feautrier_order_2, solver.tpp:2546-2559) */
-                const double I_l = boundary_intensity(kp, ip, freq * shift_centre);
-                Ival = 2.0 * fe_last(fe, prev_Snext, I_l) - boundary_intensity(kp, ip, nu_ip);
-            }
-        }
-        I[(size_t)pix * F + f] = Ival;
+    const uint32_t F = m.nfreqs, lane = threadIdx.x & (MGX_WAVE - 1), grp = lane >> 5;
+    const double freq = gld(&m.nu[(size_t)w.ip * F + (f < F ? f : F - 1)]);
+    const double fmin = group32(freq, [](double a, double b) { return a < b ? a : b; });
+    const double fmax = group32(freq, [](double a, double b) { return a < b ? b : a; });
+    __syncthreads();
+    if ((lane & 31) == 0) {
+        const uint32_t ub = upper_bound_d(m.sorted_line, m.nlines, 0.5 * (fmin + fmax));
+        GroupRay r;
+        r.o = w.ip;
+        r.line = gld(&m.sorted_line_map[ub > 0 ? ub - 1 : 0]);
+        r.S = w.S;
+        r.list = grp;
+        r.shift0 = w.shift0;
+        r.shift_c = w.shift_centre;
+        r.fmin = fmin;
+        r.fmax = fmax;
+        r.ol = own_line(m, r.line);
+        *g = r;
     }
+    __syncthreads();
+    return freq;
 }
 
-/* One pixel per wave, or two when the image has at most 32 frequencies: then the
-   wave walks both pixels' rays and each half-wave takes one pixel's frequencies.
-   Returns false when a walk outgrew the walk buffer. */
+/* The images of npix pixels from pix0 on: two, one per half-wave, when a half-wave covers
+   the frequencies, else one, whose frequencies both half-waves share.  Returns false when a
+   walk outgrew the walk buffer. */
 template <int APPROX, int PREC, int KIND>
 __device__ bool image_pixels(const KParams &kp, const ImageFrame &fr, uint32_t pix0, uint32_t npix,
                              unsigned char *smem, double *I, double *ImX, double *ImY)
 {
-    const uint32_t lane = threadIdx.x & (MGX_WAVE - 1);
-    PixelWalk w0 = pixel_slot(smem, kp.cap, 0);
-    const bool ok0 = image_walk(kp, fr, pix0, w0, ImX, ImY);
-    if (npix == 1) {
-        if (!ok0) return false;
-        image_freqs<APPROX, PREC, KIND>(kp, w0, pix0, lane, MGX_WAVE, I);
-        return true;
+    constexpr int METHOD = KIND == IMG_OPTICAL_DEPTH ? METHOD_TAU : METHOD_FEAUTRIER;
+    const mgx_model &m = kp.m;
+    const uint32_t F = m.nfreqs, lane = threadIdx.x & (MGX_WAVE - 1), grp = lane >> 5;
+    const uint32_t pix = npix == 2 ? pix0 + grp : pix0;
+    PixelWalk w;
+    /* both rays are walked even when one outgrows the buffer, so that its length is
+       reported too */
+    const bool ok = image_walk(kp, fr, pix, smem, w, ImX, ImY);
+    if (__ballot(!ok)) return false;
+    __syncthreads();
+    GroupRay *g = reinterpret_cast<GroupRay *>(smem + group_lds_offset(kp.cap, kp.stage)) + grp;
+    StagedEntry *chunk = reinterpret_cast<StagedEntry *>(smem + stage_lds_offset(kp.cap)) + grp * kp.stage;
+    for (uint32_t fb = 0; fb < F; fb += npix == 2 ? 32 : 64) {
+        const uint32_t f = fb + (npix == 2 ? lane & 31 : lane);
+        const bool active = f < F;
+        const double freq = image_group(kp, smem, w, f, g);
+        count_entries<true>(kp, smem, g);
+        Sweep sw;
+        BandRing<0> ring;
+        staged_sweep<APPROX, PREC, METHOD, 0>(kp, smem, g, false, freq, active, chunk, 0.0, sw, ring);
+        if (!active) continue;
+        double val;
+        if constexpr (KIND == IMG_OPTICAL_DEPTH) {
+            val = sw.Y; /* image_optical_depth (solver.tpp:2718-2758); 0 without a segment */
+        } else if (w.S == 0) {
+            val = boundary_intensity(kp, w.ip, freq); /* n_tot = 1 */
+        } else {
+            /* last row at the start point (image_feautrier_order_2, solver.tpp:2546-2559) */
+            const FwdElim fe = {sw.X, sw.XI, sw.Y, sw.prev_dtau, true};
+            val = 2.0 * fe_last(fe, sw.S_inner, boundary_intensity(kp, w.ip, freq * w.shift_centre)) -
+                  boundary_intensity(kp, w.ip, freq);
+        }
+        I[(size_t)pix * F + f] = val;
     }
-    /* the second ray is walked even when the first outgrew the buffer, so that
-       its length is reported too */
-    PixelWalk w1 = pixel_slot(smem, kp.cap, 1);
-    const bool ok1 = image_walk(kp, fr, pix0 + 1, w1, ImX, ImY);
-    if (!ok0 || !ok1) return false;
-    const uint32_t half = lane >> 5;
-    image_freqs<APPROX, PREC, KIND>(kp, half ? w1 : w0, pix0 + half, lane & 31, 32, I);
     return true;
 }
-
 
 /* one wave per ppw (1 or 2) consecutive pixels of one model's image */
 template <int APPROX, int PREC, int KIND>
@@ -2948,915 +2931,6 @@ __global__ __launch_bounds__(MGX_WAVE) void image_ray_kernel(const KParams *__re
 /* branch of every segment, the CloseLines windows and the interpolation      */
 /* counts are held fixed.                                                     */
 
-/* Emissivity and opacity of an entry; phi is the line profile value when the
-   entry has only its own line in the CloseLines window and no interpolation
-   partner (then eta = phi eps and chi = chi_min + phi kappa), NaN otherwise. */
-struct PointECT {
-    double eta, chi, phi;
-    bool valid;
-};
-
-template <int APPROX, int PREC>
-__device__ inline void eta_chi_tape(const KParams &kp, const OwnLine &ol, const Entry &e,
-                                    uint32_t line, double freq, PointECT &ec)
-{
-    ec.valid = true;
-    ec.phi = __builtin_nan("");
-    if (APPROX == MGX_APPROX_CLOSE_LINES && e.ifac == 0.0) {
-        const double W = kp.op.max_distance_opacity_contribution * (freq * gld(&kp.pts[e.nr].ub));
-        const double left = freq - W, right = freq + W;
-        if (!(ol.a_g < left) && ol.a_lo < left && !(right < ol.a_g) && right < ol.a_hi) {
-            /* the arithmetic of eta_chi_interp for a one-line window at t = 0 */
-            const double4 a = lp(kp, e.nr, kp.m.sorted_line_map[ol.g]);
-            const double prof = gaussian<PREC>(a.x, freq - ol.a_g);
-            ec.eta = 0.0 + prof * a.y;
-            ec.chi = kp.op.min_opacity + prof * a.z;
-            ec.phi = prof;
-            return;
-        }
-        if ((ol.a_g < left && right < ol.a_hi) || (right < ol.a_g && ol.a_lo < left)) {
-            /* no line in the window: eta = 0, chi = chi_min (phi = 0 reproduces both) */
-            ec.eta = 0.0;
-            ec.chi = kp.op.min_opacity;
-            ec.phi = 0.0;
-            return;
-        }
-    }
-    eta_chi_interp<APPROX, PREC>(kp, ol, e.nr, e.nri, e.ifac, line, freq, gld(&kp.pts[e.nr].ub),
-                                 ec.eta, ec.chi);
-}
-
-/* Segment kinds recorded for the reverse pass */
-#define MGX_SEG_ERF_GENERIC (-1.0)
-#define MGX_SEG_TRAPEZOID (-2.0)
-#define MGX_SEG_ERF_EMPTY (-3.0) /* no line in the window: no dependence on the lines */
-
-/*
- * segment() for the adjoint's forward sweep: the same values, plus the kind of
- * the segment for the reverse pass in g: g >= 0 for a line-integrated segment
- * with only the own line in the window, no interpolation partner and no
- * clamp (g = d dtau / d mean-opacity), MGX_SEG_ERF_GENERIC for the other
- * line-integrated segments, MGX_SEG_TRAPEZOID for the trapezoid rule.
- */
-template <int APPROX, int PREC>
-__device__ inline void segment_tape(const KParams &kp, const double *erf_tab, const OwnLine &ol,
-                                    const Entry &cu, const Entry &nx, double dZ, double freq,
-                                    uint32_t line, PointECT &ec_cu, PointECT &ec_nx,
-                                    double &dtau, double &S_cu, double &S_nx, double &g)
-{
-    const mgx_model &m = kp.m;
-    const double dshift = nx.shift - cu.shift;
-    const double dshift_abs = fabs(dshift);
-    const double2 du_c = dsm_ub(kp, cu.nr), du_n = dsm_ub(kp, nx.nr);
-    const double a = du_c.x, b = du_n.x;
-    const double dshift_max = (b < a) ? b : a;
-    const double cf = freq * cu.shift, nf = freq * nx.shift;
-    if (dshift_abs > dshift_max) {
-        if (APPROX == MGX_APPROX_CLOSE_LINES && cu.ifac == 0.0 && nx.ifac == 0.0) {
-            double left_freq, right_freq;
-            if (cf < nf) {
-                left_freq = cf;
-                right_freq = nf;
-            } else {
-                right_freq = cf;
-                left_freq = nf;
-            }
-            const double cb = kp.op.max_distance_opacity_contribution * (right_freq * du_c.y);
-            const double nb = kp.op.max_distance_opacity_contribution * (right_freq * du_n.y);
-            const double W = (cb < nb) ? nb : cb;
-            const double left = left_freq - W, right = right_freq + W;
-            if (!(ol.a_g < left) && ol.a_lo < left && !(right < ol.a_g) && right < ol.a_hi) {
-                /* the arithmetic of S_dtau_line_integrated for one line at t = 0 */
-                const uint32_t l = m.sorted_line_map[ol.g];
-                const double4 c = lp(kp, cu.nr, l), n = lp(kp, nx.nr, l);
-                const double linefreq = m.line[l];
-                const double avg_iw = (c.x + n.x) / 2.0;
-                double line_dtau, dop;
-                if (cf == nf) {
-                    const double prof = gaussian<PREC>(avg_iw, cf - linefreq);
-                    line_dtau = dZ * (prof * ((c.z + n.z) / 2.0) + kp.op.min_opacity);
-                    dop = dZ * prof;
-                } else {
-                    const double next_pos = (linefreq - nf) * avg_iw;
-                    const double curr_pos = (linefreq - cf) * avg_iw;
-                    const double diff_pos = next_pos - curr_pos;
-                    const double avg_op = (n.z + c.z) / 2.0;
-                    const float erf_diff = f_erf<PREC>((float)next_pos, erf_tab) -
-                                           f_erf<PREC>((float)curr_pos, erf_tab);
-                    const double h = 0.5 * rcp(diff_pos);
-                    const double erfterm = avg_op * (double)erf_diff * h;
-                    line_dtau = dZ * fma(avg_iw, erfterm, kp.op.min_opacity);
-                    dop = dZ * (avg_iw * ((double)erf_diff * h));
-                }
-                double d = 0.0 + line_dtau;
-                const double sum_Sc = fma(line_dtau, c.w, 0.0), sum_Sn = fma(line_dtau, n.w, 0.0);
-                const double bound_min_dtau = kp.op.min_opacity * dZ;
-                const bool clamped = (-bound_min_dtau < d) && (d < bound_min_dtau);
-                if (-bound_min_dtau < d) d = (bound_min_dtau < d) ? d : bound_min_dtau;
-                dtau = d;
-                const double rd = rcp(d);
-                S_cu = sum_Sc * rd;
-                S_nx = sum_Sn * rd;
-                g = clamped ? MGX_SEG_ERF_GENERIC : dop;
-                return;
-            }
-            if ((ol.a_g < left && right < ol.a_hi) || (right < ol.a_g && ol.a_lo < left)) {
-                /* empty window: the sums are zero and the depth is clamped to its bound */
-                double d = 0.0;
-                const double bound_min_dtau = kp.op.min_opacity * dZ;
-                if (-bound_min_dtau < d) d = (bound_min_dtau < d) ? d : bound_min_dtau;
-                dtau = d;
-                const double rd = rcp(d);
-                S_cu = 0.0 * rd;
-                S_nx = 0.0 * rd;
-                g = MGX_SEG_ERF_EMPTY;
-                return;
-            }
-        }
-        S_dtau_line_integrated<APPROX, PREC>(kp, erf_tab, ol, cu.nr, nx.nr, cu.nri, nx.nri, line,
-                                             cf, nf, cu.ifac, nx.ifac, dZ, du_c.y, du_n.y, dtau, S_cu,
-                                             S_nx);
-        g = MGX_SEG_ERF_GENERIC;
-        return;
-    }
-    if (!ec_cu.valid) eta_chi_tape<APPROX, PREC>(kp, ol, cu, line, cf, ec_cu);
-    if (!ec_nx.valid) eta_chi_tape<APPROX, PREC>(kp, ol, nx, line, nf, ec_nx);
-    S_cu = ec_cu.eta * rcp(ec_cu.chi);
-    S_nx = ec_nx.eta * rcp(ec_nx.chi);
-    dtau = 0.5 * (ec_cu.chi + ec_nx.chi) * dZ;
-    g = MGX_SEG_TRAPEZOID;
-}
-
-/* Tape of one half ray: segment k (counted from the outer end) stores five
-   doubles, Y, X, dtau, the segment kind g and the profile value phi of its
-   outer entry, each lane-interleaved (64 lanes side by side) within the
-   segment's record.  The words stay doubles in mixed mode too: the reverse
-   forms u_k - u_{k+1} from Y and X, which cancels where u is smooth, and the
-   inverse-width gradient sums terms of both signs over the profile, so a float
-   tape moved it by up to 6e-3 relative. */
-#define MGX_TAPE_WORDS 5
-struct Tape {
-    /* bytes of one segment's record (all 64 lanes) */
-    static constexpr size_t kRecord = (size_t)MGX_WAVE * 8 * MGX_TAPE_WORDS;
-    static __device__ __forceinline__ size_t offset(uint32_t k, uint32_t c, uint32_t lane)
-    {
-        return kRecord * k + (size_t)MGX_WAVE * 8 * c + 8 * lane;
-    }
-    static __device__ __forceinline__ void put(unsigned char *base, uint32_t k, uint32_t c,
-                                               uint32_t lane, double v)
-    {
-        *reinterpret_cast<double *>(base + offset(k, c, lane)) = v;
-    }
-    static __device__ __forceinline__ double get(const unsigned char *base, uint32_t k, uint32_t c,
-                                                 uint32_t lane)
-    {
-        return *reinterpret_cast<const double *>(base + offset(k, c, lane));
-    }
-};
-
-template <int PREC>
-struct SweepStore {
-    unsigned char *st; /* the half's tape (records of all 64 lanes) */
-    uint32_t lane;
-    uint32_t cap; /* segments that fit */
-    uint32_t n;   /* segments of the half (may exceed cap: nothing is stored past it) */
-    double I_b;   /* boundary intensity of the outer boundary row */
-};
-
-/* sweep_half of the forward kernel, recording the tape */
-template <int APPROX, int PREC>
-__device__ inline void sweep_half_tape(const KParams &kp, const double *s_erf, const OwnLine &ol,
-                                       bool backward, uint32_t S, uint32_t o, double shift0,
-                                       double shift_centre, const uint32_t *s_nxt,
-                                       const double *s_dZ, const double *s_sh,
-                                       const uint16_t *mtab, uint32_t l, double freq, Sweep &sw,
-                                       PointECT &ec_centre, SweepStore<PREC> &store)
-{
-    HalfIter it;
-    it.s = (int)S - 1;
-    hi_load_step(kp, it, l, o, shift0, s_nxt, s_dZ, s_sh, mtab);
-    Entry outer = hi_entry(it, o);
-    PointECT ec_out = {0.0, 0.0, 0.0, false};
-    sw.started = false;
-    store.n = 0;
-    for (;;) {
-        const double dz = hi_advance(kp, it, l, o, shift0, s_nxt, s_dZ, s_sh, mtab);
-        Entry inner = hi_entry(it, o);
-        if (it.s < 0) inner.shift = shift_centre;
-        PointECT ec_in = (it.s < 0) ? ec_centre : PointECT{0.0, 0.0, 0.0, false};
-        const Entry &cu = backward ? inner : outer;
-        const Entry &nx = backward ? outer : inner;
-        PointECT &ec_cu = backward ? ec_in : ec_out;
-        PointECT &ec_nx = backward ? ec_out : ec_in;
-        double dtau, S_cu, S_nx, g;
-        segment_tape<APPROX, PREC>(kp, s_erf, ol, cu, nx, dz, freq, l, ec_cu, ec_nx, dtau, S_cu,
-                                   S_nx, g);
-        const double S_out = backward ? S_nx : S_cu;
-        const double S_in = backward ? S_cu : S_nx;
-        const double S_row = backward ? (sw.started ? sw.S_prev_row : S_out) : S_out;
-        if (!sw.started) {
-            const double I_b = boundary_intensity(kp, outer.nr, freq * outer.shift);
-            store.I_b = I_b;
-            const double idt = rcp(dtau);
-            const double B_min = fma(2.0, idt, 1.0);
-            const double B = fma(2.0 * idt, idt, B_min);
-            sw.Y = fma(2.0 * I_b, idt, S_row) * rcp(B);
-            sw.X = 0.5 * B_min * dtau * dtau;
-            sw.XI = rcp(1.0 + sw.X);
-            sw.started = true;
-        } else {
-            const double avg = 0.5 * (sw.prev_dtau + dtau);
-            const double q_out = avg * sw.prev_dtau;
-            const double q_in = avg * dtau;
-            const double r = rcp(q_out);
-            sw.X = fma(r * sw.X, sw.XI, 1.0) * q_in;
-            sw.XI = rcp(1.0 + sw.X);
-            sw.Y = fma(r, sw.Y, S_row) * sw.XI * q_in;
-        }
-        sw.prev_dtau = dtau;
-        sw.S_inner = S_in;
-        sw.S_prev_row = S_in;
-        if (store.n < store.cap) {
-            typedef Tape T;
-            T::put(store.st, store.n, 0, store.lane, sw.Y);
-            T::put(store.st, store.n, 1, store.lane, sw.X);
-            T::put(store.st, store.n, 2, store.lane, dtau);
-            T::put(store.st, store.n, 3, store.lane, g);
-            T::put(store.st, store.n, 4, store.lane, ec_out.valid ? ec_out.phi : __builtin_nan(""));
-        }
-        store.n++;
-        outer = inner;
-        ec_out = ec_in;
-        if (it.s < 0) break;
-    }
-    ec_centre = ec_out;
-}
-
-/*
- * Gradient sink of one lane.  The outward walk of the reverse pass visits the
- * segments of walk step s (outer entry in step s) together, and all of them
- * touch only the two points crt_s and nxt_s; the own-line contributions for
- * those two points are summed in registers, and when the walk moves to step
- * s+1 the finished point (crt_s) is summed over the lanes that share the line
- * (width lanes, aligned) and added by one lane.  Contributions to any other
- * line are added by the lane directly.
- */
-struct GradSink {
-    double *g_eps, *g_kap;
-    uint32_t L;
-    uint32_t line;   /* own line of the reducing lanes */
-    uint32_t width;  /* lanes summed together (32 or 64), 0: no reduction */
-    uint32_t p_crt, p_nxt;
-    double e_crt, k_crt, e_nxt, k_nxt;
-    double *g_iw;    /* inverse-width gradient (IW instantiations only) */
-    double w_crt, w_nxt;
-};
-
-/* IW: the sink also carries the gradient with respect to the inverse line widths */
-template <bool IW = false>
-__device__ inline void sink_put(const GradSink &g, uint32_t p, uint32_t l, double de, double dk,
-                                double dw = 0.0)
-{
-    const size_t i = (size_t)p * g.L + l;
-    if (de != 0.0) unsafeAtomicAdd(&g.g_eps[i], de);
-    if (dk != 0.0) unsafeAtomicAdd(&g.g_kap[i], dk);
-    if (IW && dw != 0.0) unsafeAtomicAdd(&g.g_iw[i], dw);
-}
-
-template <bool IW = false>
-__device__ inline void sink_add(GradSink &g, uint32_t p, uint32_t l, double de, double dk,
-                                double dw = 0.0)
-{
-    if (l != g.line) {
-        sink_put<IW>(g, p, l, de, dk, dw);
-    } else if (p == g.p_nxt) {
-        g.e_nxt += de;
-        g.k_nxt += dk;
-        if (IW) g.w_nxt += dw;
-    } else {
-        g.e_crt += de;
-        g.k_crt += dk;
-        if (IW) g.w_crt += dw;
-    }
-}
-
-/* The sum of v over the aligned group of width lanes (2, 4, ..., 64) that holds
-   the lane, valid in the group's last lane; all lanes of the group active.
-   Within a row of 16 the partners come through DPP (lane ^ 1, lane ^ 2, then the
-   mirror images within 8 and 16 lanes, which pair the partial sums the same
-   way); rows are then joined by DPP broadcasts, row_bcast15 (0x142: lane 15 of
-   row r into row r + 1, here rows 1 and 3) and row_bcast31 (0x143: lane 31 into
-   rows 2 and 3), which leave the sum in the group's last row. */
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_rows(double v)
-{
-    const uint64_t b = __builtin_bit_cast(uint64_t, v);
-    const uint64_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, false);
-    const uint64_t hi =
-        (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, false);
-    return __builtin_bit_cast(double, (hi << 32) | lo);
-}
-
-__device__ __forceinline__ double group_sum(double v, uint32_t width)
-{
-    v += dpp_get<0xb1>(v); /* quad_perm [1, 0, 3, 2] */
-    if (width > 2) v += dpp_get<0x4e>(v); /* quad_perm [2, 3, 0, 1] */
-    if (width > 4) v += dpp_get<0x141>(v); /* row_half_mirror */
-    if (width > 8) v += dpp_get<0x140>(v); /* row_mirror */
-    if (width > 16) v += dpp_rows<0x142, 0xa>(v); /* rows 1, 3 += lane 15, 47 */
-    if (width > 32) v += dpp_rows<0x143, 0xc>(v); /* rows 2, 3 += lane 31 */
-    return v;
-}
-
-/* all lanes of a reduction group call this together */
-template <bool IW = false>
-__device__ inline void sink_flush(const GradSink &g, uint32_t p, double e, double k, double w)
-{
-    if (g.width == 0) {
-        sink_put<IW>(g, p, g.line, e, k, w);
-        return;
-    }
-    e = group_sum(e, g.width);
-    k = group_sum(k, g.width);
-    if (IW) w = group_sum(w, g.width);
-    if ((threadIdx.x & (g.width - 1)) == g.width - 1) sink_put<IW>(g, p, g.line, e, k, w);
-}
-
-/* the walk moves outward to a step whose points are (crt = old nxt, nxt) */
-template <bool IW = false>
-__device__ inline void sink_step(GradSink &g, uint32_t nxt)
-{
-    sink_flush<IW>(g, g.p_crt, g.e_crt, g.k_crt, g.w_crt);
-    g.p_crt = g.p_nxt;
-    g.e_crt = g.e_nxt;
-    g.k_crt = g.k_nxt;
-    g.w_crt = g.w_nxt;
-    g.p_nxt = nxt;
-    g.e_nxt = 0.0;
-    g.k_nxt = 0.0;
-    g.w_nxt = 0.0;
-}
-
-template <bool IW = false>
-__device__ inline void sink_finish(GradSink &g)
-{
-    sink_flush<IW>(g, g.p_crt, g.e_crt, g.k_crt, g.w_crt);
-    sink_flush<IW>(g, g.p_nxt, g.e_nxt, g.k_nxt, g.w_nxt);
-}
-
-/* partial derivatives of interpolate_log(a, b, t) = a^(1-t) b^t with value r */
-__device__ inline void interp_log_partials(double a, double b, double t, double r, double &da,
-                                           double &db)
-{
-    da = (t == 1.0) ? 0.0 : (1.0 - t) * r / a;
-    db = (t == 0.0) ? 0.0 : t * r / b;
-}
-
-/* adds (de, dk) to the gradients of (p, l) directly (the rare paths of the reverse
-   pass, which do not go through a lane's sink) */
-__device__ inline void grad_put(double *g_eps, double *g_kap, uint32_t L, uint32_t p, uint32_t l,
-                                double de, double dk)
-{
-    const size_t i = (size_t)p * L + l;
-    if (de != 0.0) unsafeAtomicAdd(&g_eps[i], de);
-    if (dk != 0.0) unsafeAtomicAdd(&g_kap[i], dk);
-}
-
-/* reverse of interpolate_linear(iw(p), iw(pi), t): partials 1 - t and t */
-__device__ inline void iw_put(double *g_iw, uint32_t L, uint32_t p, uint32_t pi, uint32_t l,
-                              double t, double bar)
-{
-    const double a = (1.0 - t) * bar;
-    if (a != 0.0) unsafeAtomicAdd(&g_iw[(size_t)p * L + l], a);
-    if (t != 0.0) {
-        const double b = t * bar;
-        if (b != 0.0) unsafeAtomicAdd(&g_iw[(size_t)pi * L + l], b);
-    }
-}
-
-/* d(gaussian(w, diff))/dw = exp(-x^2) (1 - 2 x^2) / sqrt(pi), x = w diff: the
-   derivative of the smooth profile, in double */
-__device__ inline double gaussian_dw(double w, double diff)
-{
-    const double x = w * diff;
-    return MGX_INVERSE_SQRT_PI * exp(-x * x) * (1.0 - 2.0 * x * x);
-}
-
-/* d(compute_dtau_single_line)/d(avg_iw) at fixed frequencies, of the smooth
-   function: dz avg_op d(profile)/dw when the two frequencies are equal, else the
-   derivative of dz avg_op (erf(np) - erf(cp)) / (2 (cf - nf)), np = (lf - nf) w,
-   cp = (lf - cf) w: dz avg_op (np exp(-np^2) - cp exp(-cp^2)) / (sqrt(pi) (np - cp)) */
-__device__ inline double dtau_line_dw(double avg_iw, double avg_op, double linefreq, double cf,
-                                      double nf, double dz)
-{
-    if (cf == nf) return dz * avg_op * gaussian_dw(avg_iw, cf - linefreq);
-    const double np = (linefreq - nf) * avg_iw, cp = (linefreq - cf) * avg_iw;
-    return dz * avg_op * MGX_INVERSE_SQRT_PI * (np * exp(-np * np) - cp * exp(-cp * cp)) /
-           (np - cp);
-}
-
-/* the inverse-width part of the reverse of compute_dtau_single_line; bar is the
-   adjoint of the line's optical depth */
-template <int PREC>
-__device__ inline void dtau_iw_bwd(double *g_iw, uint32_t L, uint32_t cp, uint32_t cpi,
-                                   uint32_t np, uint32_t npi, uint32_t l, double4 c, double4 cI,
-                                   double4 n, double4 nI, double op_c, double op_n, double linefreq,
-                                   double cf, double nf, double ct, double nt, double dz, double bar)
-{
-    if (bar == 0.0) return;
-    const double avg_iw = (interp_linear(c.x, cI.x, ct) + interp_linear(n.x, nI.x, nt)) / 2.0;
-    const double avg_op = (op_c + op_n) / 2.0;
-    const double wb = 0.5 * bar * dtau_line_dw(avg_iw, avg_op, linefreq, cf, nf, dz);
-    iw_put(g_iw, L, cp, cpi, l, ct, wb);
-    iw_put(g_iw, L, np, npi, l, nt, wb);
-}
-
-/* reverse of eta_chi_interp: eta_bar d(eta) + chi_bar d(chi), added directly
-   (and, with IW, the inverse widths' part into g_iw).
-   A rare path of the reverse pass (interpolated entries, several lines in the
-   window): kept out of line, with every argument by value so that the
-   caller's registers stay out of memory. */
-template <int APPROX, int PREC, bool IW = false>
-__device__ __attribute__((noinline)) void eta_chi_interp_bwd(
-    const KParams *kpp, OwnLine ol, uint32_t p1, uint32_t p2, double t, uint32_t ll, double freq,
-    double eta_bar, double chi_bar, double *g_eps, double *g_kap, double *g_iw)
-{
-    const KParams &kp = *kpp;
-    const mgx_model &m = kp.m;
-    uint32_t lo = 0, hi = m.nlines;
-    if (APPROX == MGX_APPROX_ONE_LINE) {
-        lo = ll;
-        hi = ll + 1;
-    } else if (APPROX == MGX_APPROX_CLOSE_LINES) {
-        const double W = kp.op.max_distance_opacity_contribution * (freq * gld(&kp.pts[p1].ub));
-        line_window(m, ol, freq - W, freq + W, lo, hi);
-    }
-    for (uint32_t s = lo; s < hi; s++) {
-        const uint32_t l = (APPROX == MGX_APPROX_CLOSE_LINES) ? m.sorted_line_map[s] : s;
-        const double diff = freq - m.line[l];
-        const double4 a = lp(kp, p1, l), b = lp(kp, p2, l);
-        const double iw = interp_linear(a.x, b.x, t);
-        const double prof = gaussian<PREC>(iw, diff);
-        const double ei = interp_log<PREC>(a.y, b.y, t), ki = interp_log<PREC>(a.z, b.z, t);
-        double de1, de2, dk1, dk2;
-        interp_log_partials(a.y, b.y, t, ei, de1, de2);
-        interp_log_partials(a.z, b.z, t, ki, dk1, dk2);
-        const double pe = prof * eta_bar, pk = prof * chi_bar;
-        grad_put(g_eps, g_kap, m.nlines, p1, l, pe * de1, pk * dk1);
-        if (t != 0.0) grad_put(g_eps, g_kap, m.nlines, p2, l, pe * de2, pk * dk2);
-        /* eta = prof eps_i, chi = chi_min + prof kap_i */
-        if (IW) iw_put(g_iw, m.nlines, p1, p2, l, t, gaussian_dw(iw, diff) * (eta_bar * ei + chi_bar * ki));
-    }
-}
-
-/* d(compute_dtau_single_line)/d(avg_op) */
-template <int PREC>
-__device__ double dtau_single_line_dop(const double *erf_tab, double4 c, double4 cI, double4 n,
-                                       double4 nI, double linefreq, double curr_freq,
-                                       double next_freq, double curr_interp, double next_interp,
-                                       double dz)
-{
-    const double iw_c = interp_linear(c.x, cI.x, curr_interp);
-    const double iw_n = interp_linear(n.x, nI.x, next_interp);
-    const double avg_iw = (iw_c + iw_n) / 2.0;
-    if (curr_freq == next_freq) return dz * gaussian<PREC>(avg_iw, curr_freq - linefreq);
-    const double next_pos = (linefreq - next_freq) * avg_iw;
-    const double curr_pos = (linefreq - curr_freq) * avg_iw;
-    const double diff_pos = next_pos - curr_pos;
-    const float erf_diff = f_erf<PREC>((float)next_pos, erf_tab) - f_erf<PREC>((float)curr_pos, erf_tab);
-    return dz * (avg_iw * ((double)erf_diff * (0.5 * rcp(diff_pos))));
-}
-
-/* reverse of the line terms at one end of a segment: opacity (kappa interpolation,
-   value op) and line source (interpolation of eps/kappa, value S), added directly */
-__device__ inline void line_end_bwd(double *g_eps, double *g_kap, uint32_t L, uint32_t p,
-                                    uint32_t pi, uint32_t l, double t, double4 a, double4 b,
-                                    double op, double S, double op_bar, double S_bar)
-{
-    double dk1, dk2, dR1, dR2;
-    interp_log_partials(a.z, b.z, t, op, dk1, dk2);
-    interp_log_partials(a.w, b.w, t, S, dR1, dR2);
-    /* R = eps/kappa: dR/deps = 1/kappa, dR/dkappa = -R/kappa */
-    const double r1 = S_bar * dR1 * rcp(a.z);
-    grad_put(g_eps, g_kap, L, p, l, r1, op_bar * dk1 - r1 * a.w);
-    if (t != 0.0) {
-        const double r2 = S_bar * dR2 * rcp(b.z);
-        grad_put(g_eps, g_kap, L, pi, l, r2, op_bar * dk2 - r2 * b.w);
-    }
-}
-
-/* reverse of S_dtau_line_integrated (the general case: out of line, arguments by
-   value, gradients added directly) */
-template <int APPROX, int PREC, bool IW = false>
-__device__ __attribute__((noinline)) void S_dtau_line_integrated_bwd(
-    const KParams *kpp, const double *erf_tab, OwnLine ol, uint32_t cp, uint32_t np, uint32_t cpi,
-    uint32_t npi, uint32_t lineidx, double currfreq, double nextfreq, double curr_interp,
-    double next_interp, double dZ, double dtau_bar, double Sc_bar, double Sn_bar, double *g_eps,
-    double *g_kap, double *g_iw)
-{
-    const KParams &kp = *kpp;
-    const mgx_model &m = kp.m;
-    const uint32_t L = m.nlines;
-    if (APPROX == MGX_APPROX_ONE_LINE) {
-        const double4 c = lp(kp, cp, lineidx), cI = lp(kp, cpi, lineidx);
-        const double4 n = lp(kp, np, lineidx), nI = lp(kp, npi, lineidx);
-        const double dop = dtau_single_line_dop<PREC>(erf_tab, c, cI, n, nI, m.line[lineidx],
-                                                      currfreq, nextfreq, curr_interp,
-                                                      next_interp, dZ);
-        const double op_c = interp_log<PREC>(c.z, cI.z, curr_interp);
-        const double op_n = interp_log<PREC>(n.z, nI.z, next_interp);
-        line_end_bwd(g_eps, g_kap, L, cp, cpi, lineidx, curr_interp, c, cI, op_c,
-                     interp_log<PREC>(c.w, cI.w, curr_interp), 0.5 * dop * dtau_bar, Sc_bar);
-        line_end_bwd(g_eps, g_kap, L, np, npi, lineidx, next_interp, n, nI, op_n,
-                     interp_log<PREC>(n.w, nI.w, next_interp), 0.5 * dop * dtau_bar, Sn_bar);
-        if (IW)
-            dtau_iw_bwd<PREC>(g_iw, L, cp, cpi, np, npi, lineidx, c, cI, n, nI, op_c, op_n,
-                              m.line[lineidx], currfreq, nextfreq, curr_interp, next_interp, dZ,
-                              dtau_bar);
-        return;
-    }
-    uint32_t lo = 0, hi = m.nlines;
-    if (APPROX == MGX_APPROX_CLOSE_LINES) {
-        double left_freq, right_freq;
-        if (currfreq < nextfreq) {
-            left_freq = currfreq;
-            right_freq = nextfreq;
-        } else {
-            right_freq = currfreq;
-            left_freq = nextfreq;
-        }
-        const double cb = kp.op.max_distance_opacity_contribution * (right_freq * gld(&kp.pts[cp].ub));
-        const double nb = kp.op.max_distance_opacity_contribution * (right_freq * gld(&kp.pts[np].ub));
-        const double W = (cb < nb) ? nb : cb;
-        line_window(m, ol, left_freq - W, right_freq + W, lo, hi);
-    }
-    if (hi == lo + 1) {
-        /* one line in the window: a single pass (the erf difference serves the
-           optical depth and its derivative) */
-        const uint32_t l = (APPROX == MGX_APPROX_CLOSE_LINES) ? m.sorted_line_map[lo] : lo;
-        const double4 c = lp(kp, cp, l), cI = lp(kp, cpi, l);
-        const double4 n = lp(kp, np, l), nI = lp(kp, npi, l);
-        const double linefreq = m.line[l];
-        const double iw_c = interp_linear(c.x, cI.x, curr_interp);
-        const double iw_n = interp_linear(n.x, nI.x, next_interp);
-        const double avg_iw = (iw_c + iw_n) / 2.0;
-        const double op_c = interp_log<PREC>(c.z, cI.z, curr_interp);
-        const double op_n = interp_log<PREC>(n.z, nI.z, next_interp);
-        double line_dtau, dop;
-        if (currfreq == nextfreq) {
-            const double prof = gaussian<PREC>(avg_iw, currfreq - linefreq);
-            line_dtau = dZ * (prof * ((op_c + op_n) / 2.0) + kp.op.min_opacity);
-            dop = dZ * prof;
-        } else {
-            const double next_pos = (linefreq - nextfreq) * avg_iw;
-            const double curr_pos = (linefreq - currfreq) * avg_iw;
-            const double diff_pos = next_pos - curr_pos;
-            const double avg_op = (op_n + op_c) / 2.0;
-            const float erf_diff =
-                f_erf<PREC>((float)next_pos, erf_tab) - f_erf<PREC>((float)curr_pos, erf_tab);
-            const double ed = (double)erf_diff * (0.5 * rcp(diff_pos));
-            line_dtau = dZ * fma(avg_iw, avg_op * ed, kp.op.min_opacity);
-            dop = dZ * (avg_iw * ed);
-        }
-        const double Sc = interp_log<PREC>(c.w, cI.w, curr_interp);
-        const double Sn = interp_log<PREC>(n.w, nI.w, next_interp);
-        double d = line_dtau;
-        bool clamped = false;
-        if (APPROX == MGX_APPROX_CLOSE_LINES) {
-            const double bound_min_dtau = kp.op.min_opacity * dZ;
-            if (-bound_min_dtau < d && d < bound_min_dtau) {
-                d = bound_min_dtau;
-                clamped = true;
-            }
-        }
-        const double rd = rcp(d);
-        const double sSc_bar = Sc_bar * rd, sSn_bar = Sn_bar * rd;
-        /* one line: unclamped, S = S_l exactly and the adjoint of the line depth is
-           dtau_bar; clamped, the depth is the bound and S scales with the line depth */
-        const double ld_bar = clamped ? sSc_bar * Sc + sSn_bar * Sn : dtau_bar;
-        line_end_bwd(g_eps, g_kap, L, cp, cpi, l, curr_interp, c, cI, op_c, Sc, 0.5 * dop * ld_bar,
-                     sSc_bar * line_dtau);
-        line_end_bwd(g_eps, g_kap, L, np, npi, l, next_interp, n, nI, op_n, Sn, 0.5 * dop * ld_bar,
-                     sSn_bar * line_dtau);
-        if (IW)
-            dtau_iw_bwd<PREC>(g_iw, L, cp, cpi, np, npi, l, c, cI, n, nI, op_c, op_n, linefreq,
-                              currfreq, nextfreq, curr_interp, next_interp, dZ, ld_bar);
-        return;
-    }
-    /* forward sums (the same operations as S_dtau_line_integrated) */
-    double sum_dtau = 0.0, sum_Sc = 0.0, sum_Sn = 0.0;
-    for (uint32_t s = lo; s < hi; s++) {
-        const uint32_t l = (APPROX == MGX_APPROX_CLOSE_LINES) ? m.sorted_line_map[s] : s;
-        const double4 c = lp(kp, cp, l), cI = lp(kp, cpi, l);
-        const double4 n = lp(kp, np, l), nI = lp(kp, npi, l);
-        const double line_dtau = dtau_single_line<PREC>(kp, erf_tab, c, cI, n, nI, m.line[l],
-                                                        currfreq, nextfreq, curr_interp,
-                                                        next_interp, dZ);
-        sum_dtau += line_dtau;
-        sum_Sc = fma(line_dtau, interp_log<PREC>(c.w, cI.w, curr_interp), sum_Sc);
-        sum_Sn = fma(line_dtau, interp_log<PREC>(n.w, nI.w, next_interp), sum_Sn);
-    }
-    double d = sum_dtau;
-    bool clamped = false;
-    if (APPROX == MGX_APPROX_CLOSE_LINES) {
-        const double bound_min_dtau = kp.op.min_opacity * dZ;
-        if (-bound_min_dtau < d && d < bound_min_dtau) {
-            d = bound_min_dtau;
-            clamped = true;
-        }
-    }
-    const double rd = rcp(d);
-    const double sSc_bar = Sc_bar * rd, sSn_bar = Sn_bar * rd;
-    const double sdt_bar =
-        clamped ? 0.0 : dtau_bar - sSc_bar * (sum_Sc * rd) - sSn_bar * (sum_Sn * rd);
-    for (uint32_t s = lo; s < hi; s++) {
-        const uint32_t l = (APPROX == MGX_APPROX_CLOSE_LINES) ? m.sorted_line_map[s] : s;
-        const double4 c = lp(kp, cp, l), cI = lp(kp, cpi, l);
-        const double4 n = lp(kp, np, l), nI = lp(kp, npi, l);
-        const double line_dtau = dtau_single_line<PREC>(kp, erf_tab, c, cI, n, nI, m.line[l],
-                                                        currfreq, nextfreq, curr_interp,
-                                                        next_interp, dZ);
-        const double Sc = interp_log<PREC>(c.w, cI.w, curr_interp);
-        const double Sn = interp_log<PREC>(n.w, nI.w, next_interp);
-        const double op_c = interp_log<PREC>(c.z, cI.z, curr_interp);
-        const double op_n = interp_log<PREC>(n.z, nI.z, next_interp);
-        const double ld_bar = sdt_bar + sSc_bar * Sc + sSn_bar * Sn;
-        const double dop = dtau_single_line_dop<PREC>(erf_tab, c, cI, n, nI, m.line[l], currfreq,
-                                                      nextfreq, curr_interp, next_interp, dZ);
-        line_end_bwd(g_eps, g_kap, L, cp, cpi, l, curr_interp, c, cI, op_c, Sc, 0.5 * dop * ld_bar,
-                     sSc_bar * line_dtau);
-        line_end_bwd(g_eps, g_kap, L, np, npi, l, next_interp, n, nI, op_n, Sn, 0.5 * dop * ld_bar,
-                     sSn_bar * line_dtau);
-        if (IW)
-            dtau_iw_bwd<PREC>(g_iw, L, cp, cpi, np, npi, l, c, cI, n, nI, op_c, op_n, m.line[l],
-                              currfreq, nextfreq, curr_interp, next_interp, dZ, ld_bar);
-    }
-}
-
-/* emissivity/opacity of an entry, its profile value (NaN: not of the simple
-   kind) and the adjoints collected for them from the trapezoid segments on
-   either side (one back-propagation per entry) */
-struct EntryBar {
-    double eta, chi, phi, eta_bar, chi_bar;
-    bool have;
-};
-
-template <int APPROX, int PREC>
-__device__ __attribute__((noinline)) double2 eta_chi_generic(const KParams *kpp, OwnLine ol,
-                                                             uint32_t nr, uint32_t nri,
-                                                             double ifac, double f,
-                                                             uint32_t line)
-{
-    double2 r;
-    eta_chi_interp<APPROX, PREC>(*kpp, ol, nr, nri, ifac, line, f, gld(&kpp->pts[nr].ub), r.x, r.y);
-    return r;
-}
-
-/* eta and chi of an entry for the reverse pass: from the recorded profile value
-   when there is one (the forward arithmetic of eta_chi_tape), else recomputed */
-template <int APPROX, int PREC>
-__device__ inline void entry_eta_chi(const KParams &kp, const OwnLine &ol, const Entry &e,
-                                     double freq, uint32_t line, uint32_t lown, EntryBar &eb)
-{
-    if (eb.have) return;
-    if (eb.phi == eb.phi) {
-        const double4 a = lp(kp, e.nr, lown);
-        eb.eta = 0.0 + eb.phi * a.y;
-        eb.chi = kp.op.min_opacity + eb.phi * a.z;
-    } else {
-        const double2 r =
-            eta_chi_generic<APPROX, PREC>(&kp, ol, e.nr, e.nri, e.ifac, freq * e.shift, line);
-        eb.eta = r.x;
-        eb.chi = r.y;
-    }
-    eb.have = true;
-}
-
-/* back-propagates an entry's collected (eta, chi) adjoints */
-template <int APPROX, int PREC, bool IW = false>
-__device__ inline void entry_bwd(const KParams &kp, const OwnLine &ol, const Entry &e, double freq,
-                                 uint32_t line, uint32_t lown, const EntryBar &eb, GradSink &g)
-{
-    if (eb.eta_bar == 0.0 && eb.chi_bar == 0.0) return;
-    if (eb.phi == eb.phi) {
-        /* eta = phi eps, chi = chi_min + phi kappa at this entry's own point, phi the
-           profile of its inverse width (phi = 0: no line in the window) */
-        double dw = 0.0;
-        if (IW && eb.phi != 0.0) {
-            const double4 a = lp(kp, e.nr, lown);
-            dw = gaussian_dw(a.x, freq * e.shift - ol.a_g) * (a.y * eb.eta_bar + a.z * eb.chi_bar);
-        }
-        sink_add<IW>(g, e.nr, lown, eb.phi * eb.eta_bar, eb.phi * eb.chi_bar, dw);
-    } else {
-        eta_chi_interp_bwd<APPROX, PREC, IW>(&kp, ol, e.nr, e.nri, e.ifac, line, freq * e.shift,
-                                             eb.eta_bar, eb.chi_bar, g.g_eps, g.g_kap, g.g_iw);
-    }
-}
-
-/*
- * Reverse of one segment.  dtau_bar, Sc_bar, Sn_bar are the adjoints of its
- * optical depth and of its two source values; kind is the tape's g.
- * Line-integrated segments scatter their gradients directly (from the recorded
- * d dtau / d mean-opacity when g >= 0, else by recomputation); trapezoid
- * segments add the adjoints of (eta, chi) at their two entries to ecu / enx.
- */
-template <int APPROX, int PREC, bool IW = false>
-__device__ void segment_bwd(const KParams &kp, const double *erf_tab, const OwnLine &ol,
-                            const Entry &cu, const Entry &nx, double dZ, double freq,
-                            uint32_t line, uint32_t lown, double d, double kind, double dtau_bar,
-                            double Sc_bar, double Sn_bar, GradSink &g, EntryBar &ecu,
-                            EntryBar &enx)
-{
-    if (kind >= 0.0) {
-        /* one line, no interpolation partner, not clamped: dtau = line_dtau = d */
-        const double4 c = lp(kp, cu.nr, lown), n = lp(kp, nx.nr, lown);
-        const double rd = rcp(d);
-        const double sSc_bar = Sc_bar * rd, sSn_bar = Sn_bar * rd;
-        /* the segment's sources are the line's own (S = d S_l / d): the adjoint of the
-           line depth is dtau_bar (the source terms cancel exactly) */
-        const double ld_bar = dtau_bar;
-        const double op_bar = 0.5 * kind * ld_bar;
-        const double rc = sSc_bar * d * rcp(c.z), rn = sSn_bar * d * rcp(n.z);
-        double wb = 0.0;
-        if (IW && ld_bar != 0.0)
-            wb = 0.5 * ld_bar * dtau_line_dw((c.x + n.x) / 2.0, (n.z + c.z) / 2.0, ol.a_g,
-                                             freq * cu.shift, freq * nx.shift, dZ);
-        sink_add<IW>(g, cu.nr, lown, rc, op_bar - rc * c.w, wb);
-        sink_add<IW>(g, nx.nr, lown, rn, op_bar - rn * n.w, wb);
-        return;
-    }
-    if (kind == MGX_SEG_ERF_EMPTY) return;
-    const double cf = freq * cu.shift, nf = freq * nx.shift;
-    if (kind == MGX_SEG_ERF_GENERIC) {
-        S_dtau_line_integrated_bwd<APPROX, PREC, IW>(&kp, erf_tab, ol, cu.nr, nx.nr, cu.nri,
-                                                     nx.nri, line, cf, nf, cu.ifac, nx.ifac, dZ,
-                                                     dtau_bar, Sc_bar, Sn_bar, g.g_eps, g.g_kap,
-                                                     g.g_iw);
-        return;
-    }
-    entry_eta_chi<APPROX, PREC>(kp, ol, cu, freq, line, lown, ecu);
-    entry_eta_chi<APPROX, PREC>(kp, ol, nx, freq, line, lown, enx);
-    const double ric = rcp(ecu.chi), rin = rcp(enx.chi);
-    ecu.chi_bar += 0.5 * dZ * dtau_bar - Sc_bar * ecu.eta * ric * ric;
-    enx.chi_bar += 0.5 * dZ * dtau_bar - Sn_bar * enx.eta * rin * rin;
-    ecu.eta_bar += Sc_bar * ric;
-    enx.eta_bar += Sn_bar * rin;
-}
-
-/* derivative of a row  u + A_a (u - u_a) + A_b (u - u_b) = S  with respect to d_a,
-   A_a = 2/((d_a + d_b) d_a), A_b = 2/((d_a + d_b) d_b); Da = u - u_a, Db = u - u_b */
-__device__ inline double row_dd(double da, double db, double Da, double Db)
-{
-    const double s = da + db;
-    const double rs = rcp(s);
-    const double Aa = 2.0 * rs * rcp(da), Ab = 2.0 * rs * rcp(db);
-    return -Aa * (rs + rcp(da)) * Da - Ab * rs * Db;
-}
-
-/* derivative of a boundary row  (1 + 2/d) u + (2/d^2)(u - u_n) = S + 2 I/d  w.r.t. d */
-__device__ inline double bdy_row_dd(double d, double I, double u, double Dn)
-{
-    const double r = rcp(d);
-    return 2.0 * r * r * (I - u) - 4.0 * r * r * r * Dn;
-}
-
-/*
- * Reverse pass over one half ray, outward from the centre.  With the system
- * T u = r of the ray (rows as in the reference's elimination) and the seed
- * ubar at the centre, lam = T^-T e_c ubar = D T^-1 D^-1 e_c ubar (D T is
- * symmetric, D = half the sum of a row's two segment depths, or half the one
- * depth of a boundary row), so lam_k = D_k mu_k with mu_k = XI_k mu_{k+1}, the
- * same factors that give u_k = Y_k + XI_k u_{k+1}.  dL/dS_k = lam_k and
- * dL/dd = -sum_rows lam_row dR_row/dd; the differences u_k - u_{k+1} are taken
- * as Y_k - X_k XI_k u_{k+1} (optically thin steps leave u constant to ~13
- * digits, so subtracting two u values would lose them).
- *
- * Segment sources as the reference uses them (row n takes Scurr of segment n,
- * the last row Snext of the last segment): rr-side half (backward = false):
- * segment k supplies its outer row (Sc), and its Sn feeds the centre row when
- * the centre is the last row; antipod-side half: segment k supplies the row of
- * its inner entry (Sc) and segment 0 the boundary row (Sn).
- */
-struct RevCentre {
-    double u, mu, lam; /* u, D^-1-scaled adjoint and adjoint of the centre row */
-    double dbar;       /* the centre row's part of dL/d(depth of the innermost segment) */
-    bool centre_last;  /* rr-side half only: the centre is the system's last row */
-    PointECT ec;       /* the centre entry's cache from the forward sweeps */
-};
-
-template <int APPROX, int PREC, bool IW = false>
-__device__ __forceinline__ void reverse_half(const KParams &kp, const double *s_erf, const OwnLine &ol,
-                             bool backward, uint32_t S, uint32_t o, double shift0,
-                             double shift_centre, const uint32_t *s_nxt, const double *s_dZ,
-                             const double *s_sh, const uint16_t *mtab, uint32_t l, double freq,
-                             const SweepStore<PREC> store, const RevCentre rc, GradSink g)
-{
-    const uint32_t K = store.n;
-    const uint32_t lown = kp.m.sorted_line_map[ol.g];
-    /* outward entry iterator: step s, entry i = 1..m_s */
-    HalfIter it;
-    it.s = 0;
-    hi_load_step(kp, it, l, o, shift0, s_nxt, s_dZ, s_sh, mtab);
-    it.i = 1;
-    Entry inner;
-    inner.nr = o;
-    inner.nri = o;
-    inner.ifac = 0.0;
-    inner.shift = shift_centre;
-    g.p_crt = o;
-    g.p_nxt = it.nxt;
-    g.e_crt = g.k_crt = g.e_nxt = g.k_nxt = 0.0;
-    g.w_crt = g.w_nxt = 0.0;
-
-    double u_in = rc.u, mu_in = rc.mu, lam_in = rc.lam, dbar = rc.dbar;
-    EntryBar ein = {rc.ec.eta, rc.ec.chi, rc.ec.valid ? rc.ec.phi : __builtin_nan(""), 0.0, 0.0,
-                    rc.ec.valid};
-    typedef Tape T;
-    const uint32_t ln = store.lane;
-    double Y = T::get(store.st, K - 1, 0, ln), X = T::get(store.st, K - 1, 1, ln),
-           d = T::get(store.st, K - 1, 2, ln), kind = T::get(store.st, K - 1, 3, ln),
-           phi = T::get(store.st, K - 1, 4, ln);
-    /* the record of the segment after next, loaded one iteration ahead of its use so
-       that the global load's latency overlaps a segment's reverse */
-    double fY = 0.0, fX = 0.0, fd = 0.0, fk = 0.0, fp = 0.0;
-    if (K >= 2) {
-        fY = T::get(store.st, K - 2, 0, ln);
-        fX = T::get(store.st, K - 2, 1, ln);
-        fd = T::get(store.st, K - 2, 2, ln);
-        fk = T::get(store.st, K - 2, 3, ln);
-        fp = T::get(store.st, K - 2, 4, ln);
-    }
-    for (uint32_t k = K; k-- > 0;) {
-        const Entry outer = hi_entry(it, o);
-        const double dz = it.dZ;
-        const double XI = rcp(1.0 + X);
-        const double u_k = fma(XI, u_in, Y);
-        const double mu_k = XI * mu_in;
-        const double Din = fma(-X * XI, u_in, Y); /* u_k - u_in */
-        double lam_k, dbar_next = 0.0, Yn = 0.0, Xn = 0.0, dn = 0.0, kn = 0.0, pn = 0.0;
-        if (k > 0) {
-            Yn = fY;
-            Xn = fX;
-            dn = fd;
-            kn = fk;
-            pn = fp;
-            if (k >= 2) {
-                fY = T::get(store.st, k - 2, 0, ln);
-                fX = T::get(store.st, k - 2, 1, ln);
-                fd = T::get(store.st, k - 2, 2, ln);
-                fk = T::get(store.st, k - 2, 3, ln);
-                fp = T::get(store.st, k - 2, 4, ln);
-            }
-            lam_k = 0.5 * (dn + d) * mu_k;
-            /* u_k - u_{k-1} = X_{k-1} XI_{k-1} u_k - Y_{k-1} */
-            const double XIn = rcp(1.0 + Xn);
-            const double Dout = fma(Xn * XIn, u_k, -Yn);
-            dbar -= lam_k * row_dd(d, dn, Din, Dout);
-            dbar_next = -lam_k * row_dd(dn, d, Dout, Din);
-        } else {
-            lam_k = 0.5 * d * mu_k;
-            dbar -= lam_k * bdy_row_dd(d, store.I_b, u_k, Din);
-        }
-        EntryBar eout = {0.0, 0.0, phi, 0.0, 0.0, false};
-        if (!backward) {
-            const double Sn_bar = (k == K - 1 && rc.centre_last) ? rc.lam : 0.0;
-            segment_bwd<APPROX, PREC, IW>(kp, s_erf, ol, outer, inner, dz, freq, l, lown, d, kind,
-                                      dbar, lam_k, Sn_bar, g, eout, ein);
-        } else {
-            const double Sn_bar = (k == 0) ? lam_k : 0.0;
-            segment_bwd<APPROX, PREC, IW>(kp, s_erf, ol, inner, outer, dz, freq, l, lown, d, kind,
-                                      dbar, lam_in, Sn_bar, g, ein, eout);
-        }
-        /* the inner entry has all its contributions now */
-        entry_bwd<APPROX, PREC, IW>(kp, ol, inner, freq, l, lown, ein, g);
-        if (k == 0) {
-            entry_bwd<APPROX, PREC, IW>(kp, ol, outer, freq, l, lown, eout, g);
-            break;
-        }
-        /* move outward */
-        ein = eout;
-        inner = outer;
-        u_in = u_k;
-        mu_in = mu_k;
-        lam_in = lam_k;
-        dbar = dbar_next;
-        Y = Yn;
-        X = Xn;
-        d = dn;
-        kind = kn;
-        phi = pn;
-        if (it.i < it.m_s) {
-            it.i++;
-        } else {
-            it.s++;
-            hi_load_step(kp, it, l, o, shift0, s_nxt, s_dZ, s_sh, mtab);
-            it.i = 1;
-            sink_step<IW>(g, it.nxt);
-        }
-    }
-    sink_finish<IW>(g);
-}
-
 /*
  * Centre row of a ray pair after both sweeps: u at the centre, x_c = (T^-1)_cc
  * (the Lambda diagonal), D_c and the centre row's derivative with respect to
@@ -3901,8 +2975,9 @@ __device__ inline CentreRow centre_row(const KParams &kp, uint32_t o, double fre
         if (has_fw) {
             const double Dfw = fma(fw.X * fw.XI, c.u, -fw.Y); /* u_c - u_{c-1} */
             c.Dc = 0.5 * (fw.prev_dtau + dtau_c);
-            c.dd_fw = row_dd(fw.prev_dtau, dtau_c, Dfw, Dbw);
-            c.dd_bw = row_dd(dtau_c, fw.prev_dtau, Dbw, Dfw);
+            const double2 r = row_dd(fw.prev_dtau, dtau_c, Dfw, Dbw);
+            c.dd_fw = r.x;
+            c.dd_bw = r.y;
         } else {
             const double I_f = boundary_intensity(kp, o, freq * shift_c);
             c.Dc = 0.5 * dtau_c;
@@ -3930,32 +3005,26 @@ __device__ inline CentreRow centre_row(const KParams &kp, uint32_t o, double fre
  * (dJ/d kappa)^T J_bar into g_eps, g_kap (P, L).  Persistent grid: each wave takes
  * the next origin from a counter; it keeps the elimination state of its current ray
  * pair in its own slice of the scratch (2 halves x capE tape records).
- * The lane layout is the forward kernel's (two 32-lane line slots); lanes past
- * the last quadrature bin repeat it with a zero seed so every slot reduces its
- * gradients over 32 lanes.
+ * The lane layout is the forward kernel's.
  */
 template <int APPROX, int PREC, bool IW>
-__global__ __launch_bounds__(MGX_WAVE, MGX_ADJ_WAVES_PER_SIMD) void feautrier_adjoint_kernel(
+__global__ __launch_bounds__(MGX_WAVE, IW ? 2 : MGX_J_ADJOINT_WAVES_PER_SIMD) void feautrier_adjoint_kernel(
     const KParams *__restrict__ kpp, const double *__restrict__ J_bar, double *g_eps,
     double *g_kap, double *g_iw, double *scratch, uint32_t capE)
 {
     mgx_ref_tables_init();
     const KParams &kp = *kpp;
     extern __shared__ unsigned char smem[];
-    const double *s_erf = nullptr; /* erf needs no table */
     const mgx_model &m = kp.m;
-    const uint32_t lane = threadIdx.x;
+    const uint32_t lane = threadIdx.x, grp = lane >> 5;
     const uint32_t cap = kp.cap;
     const uint32_t P = m.npoints, F = m.nfreqs, Q = m.nquads;
-    uint32_t *s_nxt0 = reinterpret_cast<uint32_t *>(smem);
-    uint32_t *s_nxt1 = s_nxt0 + cap;
-    double *s_dZ0 = reinterpret_cast<double *>(smem + 8 * ((2 * cap * 4 + 7) / 8));
-    double *s_dZ1 = s_dZ0 + cap;
-    double *s_sh0 = s_dZ1 + cap;
-    double *s_sh1 = s_sh0 + cap;
-    uint16_t *s_m = reinterpret_cast<uint16_t *>(s_sh1 + cap);
+    GroupRay *g = reinterpret_cast<GroupRay *>(smem + group_lds_offset(cap, kp.stage)) + grp;
+    StagedEntry *chunk = reinterpret_cast<StagedEntry *>(smem + stage_lds_offset(cap)) + grp * kp.stage;
+    EntryGrad *sums = reinterpret_cast<EntryGrad *>(smem + acc_lds_offset(cap, kp.stage)) + grp * kp.stage;
     unsigned char *st_wave = reinterpret_cast<unsigned char *>(scratch) +
-                             (size_t)blockIdx.x * 2 * capE * Tape::kRecord;
+                             (size_t)blockIdx.x * 2 * capE * Tape::kRecord + 8 * lane;
+    const GradOut out = {g_eps, g_kap, g_iw};
 
     /* origins are handed out by an atomic counter (status word 3, cleared before
        the launch), so the waves finish together however the origins' costs vary */
@@ -3972,11 +3041,10 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_ADJ_WAVES_PER_SIMD) void feautrier_ad
             return;
         for (uint32_t rr = 0; rr < m.hnrays; rr++) {
             const uint32_t ar = gld(&m.antipod[rr]);
-            uint32_t S0, S1;
-            double sh00, sh01;
+            uint32_t S;
+            double shift0;
             __syncthreads();
-            int e = walk_half(kp, o, rr, s_nxt0, s_dZ0, s_sh0, S0, sh00);
-            if (!e) e = walk_half(kp, o, ar, s_nxt1, s_dZ1, s_sh1, S1, sh01);
+            const int e = walk_pair(kp, o, rr, ar, smem, S, shift0);
             if (e) {
                 if (lane == 0) {
                     atomicOr(&kp.status[0], (uint32_t)e);
@@ -3985,70 +3053,90 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_ADJ_WAVES_PER_SIMD) void feautrier_ad
                 return;
             }
             __syncthreads();
+            const uint32_t S0 = (uint32_t)__builtin_amdgcn_readlane((int)S, 0);
+            const uint32_t S1 = (uint32_t)__builtin_amdgcn_readlane((int)S, 32);
+            const double sh00 = read_lane(shift0, 0), sh01 = read_lane(shift0, 32);
             if (S0 == 0 && S1 == 0) continue; /* u = I_bdy: no dependence */
             const double w = ray_weight(m, o, rr);
-            const uint32_t Sall = S0 + S1;
             for (uint32_t slot0 = 0; slot0 < kp.nslots; slot0 += 2) {
-                const uint32_t lA = slot0 / kp.slots_per_line;
-                const uint32_t lB = (slot0 + 1 < kp.nslots) ? (slot0 + 1) / kp.slots_per_line : lA;
-                __syncthreads();
-                for (uint32_t i = lane; i < 2 * Sall; i += MGX_WAVE) {
-                    const uint32_t j = i / Sall, r = i % Sall;
-                    const uint32_t h = (r < S0) ? 0 : 1;
-                    const uint32_t stp = h ? r - S0 : r;
-                    const uint32_t *nx = h ? s_nxt1 : s_nxt0;
-                    const uint32_t crt = (stp == 0) ? o : nx[stp - 1];
-                    const uint32_t mm = n_interp_for_line(kp, j ? lB : lA, crt, nx[stp]);
-                    if (mm > 0xffffu) atomicOr(&kp.status[0], (uint32_t)ERR_INTERP);
-                    s_m[(j * 2 + h) * cap + stp] = (uint16_t)(mm > 0xffffu ? 0xffffu : mm);
-                }
-                __syncthreads();
-                const uint32_t jj = lane >> 5;
-                const uint32_t slot = slot0 + jj;
-                if (slot >= kp.nslots) continue; /* whole 32-lane half idle */
-                const uint32_t l = jj ? lB : lA;
-                const uint32_t z0 = (slot % kp.slots_per_line) * 32 + (lane & 31);
-                const uint32_t z = (z0 < Q) ? z0 : Q - 1;
-                const OwnLine ol = own_line(m, l);
-                const uint32_t f = l * Q + z;
+                const bool alone = slot0 + 1 == kp.nslots;
+                const uint32_t slot = alone ? slot0 : slot0 + grp;
+                const uint32_t l = slot / kp.slots_per_line;
+                const uint32_t z = (slot % kp.slots_per_line) * 32 + (lane & 31);
+                const bool active = z < Q;
+                const uint32_t f = l * Q + (active ? z : Q - 1);
                 const size_t of = (size_t)o * F + f;
                 const double freq = gld(&m.nu[of]);
-                const double ubar = (z0 < Q) ? 2.0 * w * J_bar[of] : 0.0;
-                PointECT ec_cent = {0.0, 0.0, 0.0, false};
-                Sweep bw, fw;
-                bw.started = fw.started = false;
-                SweepStore<PREC> st0{st_wave, lane, capE, 0, 0.0},
-                    st1{st_wave + (size_t)capE * Tape::kRecord, lane, capE, 0, 0.0};
-                if (S1 > 0)
-                    sweep_half_tape<APPROX, PREC>(kp, s_erf, ol, true, S1, o, sh01, 1.0, s_nxt1,
-                                                  s_dZ1, s_sh1, s_m + (jj * 2 + 1) * cap, l, freq,
-                                                  bw, ec_cent, st1);
-                if (S0 > 0)
-                    sweep_half_tape<APPROX, PREC>(kp, s_erf, ol, false, S0, o, sh00, 1.0, s_nxt0,
-                                                  s_dZ0, s_sh0, s_m + (jj * 2 + 0) * cap, l, freq,
-                                                  fw, ec_cent, st0);
-                if (st0.n > capE || st1.n > capE) {
+                const double ubar = active ? 2.0 * w * gld(&J_bar[of]) : 0.0;
+                const double fmin = group32(freq, [](double a, double b) { return a < b ? a : b; });
+                const double fmax = group32(freq, [](double a, double b) { return a < b ? b : a; });
+                /* the half ray that pass 0 (the antipod side) or 1 (the rr side) sweeps; a slot
+                   left alone puts one half on each group, in one pass */
+                const auto half_ray = [&](bool back) {
+                    __syncthreads();
                     if ((lane & 31) == 0) {
-                        atomicOr(&kp.status[0], (uint32_t)ERR_CAPE);
-                        atomicMax(&kp.status[2], st0.n > st1.n ? st0.n : st1.n);
+                        GroupRay r;
+                        r.o = o;
+                        r.line = l;
+                        r.S = back ? S1 : S0;
+                        r.list = back ? 1 : 0;
+                        r.shift0 = back ? sh01 : sh00;
+                        r.shift_c = 1.0;
+                        r.fmin = fmin;
+                        r.fmax = fmax;
+                        r.ol = own_line(m, l);
+                        *g = r;
                     }
-                    continue;
+                    __syncthreads();
+                    count_entries<false>(kp, smem, g);
+                };
+                Sweep fw, bw;
+                BandRing<0> ring;
+                double I_f = 0.0, I_b = 0.0; /* boundary intensities of the swept halves */
+                bool full = false;
+                const uint32_t passes = alone ? 1 : 2;
+#pragma unroll 1
+                for (uint32_t pass = 0; pass < passes; pass++) {
+                    const bool back = alone ? grp == 1 : pass == 0;
+                    half_ray(back);
+                    const uint32_t n = g->n;
+                    if (__ballot(n > capE)) {
+                        if ((lane & 31) == 0 && n > capE) {
+                            atomicOr(&kp.status[0], (uint32_t)ERR_CAPE);
+                            atomicMax(&kp.status[2], n);
+                        }
+                        full = true;
+                        break;
+                    }
+                    if (pass == 1) {
+                        bw = fw;
+                        I_b = I_f;
+                    }
+                    const Tape tape = {st_wave + (size_t)(back ? capE : 0) * Tape::kRecord, capE};
+                    staged_sweep<APPROX, PREC, METHOD_FEAUTRIER, 0, true>(kp, smem, g, back, freq, active, chunk,
+                                                                          0.0, fw, ring, &tape, &I_f);
                 }
-                const CentreRow c = centre_row<PREC>(kp, o, freq, 1.0, S0 > 0, S1 > 0, fw, bw);
+                if (full) continue;
+                if (alone) {
+                    Sweep other = fw;
+                    exchange_halves<METHOD_FEAUTRIER, 0>(other, ring);
+                    bw = grp ? fw : other;
+                    fw = grp ? other : fw;
+                }
+                CentreRow c = {0.0, 0.0, 1.0, 0.0, 0.0};
+                if (active) c = centre_row<PREC>(kp, o, freq, 1.0, S0 > 0, S1 > 0, fw, bw);
                 const double mu_c = ubar * c.xc * rcp(c.Dc);
                 const double lam_c = ubar * c.xc;
-                GradSink g{g_eps, g_kap, m.nlines, l, 32, 0, 0, 0.0, 0.0, 0.0, 0.0, g_iw, 0.0, 0.0};
-                if (S0 > 0) {
-                    const RevCentre rc{c.u, mu_c, lam_c, -lam_c * c.dd_fw, S1 == 0, ec_cent};
-                    reverse_half<APPROX, PREC, IW>(kp, s_erf, ol, false, S0, o, sh00, 1.0, s_nxt0,
-                                                   s_dZ0, s_sh0, s_m + (jj * 2 + 0) * cap, l,
-                                                   freq, st0, rc, g);
-                }
-                if (S1 > 0) {
-                    const RevCentre rc{c.u, mu_c, lam_c, -lam_c * c.dd_bw, false, ec_cent};
-                    reverse_half<APPROX, PREC, IW>(kp, s_erf, ol, true, S1, o, sh01, 1.0, s_nxt1,
-                                                   s_dZ1, s_sh1, s_m + (jj * 2 + 1) * cap, l,
-                                                   freq, st1, rc, g);
+                /* the rr side first: its counts are still there */
+#pragma unroll 1
+                for (uint32_t pass = 0; pass < passes; pass++) {
+                    const bool back = alone ? grp == 1 : pass == 1;
+                    if (pass == 1) half_ray(true);
+                    const Tape tape = {st_wave + (size_t)(back ? capE : 0) * Tape::kRecord, capE};
+                    const RevCentre rc = {c.u, mu_c, lam_c, -lam_c * (back ? c.dd_bw : c.dd_fw),
+                                          !back && S1 == 0};
+                    reverse_half<APPROX, PREC, IW>(kp, smem, g, back, freq, active, chunk, sums, tape,
+                                                   pass == 1 ? I_b : I_f, rc, out);
                 }
             }
         }
@@ -4057,87 +3145,73 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_ADJ_WAVES_PER_SIMD) void feautrier_ad
 
 /*
  * Adjoint of the projection-surface image: given I_bar (nx*ny, F), adds
- * (dI/d eps)^T I_bar and (dI/d kappa)^T I_bar into g_eps, g_kap.  One wave per
- * pixel (persistent grid), lanes across image frequencies in chunks of 64
- * (lanes past F repeat the last frequency with a zero seed).  I = 2 u_last -
- * I_bdy, so the seed of u at the start point is 2 I_bar.
+ * (dI/d eps)^T I_bar and (dI/d kappa)^T I_bar into g_eps, g_kap.  The lane layout is the
+ * imager's (persistent grid).  I = 2 u_last - I_bdy, so the seed of u at the start point
+ * is 2 I_bar.
  */
 template <int APPROX, int PREC, bool IW>
-__global__ __launch_bounds__(MGX_WAVE, MGX_ADJ_WAVES_PER_SIMD) void image_adjoint_kernel(
+__global__ __launch_bounds__(MGX_WAVE, MGX_IMAGE_ADJOINT_WAVES_PER_SIMD) void image_adjoint_kernel(
     const KParams *__restrict__ kpp, const ImageFrame *frp, const double *__restrict__ I_bar,
     double *g_eps, double *g_kap, double *g_iw, double *scratch, uint32_t capE)
 {
     mgx_ref_tables_init();
     const KParams &kp = *kpp;
     extern __shared__ unsigned char smem[];
-    const double *s_erf = nullptr; /* erf needs no table */
     const mgx_model &m = kp.m;
     const ImageFrame fr = *frp;
-    const uint32_t lane = threadIdx.x;
+    const uint32_t lane = threadIdx.x, grp = lane >> 5;
     const uint32_t F = m.nfreqs;
     const uint32_t npix = fr.nx * fr.ny;
     /* two pixels per wave when a half-wave covers the frequencies (image_pixels) */
     const uint32_t ppw = F <= 32 ? 2 : 1;
     const uint32_t nitems = (npix + ppw - 1) / ppw;
-    unsigned char *st_wave = reinterpret_cast<unsigned char *>(scratch) +
-                             (size_t)blockIdx.x * capE * Tape::kRecord;
+    GroupRay *g = reinterpret_cast<GroupRay *>(smem + group_lds_offset(kp.cap, kp.stage)) + grp;
+    StagedEntry *chunk = reinterpret_cast<StagedEntry *>(smem + stage_lds_offset(kp.cap)) + grp * kp.stage;
+    EntryGrad *sums = reinterpret_cast<EntryGrad *>(smem + acc_lds_offset(kp.cap, kp.stage)) + grp * kp.stage;
+    const Tape tape = {reinterpret_cast<unsigned char *>(scratch) + (size_t)blockIdx.x * capE * Tape::kRecord +
+                           8 * lane,
+                       capE};
+    const GradOut out = {g_eps, g_kap, g_iw};
 
-    for (uint32_t q = blockIdx.x; q < nitems; q += gridDim.x) {
+    for (uint32_t it = blockIdx.x; it < nitems; it += gridDim.x) {
         /* a buffer of this launch overflowed: the host clears the gradients and
            relaunches, so the remaining pixels are skipped */
         if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(&kp.status[0], __ATOMIC_RELAXED,
                                                              __HIP_MEMORY_SCOPE_AGENT)) &
             (ERR_CAP | ERR_CAPE))
             return;
-        const uint32_t p0 = q * ppw;
+        const uint32_t p0 = it * ppw;
         const uint32_t n = (p0 + ppw <= npix) ? ppw : npix - p0;
+        const uint32_t pix = n == 2 ? p0 + grp : p0;
         __syncthreads();
-        PixelWalk w0 = pixel_slot(smem, kp.cap, 0), w1 = pixel_slot(smem, kp.cap, 1);
-        const bool ok0 = image_walk(kp, fr, p0, w0, nullptr, nullptr);
-        const bool ok1 = n < 2 || image_walk(kp, fr, p0 + 1, w1, nullptr, nullptr);
-        if (!ok0 || !ok1) return;
-        /* the lanes of a group (the wave, or a half-wave per pixel) take one pixel */
-        const uint32_t gw = (n == 2) ? 32 : 64;
-        const uint32_t half = (n == 2) ? (lane >> 5) : 0;
-        const PixelWalk &w = half ? w1 : w0;
-        const uint32_t pix = p0 + half;
-        const uint32_t S = w.S, ip = w.ip;
-        if (S == 0) continue; /* I = I_bdy: no dependence (for the whole group) */
-        for (uint32_t fb = 0; fb < F; fb += gw) {
-            const uint32_t fl = fb + (lane & (gw - 1));
-            const uint32_t f = (fl < F) ? fl : F - 1;
-            const double freq = m.nu[(size_t)ip * F + f];
-            const uint32_t line = m.f_line[f];
-            const uint32_t ub_idx = upper_bound_d(m.sorted_line, m.nlines, freq);
-            const uint32_t own_l = m.sorted_line_map[ub_idx > 0 ? ub_idx - 1 : 0];
-            const OwnLine ol = own_line(m, own_l);
-            const double ubar = (fl < F) ? 2.0 * I_bar[(size_t)pix * F + f] : 0.0;
-            Sweep fw;
-            fw.started = false;
-            PointECT ec = {0.0, 0.0, 0.0, false};
-            SweepStore<PREC> st{st_wave, lane, capE, 0, 0.0};
-            sweep_half_tape<APPROX, PREC>(kp, s_erf, ol, false, S, ip, w.shift0, w.shift_centre,
-                                          w.nxt, w.dZ, w.sh, w.m, line, freq, fw, ec, st);
-            if (st.n > capE) {
-                if (lane == 0 || lane == 32) {
+        PixelWalk w;
+        const bool ok = image_walk(kp, fr, pix, smem, w, nullptr, nullptr);
+        if (__ballot(!ok)) return;
+        __syncthreads();
+        for (uint32_t fb = 0; fb < F; fb += n == 2 ? 32 : 64) {
+            const uint32_t f = fb + (n == 2 ? lane & 31 : lane);
+            const bool active = f < F && w.S > 0; /* without a segment I = I_bdy: no dependence */
+            const double freq = image_group(kp, smem, w, f, g);
+            const double ubar = active ? 2.0 * gld(&I_bar[(size_t)pix * F + f]) : 0.0;
+            count_entries<true>(kp, smem, g);
+            const uint32_t ne = g->n;
+            if (__ballot(ne > capE)) {
+                if ((lane & 31) == 0 && ne > capE) {
                     atomicOr(&kp.status[0], (uint32_t)ERR_CAPE);
-                    atomicMax(&kp.status[2], st.n);
+                    atomicMax(&kp.status[2], ne);
                 }
                 continue;
             }
-            const CentreRow c = centre_row<PREC>(kp, ip, freq, w.shift_centre, true, false, fw, fw);
-            const double mu_c = ubar * c.xc * rcp(c.Dc);
+            Sweep fw;
+            BandRing<0> ring;
+            double I_f = 0.0;
+            staged_sweep<APPROX, PREC, METHOD_FEAUTRIER, 0, true>(kp, smem, g, false, freq, active, chunk, 0.0, fw,
+                                                                  ring, &tape, &I_f);
+            CentreRow c = {0.0, 0.0, 1.0, 0.0, 0.0};
+            if (active) c = centre_row<PREC>(kp, w.ip, freq, w.shift_centre, true, false, fw, fw);
             const double lam_c = ubar * c.xc;
-            /* one reduction per group when the group's lanes share their own line */
-            const uint32_t l0 = __shfl(own_l, (int)(lane & ~(gw - 1)), MGX_WAVE);
-            const uint64_t same = __ballot(own_l == l0);
-            const uint64_t gmask = (gw == 64) ? ~0ull : (0xffffffffull << (32 * half));
-            const bool uniform = (same & gmask) == gmask;
-            GradSink g{g_eps, g_kap, m.nlines, own_l, uniform ? gw : 0u, 0, 0, 0.0, 0.0, 0.0, 0.0,
-                       g_iw, 0.0, 0.0};
-            const RevCentre rc{c.u, mu_c, lam_c, -lam_c * c.dd_fw, true, ec};
-            reverse_half<APPROX, PREC, IW>(kp, s_erf, ol, false, S, ip, w.shift0, w.shift_centre,
-                                           w.nxt, w.dZ, w.sh, w.m, line, freq, st, rc, g);
+            const RevCentre rc = {c.u, ubar * c.xc * rcp(c.Dc), lam_c, -lam_c * c.dd_fw, true};
+            reverse_half<APPROX, PREC, IW>(kp, smem, g, false, freq, active, chunk, sums, tape, I_f, rc, out);
         }
     }
 }
@@ -4247,8 +3321,7 @@ const uint32_t kMaxCap = 8192; /* walk steps per half ray: a ceiling above any L
 /*
  * State shared by the solver's two translation units: this file, and
  * mgx_adjoint.hip, which compiles it again with MGX_ADJOINT_TU for the adjoint
- * entry points (so that the adjoint kernels get code-generation options of their
- * own).  Kernel timing, the per-call workspace and the walk-capacity hints are
+ * entry points (so that the two halves of the kernels compile side by side).  Kernel timing, the per-call workspace and the walk-capacity hints are
  * defined here and declared in the adjoint unit.
  */
 #ifdef MGX_ADJOINT_TU
@@ -4675,7 +3748,8 @@ int adjoint_launch(hipStream_t st, DevBuffers &b, KParams &kp, const WalkKey &ke
     } report{total_ms};
     for (;;) {
         kp.cap = cap;
-        const size_t lds = walk_lds_bytes(cap);
+        kp.stage = stage_entries(cap, kp.m.nlines);
+        const size_t lds = adjoint_lds_bytes(cap, kp.stage);
         const uint32_t grid = grid_of(lds);
         const size_t bytes = (size_t)grid * per_wave_segments_factor * capE * Tape::kRecord;
         if (int e = ensure_workspace(bytes)) return e;
@@ -4899,7 +3973,7 @@ bool batch_images(const mgx_batch &B) { return B.n_img == B.n && B.images_on; }
 /* persistent grid of the image kernel (resident waves, at most the chunk count) */
 uint32_t image_grid_size(const mgx_batch &B)
 {
-    const size_t lds = walk_lds_bytes(B.cap);
+    const size_t lds = acc_lds_offset(B.cap, batch_stage(B));
     const uint32_t work = B.n_chunks ? B.n_chunks : 1;
     const bool fp64 = B.op.precision == MGX_PREC_FP64;
     if (B.op.approx == MGX_APPROX_NONE)
@@ -4911,7 +3985,7 @@ uint32_t image_grid_size(const mgx_batch &B)
 
 void launch_image_batch(const mgx_batch &B, hipStream_t st, uint32_t grid)
 {
-    const size_t lds = walk_lds_bytes(B.cap);
+    const size_t lds = acc_lds_offset(B.cap, batch_stage(B));
     const bool fp64 = B.op.precision == MGX_PREC_FP64;
     const dim3 g(grid), blk(MGX_WAVE);
 #define MGX_IMG_ARGS B.img_kps_dev, B.frames_dev, B.chunk_start_dev, B.slot_model_dev, B.n_img, \
@@ -4998,7 +4072,10 @@ int batch_upload(mgx_batch &B, hipStream_t st)
     HIP_TRY(hipMemcpyAsync(B.kps_dev, B.kps.data(), B.kps.size() * sizeof(KParams),
                            hipMemcpyHostToDevice, st));
     if (B.n_img) {
-        for (auto &k : B.img_kps) k.cap = B.cap;
+        for (auto &k : B.img_kps) {
+            k.cap = B.cap;
+            k.stage = batch_stage(B);
+        }
         HIP_TRY(hipMemcpyAsync(B.img_kps_dev, B.img_kps.data(), B.img_kps.size() * sizeof(KParams),
                                hipMemcpyHostToDevice, st));
     }
@@ -5529,7 +4606,8 @@ int mgx_image_device(const mgx_model *model, const mgx_options *opts, const doub
     ImageFrame *dfr = nullptr;
     if (int e = image_setup(model, opts, raydir, nx, ny, st, b, kp, dfr)) return e;
     const WalkKey ikey = image_key(*model, raydir, nx, ny);
-    return launch_with_capacity(st, b, kp, [&](size_t lds) {
+    return launch_with_capacity(st, b, kp, [&](size_t) {
+        const size_t lds = acc_lds_offset(kp.cap, kp.stage);
         /* two pixels per wave when a half-wave covers the frequencies */
         const uint32_t ppw = model->nfreqs <= 32 ? 2 : 1;
         const dim3 grid((nx * ny + ppw - 1) / ppw), block(MGX_WAVE);
@@ -5566,7 +4644,8 @@ int mgx_image_optical_depth_device(const mgx_model *model, const mgx_options *op
     ImageFrame *dfr = nullptr;
     if (int e = image_setup(model, opts, raydir, nx, ny, st, b, kp, dfr)) return e;
     const WalkKey ikey = image_key(*model, raydir, nx, ny);
-    return launch_with_capacity(st, b, kp, [&](size_t lds) {
+    return launch_with_capacity(st, b, kp, [&](size_t) {
+        const size_t lds = acc_lds_offset(kp.cap, kp.stage);
         /* two pixels per wave when a half-wave covers the frequencies */
         const uint32_t ppw = model->nfreqs <= 32 ? 2 : 1;
         const dim3 grid((nx * ny + ppw - 1) / ppw), block(MGX_WAVE);

@@ -284,17 +284,19 @@ __device__ inline void stage_entry(const KParams &kp, const GroupRay &g, const W
     *out = r;
 }
 
-/* Stages the entries from number k0 on (at most count, and not beyond the origin's) of
-   every group into its part of the chunk; all lanes of the wave call this together. */
+/* Stages the entries from number k0 on (count of them, those that exist) of every group
+   into its part of the chunk; k0 is the group's own.  All lanes of the wave call this
+   together. */
 template <int APPROX, int PREC>
-__device__ inline void stage_chunk(const KParams &kp, unsigned char *smem, const GroupRay *g, uint32_t k0,
+__device__ inline void stage_chunk(const KParams &kp, unsigned char *smem, const GroupRay *g, int k0,
                                    uint32_t count, StagedEntry *chunk)
 {
     const uint32_t q = threadIdx.x & 31;
+    const int k = k0 + (int)q;
     __syncthreads();
-    if (g->S > 0 && q < count && k0 + q <= g->n) {
+    if (g->S > 0 && q < count && k >= 0 && (uint32_t)k <= g->n) {
         const WalkList w = walk_list(smem, kp.cap, g->list, (threadIdx.x & (MGX_WAVE - 1)) >> 5);
-        stage_entry<APPROX, PREC>(kp, *g, w, k0 + q, chunk + q);
+        stage_entry<APPROX, PREC>(kp, *g, w, (uint32_t)k, chunk + q);
     }
     __syncthreads();
 }
@@ -311,7 +313,7 @@ struct WindowLine {
     double f;                /* line frequency */
     double iw_o, kap_o, src_o; /* outer end; an entry: iw, kap, eps */
     double iw_i, kap_i, src_i; /* inner end */
-    double pad;
+    uint32_t l, pad;         /* the line */
 };
 
 /* line data of line l at a staged entry; EPS: the emissivity in the place of the source */
@@ -333,18 +335,26 @@ __device__ __forceinline__ void line_at(const KParams &kp, const StagedEntry *e,
 }
 
 /* optical depth of one line between two ends at frequencies f_o and f_i
-   (compute_dtau_single_line, solver.tpp:2374-2455; the ends may be swapped) */
+   (compute_dtau_single_line, solver.tpp:2374-2455; the ends may be swapped), and its
+   derivative dop with respect to the mean opacity */
 template <int PREC>
 __device__ __forceinline__ double line_depth(double iw_o, double iw_i, double kap_o, double kap_i, double f_o,
-                                             double f_i, double linefreq, double dz, double min_opacity)
+                                             double f_i, double linefreq, double dz, double min_opacity,
+                                             double &dop)
 {
     const double avg_iw = (iw_o + iw_i) / 2.0;
     const double avg_op = (kap_o + kap_i) / 2.0;
-    if (f_o == f_i) return dz * (gaussian<PREC>(avg_iw, f_o - linefreq) * avg_op + min_opacity);
+    if (f_o == f_i) {
+        const double prof = gaussian<PREC>(avg_iw, f_o - linefreq);
+        dop = dz * prof;
+        return dz * (prof * avg_op + min_opacity);
+    }
     const double pos_i = (linefreq - f_i) * avg_iw;
     const double pos_o = (linefreq - f_o) * avg_iw;
     const float erf_diff = mgx_ref_erff((float)pos_i) - mgx_ref_erff((float)pos_o);
-    const double erfterm = avg_op * (double)erf_diff * (0.5 * rcp(pos_i - pos_o));
+    const double h = 0.5 * rcp(pos_i - pos_o);
+    const double erfterm = avg_op * (double)erf_diff * h;
+    dop = dz * (avg_iw * ((double)erf_diff * h));
     return dz * fma(avg_iw, erfterm, min_opacity);
 }
 
@@ -354,10 +364,13 @@ struct WindowSum {
     double a, b, c;
 };
 
-template <int APPROX, int PREC, bool ENTRY>
-__device__ __forceinline__ WindowSum window_sum(const KParams &kp, const GroupRay *g, WindowLine *lines, uint32_t nw,
-                                                const StagedEntry *eo, const StagedEntry *ei, double f_o,
-                                                double f_i, bool mine)
+/* Stages the lines in the windows round by round and hands each to take(line, its index,
+   whether it is in the bin's window), in the sorted order; mine marks the bins that have a
+   window here.  All lanes of the wave call this together, and take too. */
+template <int APPROX, int PREC, bool ENTRY, typename Take>
+__device__ __forceinline__ void window_lines_of(const KParams &kp, const GroupRay *g, WindowLine *lines,
+                                                uint32_t nw, const StagedEntry *eo, const StagedEntry *ei,
+                                                double f_o, double f_i, bool mine, Take take)
 {
     const mgx_model &m = kp.m;
     const uint32_t q = threadIdx.x & 31, grp = (threadIdx.x & (MGX_WAVE - 1)) >> 5;
@@ -367,7 +380,6 @@ __device__ __forceinline__ WindowSum window_sum(const KParams &kp, const GroupRa
        staged, and their point is not read */
     double ub = ei->ubm;
     if (ENTRY && any) ub = gld(&kp.pts[ei->nr].ub);
-    WindowSum r = {0.0, ENTRY ? kp.op.min_opacity : 0.0, 0.0};
     double left = -__builtin_inf(), right = __builtin_inf(); /* the bin's window */
     double left_all = left, right_all = right;               /* the group's */
     if (APPROX == MGX_APPROX_CLOSE_LINES) {
@@ -388,6 +400,7 @@ __device__ __forceinline__ WindowSum window_sum(const KParams &kp, const GroupRa
     for (uint32_t s0 = 0; s0 < m.nlines; s0 += nw) {
         bool in = false;
         double f = 0.0;
+        uint32_t l = 0;
         if (any && q < nw && s0 + q < m.nlines) {
             f = APPROX == MGX_APPROX_CLOSE_LINES ? gld(&m.sorted_line[s0 + q]) : gld(&m.line[s0 + q]);
             in = !(f < left_all) && !(right_all < f);
@@ -396,7 +409,7 @@ __device__ __forceinline__ WindowSum window_sum(const KParams &kp, const GroupRa
         if (b == 0) continue;
         __syncthreads();
         if (in) {
-            const uint32_t l = APPROX == MGX_APPROX_CLOSE_LINES ? gld(&m.sorted_line_map[s0 + q]) : s0 + q;
+            l = APPROX == MGX_APPROX_CLOSE_LINES ? gld(&m.sorted_line_map[s0 + q]) : s0 + q;
             WindowLine w;
             w.f = f;
             line_at<PREC, ENTRY>(kp, ENTRY ? ei : eo, l, w.iw_o, w.kap_o, w.src_o);
@@ -405,29 +418,46 @@ __device__ __forceinline__ WindowSum window_sum(const KParams &kp, const GroupRa
             } else {
                 line_at<PREC, false>(kp, ei, l, w.iw_i, w.kap_i, w.src_i);
             }
-            w.pad = 0.0;
+            w.l = l;
             lines[q] = w;
         }
         __syncthreads();
-        uint32_t set = (uint32_t)(b >> (32 * grp));
-        while (set) {
-            const WindowLine *w = lines + (__ffs((int)set) - 1);
-            set &= set - 1;
-            if (!mine || w->f < left || right < w->f) continue;
+        /* both groups' lines in turn, so that the lanes of the wave stay together */
+        const uint32_t set = (uint32_t)(b >> (32 * grp));
+        uint32_t all = (uint32_t)b | (uint32_t)(b >> 32);
+        while (all) {
+            const uint32_t i = (uint32_t)__ffs((int)all) - 1;
+            all &= all - 1;
+            const WindowLine *w = lines + i;
+            const bool here = mine && ((set >> i) & 1) != 0 && !(w->f < left) && !(right < w->f);
+            take(w, w->l, here);
+        }
+    }
+    __syncthreads();
+}
+
+template <int APPROX, int PREC, bool ENTRY>
+__device__ __forceinline__ WindowSum window_sum(const KParams &kp, const GroupRay *g, WindowLine *lines,
+                                                uint32_t nw, const StagedEntry *eo, const StagedEntry *ei,
+                                                double f_o, double f_i, bool mine)
+{
+    WindowSum r = {0.0, ENTRY ? kp.op.min_opacity : 0.0, 0.0};
+    window_lines_of<APPROX, PREC, ENTRY>(
+        kp, g, lines, nw, eo, ei, f_o, f_i, mine, [&](const WindowLine *w, uint32_t, bool in) {
+            if (!in) return;
             if (ENTRY) {
                 const double prof = gaussian<PREC>(w->iw_o, f_i - w->f);
                 r.a += prof * w->src_o;
                 r.b += prof * w->kap_o;
             } else {
+                double dop;
                 const double d = line_depth<PREC>(w->iw_o, w->iw_i, w->kap_o, w->kap_i, f_o, f_i, w->f, ei->dz,
-                                                  kp.op.min_opacity);
+                                                  kp.op.min_opacity, dop);
                 r.a += d;
                 r.b = fma(d, w->src_o, r.b);
                 r.c = fma(d, w->src_i, r.c);
             }
-        }
-    }
-    __syncthreads();
+        });
     return r;
 }
 
@@ -478,13 +508,16 @@ __device__ __forceinline__ void staged_eta_chi(const KParams &kp, const GroupRay
  * solver.tpp:2140-2186).  Its value does not depend on which end is the current one.
  * ec_out / ec_in cache the ends' emissivity and opacity (ec_out from the segment
  * before, when that took the trapezoid rule too).  All lanes of the wave call this
- * together; those without a segment pass on = false.
+ * together; those without a segment pass on = false.  dop is d depth / d mean opacity of a
+ * segment with the own line alone, its lowest bit set when the depth was clamped (for the
+ * adjoint's tape; it costs the other sweeps nothing).
  */
 template <int APPROX, int PREC>
 __device__ __forceinline__ void staged_segment(const KParams &kp, const GroupRay *g, WindowLine *lines, uint32_t nw,
                                                const BinLine &bin, const StagedEntry *eo,
                                                const StagedEntry *ei, bool on, OuterEnd &out, PointEC &ec_out,
-                                               PointEC &ec_in, double &dtau, double &S_out, double &S_in)
+                                               PointEC &ec_in, double &dtau, double &S_out, double &S_in,
+                                               double &dop)
 {
     const uint32_t kind = ei->kind;
     const double dz = ei->dz;
@@ -496,14 +529,15 @@ __device__ __forceinline__ void staged_segment(const KParams &kp, const GroupRay
     const double bound = kp.op.min_opacity * dz;
     uint32_t seg = on ? kind & SEG_MASK : SEG_EMPTY;
     dtau = bound;
-    S_out = S_in = 0.0;
+    dop = S_out = S_in = 0.0;
     if (seg == SEG_LANE) {
         const uint32_t w = lane_window<APPROX>(kp, g->ol, out.f, in.f, ei->ubm);
         seg = w == 1 ? SEG_SOLO : (w == 0 && bound > 0.0) ? SEG_EMPTY : SEG_LANE;
     }
     if (seg == SEG_SOLO) {
         const double d = line_depth<PREC>(out.iw, in.iw, out.kap, in.kap, out.f, in.f, bin.a_g, dz,
-                                          kp.op.min_opacity);
+                                          kp.op.min_opacity, dop);
+        uint64_t bits = __builtin_bit_cast(uint64_t, dop) & ~1ull;
         S_out = out.src;
         S_in = in.src;
         dtau = d;
@@ -513,7 +547,9 @@ __device__ __forceinline__ void staged_segment(const KParams &kp, const GroupRay
             dtau = bound;
             S_out *= share;
             S_in *= share;
+            bits |= 1;
         }
+        dop = __builtin_bit_cast(double, bits);
     }
     if (__ballot(seg >= SEG_LANE)) {
         if (__ballot(seg == SEG_LANE)) {
