@@ -62,11 +62,38 @@ constexpr int NL_RED_THREADS = 256;
 constexpr int NL_GRAM_BLOCKS = 512;
 
 /* device tables */
+
+/* One transition in a level's list: its index, and in at the level's place in it (1 the
+   upper, 2 the lower level, 3 both) and the other level (at = place | other << 2). */
+struct LevelRef {
+    uint32_t k, at;
+};
+
 struct NCol {
     uint32_t num, op, ntmp, ncol;
     const uint32_t *icol, *jcol;
     const double *tmp, *Cd, *Ce;
+    const uint32_t *start; /* (nlev + 1): level i's transitions are refs[start[i]] .. */
+    const LevelRef *refs;  /* in the order of the transitions */
 };
+
+/* global-address-space load (pointers read from the tables would give flat loads, which
+   wait for LDS too) */
+template <typename T>
+__device__ __forceinline__ T gl(const T *p)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return *(const __attribute__((address_space(1))) T *)p;
+#else
+    return *p;
+#endif
+}
+
+__device__ __forceinline__ LevelRef gl_ref(const LevelRef *p)
+{
+    const uint64_t v = gl(reinterpret_cast<const uint64_t *>(p));
+    return LevelRef{(uint32_t)v, (uint32_t)(v >> 32)};
+}
 
 struct NSpec {
     uint32_t num, nlev, nrad, lid0;
@@ -74,6 +101,8 @@ struct NSpec {
     uint64_t pop_off;
     const double *energy, *weight, *A, *Bs, *Ba, *freq;
     const uint32_t *irad, *jrad;
+    const uint32_t *rstart; /* the levels' radiative transitions, as NCol's */
+    const LevelRef *rrefs;
 };
 
 /* kernel arguments shared by the per-point kernels */
@@ -91,14 +120,14 @@ struct NView {
 
 __device__ inline double line_emissivity(const NSpec &S, uint32_t k, double ni, double mn)
 {
-    const double e = S.freq[k] * MGX_HH_OVER_FOUR_PI * S.A[k] * ni;
+    const double e = gl(&S.freq[k]) * MGX_HH_OVER_FOUR_PI * gl(&S.A[k]) * ni;
     return e > mn ? e : mn;
 }
 
 __device__ inline double line_opacity(const NSpec &S, uint32_t k, double ni, double nj,
                                       double mn)
 {
-    const double o = S.freq[k] * MGX_HH_OVER_FOUR_PI * (nj * S.Ba[k] - ni * S.Bs[k]);
+    const double o = gl(&S.freq[k]) * MGX_HH_OVER_FOUR_PI * (nj * gl(&S.Ba[k]) - ni * gl(&S.Bs[k]));
     return o > mn ? o : mn;
 }
 
@@ -117,18 +146,41 @@ __device__ inline uint32_t search_tmp(const double *x, uint32_t n, double v)
     return stop;
 }
 
-/* wave-uniform argmax of val with the smallest lane winning ties */
-__device__ inline int wave_argmax(double val, int idx)
+template <int CTRL>
+__device__ __forceinline__ double max_dpp(double v)
 {
-    for (int o = 32; o > 0; o >>= 1) {
-        const double ov = __shfl_xor(val, o);
-        const int oi = __shfl_xor(idx, o);
-        if (ov > val || (ov == val && oi < idx)) {
-            val = ov;
-            idx = oi;
-        }
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint64_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, false);
+    const uint64_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, false);
+    const double o = __builtin_bit_cast(double, (hi << 32) | lo);
+    return o > v ? o : v;
+}
+
+__device__ __forceinline__ double lane_value(double v, int l)
+{
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, l);
+    const uint64_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), l);
+    return __builtin_bit_cast(double, (hi << 32) | lo);
+}
+
+/* the lane of the largest val (no NaN), the smallest one of several: the maximum of each row
+   of 16 by DPP (lane ^ 1, ^ 2, the half-row's and the row's mirror image), the rows' from
+   their first lanes */
+__device__ inline int wave_argmax(double val)
+{
+    double m = max_dpp<0xb1>(val);
+    m = max_dpp<0x4e>(m);
+    m = max_dpp<0x141>(m);
+    m = max_dpp<0x140>(m);
+    double t = lane_value(m, 0);
+#pragma unroll
+    for (int r = 16; r < NL_WAVE; r += 16) {
+        const double o = lane_value(m, r);
+        t = o > t ? o : t;
     }
-    return __shfl(idx, 0);
+    const unsigned long long b = __ballot(val == t);
+    return b ? (int)__ffsll((long long)b) - 1 : 0;
 }
 
 __device__ inline int lane_of_step(int my_step, int c)
@@ -172,8 +224,8 @@ __device__ double finish_point(const NView &v, const NSpec &S, uint32_t p, uint3
     __syncthreads();
     bool any = false;
     for (uint32_t k = lane; k < S.nrad; k += NL_WAVE) {
-        const double ni = pv[S.irad[k]], nj = pv[S.jrad[k]];
-        any = any || (nj < S.Bs[k] / S.Ba[k] * ni * v.inv_frac);
+        const double ni = pv[gl(&S.irad[k])], nj = pv[gl(&S.jrad[k])];
+        any = any || (nj < gl(&S.Bs[k]) / gl(&S.Ba[k]) * ni * v.inv_frac);
     }
     if (__ballot(any)) {
         if (lane == 0) {
@@ -247,7 +299,7 @@ __device__ double finish_point(const NView &v, const NSpec &S, uint32_t p, uint3
     if (lane < n) pv[lane] = x;
     __syncthreads();
     for (uint32_t k = lane; k < S.nrad; k += NL_WAVE) {
-        const double ni = pv[S.irad[k]], nj = pv[S.jrad[k]];
+        const double ni = pv[gl(&S.irad[k])], nj = pv[gl(&S.jrad[k])];
         const size_t idx = (size_t)p * v.L + S.lid0 + k;
         const double o = line_opacity(S, k, ni, nj, v.min_o);
         eps[idx] = line_emissivity(S, k, ni, v.min_e);
@@ -268,10 +320,10 @@ __device__ inline void two_sum(double a, double b, double &s, double &e)
     e = (a - (s - bb)) + (b - bb);
 }
 
-/* LDS per wave (doubles): A0[n n], LU[n n], xs[n], jeff[maxnrad], kold[maxnrad], pv[2 n] */
+/* LDS per wave (doubles): A0[n n], jeff[maxnrad], kold[maxnrad], pv[2 n] */
 __host__ __device__ inline size_t stateq_lds_doubles(uint32_t n, uint32_t maxnrad)
 {
-    return 2 * (size_t)n * n + n + 2 * (size_t)maxnrad + 2 * (size_t)n;
+    return (size_t)n * n + 2 * (size_t)maxnrad + 2 * (size_t)n;
 }
 
 /*
@@ -291,7 +343,18 @@ struct GlobalIn {
     unsigned long long *dmax;   /* largest |x_out - x_it| / n_tot (bits of a positive double) */
 };
 
-template <bool GLOBAL>
+/*
+ * One wave per (point, species), a row of the rate matrix per lane.  What bounds it is
+ * latency -- the chain of pivot steps and substitutions of one small system -- and how many
+ * such chains a CU holds.  The rows live in registers (NMAX columns, turned by one at every
+ * step so that the code names fixed registers), the pivot row reaches the other lanes through
+ * scalar registers instead of LDS reads, and LDS keeps only the matrix itself for the residuals.
+ * Each level's transitions come from its own list, four gathers at a time, instead of every
+ * lane looking through all of them.  5832 points x 41 levels: 2.77 ms before (two matrices
+ * in LDS, five waves per CU, 820 transitions looked through by every lane), 0.39 ms now; the
+ * same results to the last bit.
+ */
+template <bool GLOBAL, int NMAX>
 __global__ __launch_bounds__(NL_WAVE) void stateq_kernel(NView v, const double *__restrict__ J,
                                                          const double *__restrict__ lam,
                                                          const double *__restrict__ old_all,
@@ -306,9 +369,7 @@ __global__ __launch_bounds__(NL_WAVE) void stateq_kernel(NView v, const double *
     const NSpec S = v.spec[s];
     const uint32_t n = S.nlev, nrad = S.nrad;
     double *A0 = sm;
-    double *LU = A0 + (size_t)n * n;
-    double *xs = LU + (size_t)n * n;
-    double *jeff = xs + n;
+    double *jeff = A0 + (size_t)n * n;
     double *kold = jeff + v.maxnrad;
     double *pv = kold + v.maxnrad;
     const double *old = old_all + S.pop_off + (size_t)p * n;
@@ -321,8 +382,10 @@ __global__ __launch_bounds__(NL_WAVE) void stateq_kernel(NView v, const double *
         const double *Jp = J + (size_t)p * v.F + (size_t)lid * v.Q;
         const double *w = v.quad_weights + (size_t)s * v.Q;
         double jl = 0.0;
-        for (uint32_t z = 0; z < v.Q; z++) jl += w[z] * Jp[z];
-        const double ni = old[S.irad[k]], nj = old[S.jrad[k]];
+        #pragma unroll 8
+        for (uint32_t z = 0; z < v.Q; z++) jl += gl(&w[z]) * gl(&Jp[z]);
+        const uint32_t iu = gl(&S.irad[k]);
+        const double ni = gl(&old[iu]), nj = gl(&old[gl(&S.jrad[k])]);
         double diff;
         if constexpr (GLOBAL) {
             /* Model::compute_Jeff (model.cpp:514-545): the list's elements times the upper
@@ -331,7 +394,7 @@ __global__ __launch_bounds__(NL_WAVE) void stateq_kernel(NView v, const double *
             diff = 0.0;
             for (uint32_t m = 0; m < g.count[pl]; m++) {
                 const uint32_t q = g.nr[pl * g.cap + m];
-                diff += g.val[pl * g.cap + m] * old_all[S.pop_off + (size_t)q * n + S.irad[k]];
+                diff += g.val[pl * g.cap + m] * old_all[S.pop_off + (size_t)q * n + iu];
             }
         } else {
             diff = lam[(size_t)p * v.L + lid] * ni;
@@ -349,22 +412,25 @@ __global__ __launch_bounds__(NL_WAVE) void stateq_kernel(NView v, const double *
     const uint32_t r = lane;
     double yoff = 0.0; /* right-hand side of row r from other points (global mode) */
     if (r < n) {
-        for (uint32_t k = 0; k < nrad; k++) {
-            const uint32_t I = S.irad[k], Jl = S.jrad[k];
+        const uint32_t e0 = gl(&S.rstart[r]), e1 = gl(&S.rstart[r + 1]);
+        for (uint32_t e = e0; e < e1; e++) {
+            const LevelRef ref = gl_ref(&S.rrefs[e]);
+            const uint32_t k = ref.k, other = ref.at >> 2;
             const double je = jeff[k];
-            const double v_IJ = S.A[k] + S.Bs[k] * je;
-            const double v_JI = S.Ba[k] * je;
-            if (r == Jl) {
-                A0[(size_t)I * n + r] += v_IJ;
-                A0[(size_t)Jl * n + r] -= v_JI;
+            const double v_IJ = gl(&S.A[k]) + gl(&S.Bs[k]) * je;
+            const double v_JI = gl(&S.Ba[k]) * je;
+            if (ref.at & 2) {
+                A0[(size_t)other * n + r] += v_IJ;
+                A0[(size_t)r * n + r] -= v_JI;
             }
-            if (r == I) {
-                A0[(size_t)Jl * n + r] += v_JI;
-                A0[(size_t)I * n + r] -= v_IJ;
+            if (ref.at & 1) {
+                A0[(size_t)other * n + r] += v_JI;
+                A0[(size_t)r * n + r] -= v_IJ;
             }
         }
-        for (uint32_t k = 0; k < nrad; k++) {
-            const uint32_t I = S.irad[k], Jl = S.jrad[k];
+        for (uint32_t e = e0; e < e1; e++) {
+            const LevelRef ref = gl_ref(&S.rrefs[e]);
+            const uint32_t k = ref.k, other = ref.at >> 2;
             if constexpr (GLOBAL) {
                 /* elements at this point stay in the block; one at another point q couples
                    row (p, lower) to that point's upper level: moved to the right-hand side
@@ -372,18 +438,18 @@ __global__ __launch_bounds__(NL_WAVE) void stateq_kernel(NView v, const double *
                 const size_t pl = (size_t)p * v.L + S.lid0 + k;
                 for (uint32_t m = 0; m < g.count[pl]; m++) {
                     const uint32_t q = g.nr[pl * g.cap + m];
-                    const double v_IJ = -g.val[pl * g.cap + m] * kold[k] / S.freq[k];
+                    const double v_IJ = -g.val[pl * g.cap + m] * kold[k] / gl(&S.freq[k]);
                     if (q == p) {
-                        if (r == Jl) A0[(size_t)I * n + r] += v_IJ;
-                        if (r == I) A0[(size_t)I * n + r] -= v_IJ;
-                    } else if (r == Jl) {
-                        yoff -= v_IJ * g.x_it[S.pop_off + (size_t)q * n + I];
+                        if (ref.at & 2) A0[(size_t)other * n + r] += v_IJ;
+                        if (ref.at & 1) A0[(size_t)r * n + r] -= v_IJ;
+                    } else if (ref.at & 2) {
+                        yoff -= v_IJ * g.x_it[S.pop_off + (size_t)q * n + other];
                     }
                 }
             } else {
-                const double v_IJ = -lam[(size_t)p * v.L + S.lid0 + k] * kold[k] / S.freq[k];
-                if (r == Jl) A0[(size_t)I * n + r] += v_IJ;
-                if (r == I) A0[(size_t)I * n + r] -= v_IJ;
+                const double v_IJ = -gl(&lam[(size_t)p * v.L + S.lid0 + k]) * kold[k] / gl(&S.freq[k]);
+                if (ref.at & 2) A0[(size_t)other * n + r] += v_IJ;
+                if (ref.at & 1) A0[(size_t)r * n + r] -= v_IJ;
             }
         }
         if constexpr (GLOBAL) A0[(size_t)r * n + r] += g.dextra[S.pop_off + (size_t)p * n + r];
@@ -401,19 +467,33 @@ __global__ __launch_bounds__(NL_WAVE) void stateq_kernel(NView v, const double *
             const double step = edge ? 0.0 : (T - C.tmp[t - 1]) / (C.tmp[t] - C.tmp[t - 1]);
             const double *Cd1 = C.Cd + (size_t)t * C.ncol, *Ce1 = C.Ce + (size_t)t * C.ncol;
             const double *Cd0 = edge ? Cd1 : Cd1 - C.ncol, *Ce0 = edge ? Ce1 : Ce1 - C.ncol;
-            for (uint32_t k = 0; k < C.ncol; k++) {
-                const uint32_t I = C.icol[k], Jl = C.jcol[k];
-                if (r != I && r != Jl) continue;
-                const double cd = edge ? Cd1[k] : Cd0[k] + (Cd1[k] - Cd0[k]) * step;
-                const double ce = edge ? Ce1[k] : Ce0[k] + (Ce1[k] - Ce0[k]) * step;
-                const double v_IJ = cd * abn, v_JI = ce * abn;
-                if (r == Jl) {
-                    A0[(size_t)I * n + r] += v_IJ;
-                    A0[(size_t)Jl * n + r] -= v_JI;
+            /* four transitions of the level at a time, their gathers together */
+            const uint32_t c0 = gl(&C.start[r]), c1 = gl(&C.start[r + 1]);
+            for (uint32_t e = c0; e < c1; e += 4) {
+                LevelRef ref[4];
+                double cd[4], ce[4];
+#pragma unroll
+                for (uint32_t i = 0; i < 4; i++) ref[i] = gl_ref(&C.refs[e + i < c1 ? e + i : c1 - 1]);
+#pragma unroll
+                for (uint32_t i = 0; i < 4; i++) {
+                    const uint32_t k = ref[i].k;
+                    const double d1 = gl(&Cd1[k]), u1 = gl(&Ce1[k]), d0 = gl(&Cd0[k]), u0 = gl(&Ce0[k]);
+                    cd[i] = edge ? d1 : d0 + (d1 - d0) * step;
+                    ce[i] = edge ? u1 : u0 + (u1 - u0) * step;
                 }
-                if (r == I) {
-                    A0[(size_t)Jl * n + r] += v_JI;
-                    A0[(size_t)I * n + r] -= v_IJ;
+#pragma unroll
+                for (uint32_t i = 0; i < 4; i++) {
+                    if (e + i >= c1) break;
+                    const uint32_t other = ref[i].at >> 2;
+                    const double v_IJ = cd[i] * abn, v_JI = ce[i] * abn;
+                    if (ref[i].at & 2) {
+                        A0[(size_t)other * n + r] += v_IJ;
+                        A0[(size_t)r * n + r] -= v_JI;
+                    }
+                    if (ref[i].at & 1) {
+                        A0[(size_t)other * n + r] += v_JI;
+                        A0[(size_t)r * n + r] -= v_IJ;
+                    }
                 }
             }
         }
@@ -421,74 +501,94 @@ __global__ __launch_bounds__(NL_WAVE) void stateq_kernel(NView v, const double *
             for (uint32_t c = 0; c < n; c++) A0[(size_t)c * n + r] = 1.0;
     }
     __syncthreads();
-    for (uint32_t i = lane; i < n * n; i += NL_WAVE) LU[i] = A0[i];
+    /* lane r's row, in registers; columns past n are zero */
+    double row[NMAX];
+#pragma unroll
+    for (int j = 0; j < NMAX; j++) row[j] = (r < n && (uint32_t)j < n) ? A0[(size_t)j * n + r] : 0.0;
     const double y0 = (r == n - 1) ? ptot : yoff;
     double yv = y0;
-    __syncthreads();
 
     /* Gaussian elimination with partial pivoting; my_step = the column this
-       lane's row became the pivot of (n while not yet) */
+       lane's row became the pivot of (n while not yet).  Every step works on the first
+       register and turns the row by one, the multiplier taking the place of the column
+       that is done: after NMAX turns register j holds the multiplier of step j, or from the
+       lane's own step on its row of U.  A pivot row reaches the other lanes through scalar
+       registers. */
     int my_step = (int)n;
-    for (uint32_t c = 0; c < n; c++) {
-        double val = (r < n && my_step == (int)n) ? fabs(LU[(size_t)c * n + r]) : -1.0;
-        if (val != val) val = 0.0; /* a NaN row is picked only when nothing else is left */
-        const int pr = wave_argmax(val, (int)lane);
-        if ((int)lane == pr) my_step = (int)c;
-        const double pivot = LU[(size_t)c * n + pr];
-        const double ypiv = __shfl(yv, pr);
-        if (r < n && my_step > (int)c) {
-            const double f = pivot != 0.0 ? LU[(size_t)c * n + r] / pivot : 0.0;
-            LU[(size_t)c * n + r] = f;
-            for (uint32_t j = c + 1; j < n; j++)
-                LU[(size_t)j * n + r] = fma(-f, LU[(size_t)j * n + pr], LU[(size_t)j * n + r]);
-            yv = fma(-f, ypiv, yv);
-        }
-        __syncthreads();
-    }
-    /* back substitution by columns; lane c ends with x_c */
-    double x = 0.0;
-    for (int c = (int)n - 1; c >= 0; c--) {
-        const int pr = lane_of_step(my_step, c);
-        const double d = LU[(size_t)c * n + pr];
-        double xc = ((int)lane == pr && d != 0.0) ? yv / d : 0.0;
-        xc = __shfl(xc, pr);
-        if ((int)lane == c) x = xc;
-        if (r < n && my_step < c) yv = fma(-LU[(size_t)c * n + r], xc, yv);
-    }
-    /* iterative refinement with compensated residuals */
-    for (int it = 0; it < 2; it++) {
-        if (r < n) xs[r] = x;
-        __syncthreads();
-        double res = 0.0;
-        if (r < n) {
-            double hi = y0, lo = 0.0;
-            for (uint32_t j = 0; j < n; j++) {
-                const double a = A0[(size_t)j * n + r], b = xs[j];
-                const double pr_ = a * b;
-                const double pe = fma(a, b, -pr_);
-                double s_, e_;
-                two_sum(hi, -pr_, s_, e_);
-                hi = s_;
-                lo += e_ - pe;
+    double diag = 1.0; /* the pivot of the lane's own step */
+#pragma unroll 1
+    for (uint32_t c = 0; c < (uint32_t)NMAX; c++) {
+        double f = 0.0, keep = row[0];
+        int pr = 0;
+        if (c < n) {
+            double val = (r < n && my_step == (int)n) ? fabs(row[0]) : -1.0;
+            if (val != val) val = 0.0; /* a NaN row is picked only when nothing else is left */
+            pr = wave_argmax(val);
+            if ((int)lane == pr) {
+                my_step = (int)c;
+                diag = row[0];
             }
-            res = hi + lo;
+            const double pivot = lane_value(row[0], pr);
+            const double ypiv = lane_value(yv, pr);
+            if (r < n && my_step > (int)c) {
+                f = pivot != 0.0 ? row[0] / pivot : 0.0;
+                keep = f;
+                yv = fma(-f, ypiv, yv);
+            }
         }
-        __syncthreads();
-        for (uint32_t c = 0; c < n; c++) {
-            const int pr = lane_of_step(my_step, (int)c);
-            const double dp = __shfl(res, pr);
-            if (r < n && my_step > (int)c) res = fma(-LU[(size_t)c * n + r], dp, res);
+#pragma unroll
+        for (int j = 1; j < NMAX; j++) {
+            /* registers from NMAX - c on hold the multipliers of the steps done */
+            const double u = (uint32_t)j < (uint32_t)NMAX - c ? lane_value(row[j], pr) : 0.0;
+            row[j - 1] = fma(-f, u, row[j]);
+            /* a few pivot entries in scalar registers at a time */
+            if (j % 8 == 0) __builtin_amdgcn_sched_barrier(0);
         }
-        double dx = 0.0;
-        for (int c = (int)n - 1; c >= 0; c--) {
+        row[NMAX - 1] = keep;
+    }
+    const double rdiag = 1.0 / diag;
+    /* U x = b by columns from the last: lane c's x_c */
+    const auto back = [&](double b) {
+        double x = 0.0;
+#pragma unroll
+        for (int c = NMAX - 1; c >= 0; c--) {
+            if ((uint32_t)c >= n) continue;
             const int pr = lane_of_step(my_step, c);
-            const double d = LU[(size_t)c * n + pr];
-            double xc = ((int)lane == pr && d != 0.0) ? res / d : 0.0;
-            xc = __shfl(xc, pr);
-            if ((int)lane == c) dx = xc;
-            if (r < n && my_step < c) res = fma(-LU[(size_t)c * n + r], xc, res);
+            /* b / diag to the last bit: the quotient and one correction */
+            double q = b * rdiag;
+            q = fma(fma(-q, diag, b), rdiag, q);
+            if (diag == 0.0) q = 0.0;
+            const double xc = lane_value(q, pr);
+            if ((int)lane == c) x = xc;
+            if (r < n && my_step < c) b = fma(-row[c], xc, b);
+            if (c % 8 == 0) __builtin_amdgcn_sched_barrier(0);
         }
-        x += dx;
+        return x;
+    };
+    double x = back(yv);
+    /* iterative refinement with compensated residuals */
+#pragma unroll 1
+    for (int it = 0; it < 2; it++) {
+        double hi = y0, lo = 0.0;
+#pragma unroll 8
+        for (uint32_t j = 0; j < n; j++) {
+            const double a = r < n ? A0[(size_t)j * n + r] : 0.0, b = lane_value(x, (int)j);
+            const double pr_ = a * b;
+            const double pe = fma(a, b, -pr_);
+            double s_, e_;
+            two_sum(hi, -pr_, s_, e_);
+            hi = s_;
+            lo += e_ - pe;
+        }
+        double res = hi + lo;
+#pragma unroll
+        for (int c = 0; c < NMAX; c++) {
+            if ((uint32_t)c >= n) continue;
+            const double dp = lane_value(res, lane_of_step(my_step, c));
+            if (r < n && my_step > c) res = fma(-row[c], dp, res);
+            if (c % 8 == 0) __builtin_amdgcn_sched_barrier(0);
+        }
+        x += back(res);
     }
     __syncthreads();
     if constexpr (GLOBAL) {
@@ -1025,6 +1125,29 @@ std::vector<const double *> history_ptrs(const mgx_nlte *h)
     return v;
 }
 
+/* stateq_kernel with rows of 8, 16, 32, 48 or 64 registers, the fewest that hold the
+   species' levels: a row's registers bound the waves that are resident (41 levels: 48, three
+   waves per SIMD), and every step works on all of them */
+template <bool GLOBAL, int NMAX, typename... Args>
+int launch_stateq_n(mgx_nlte *h, size_t lds, hipStream_t st, Args... args)
+{
+    if (int e = set_lds_limit((const void *)stateq_kernel<GLOBAL, NMAX>, lds)) return e;
+    hipLaunchKernelGGL((stateq_kernel<GLOBAL, NMAX>), dim3(h->P, h->nlspecs), dim3(NL_WAVE), lds, st,
+                       make_view(h), args...);
+    NL_TRY(hipGetLastError());
+    return MGX_OK;
+}
+
+template <bool GLOBAL, typename... Args>
+int launch_stateq(mgx_nlte *h, size_t lds, hipStream_t st, Args... args)
+{
+    if (h->maxnlev <= 8) return launch_stateq_n<GLOBAL, 8>(h, lds, st, args...);
+    if (h->maxnlev <= 16) return launch_stateq_n<GLOBAL, 16>(h, lds, st, args...);
+    if (h->maxnlev <= 32) return launch_stateq_n<GLOBAL, 32>(h, lds, st, args...);
+    if (h->maxnlev <= 48) return launch_stateq_n<GLOBAL, 48>(h, lds, st, args...);
+    return launch_stateq_n<GLOBAL, 64>(h, lds, st, args...);
+}
+
 int launch_finish(mgx_nlte *h, const double *old, double *eps, double *kap, double *ic,
                   hipStream_t st)
 {
@@ -1195,6 +1318,24 @@ int mgx_nlte_create(const mgx_model *m, uint32_t nlspecs, const mgx_linedata *ld
         rel.push_back({base + offsetof(NSpec, freq), put(d.frequency, 8 * (size_t)d.nrad)});
         rel.push_back({base + offsetof(NSpec, irad), put(d.irad, 4 * (size_t)d.nrad)});
         rel.push_back({base + offsetof(NSpec, jrad), put(d.jrad, 4 * (size_t)d.nrad)});
+        /* the transitions of every level, in their order */
+        const auto put_refs = [&](uint32_t n, const uint32_t *iu, const uint32_t *jl, size_t start_field,
+                                  size_t refs_field) {
+            std::vector<uint32_t> start(d.nlev + 1, 0);
+            std::vector<LevelRef> refs;
+            for (uint32_t lev = 0; lev < d.nlev; lev++) {
+                for (uint32_t k = 0; k < n; k++) {
+                    if (iu[k] != lev && jl[k] != lev) continue;
+                    const uint32_t place = (iu[k] == lev ? 1u : 0u) | (jl[k] == lev ? 2u : 0u);
+                    refs.push_back(LevelRef{k, place | (iu[k] == lev ? jl[k] : iu[k]) << 2});
+                }
+                start[lev + 1] = (uint32_t)refs.size();
+            }
+            if (refs.empty()) refs.push_back(LevelRef{0, 0});
+            rel.push_back({start_field, put(start.data(), 4 * start.size())});
+            rel.push_back({refs_field, put(refs.data(), sizeof(LevelRef) * refs.size())});
+        };
+        put_refs(d.nrad, d.irad, d.jrad, base + offsetof(NSpec, rstart), base + offsetof(NSpec, rrefs));
         for (uint32_t c = 0; c < S.ncolpar; c++, c0++) {
             const mgx_colldata &C = colpar[c0];
             NCol &Cc = cp[c0];
@@ -1208,6 +1349,7 @@ int mgx_nlte_create(const mgx_model *m, uint32_t nlspecs, const mgx_linedata *ld
             rel.push_back({cb + offsetof(NCol, tmp), put(C.tmp, 8 * (size_t)C.ntmp)});
             rel.push_back({cb + offsetof(NCol, Cd), put(C.Cd, 8 * (size_t)C.ntmp * C.ncol)});
             rel.push_back({cb + offsetof(NCol, Ce), put(C.Ce, 8 * (size_t)C.ntmp * C.ncol)});
+            put_refs(C.ncol, C.icol, C.jcol, cb + offsetof(NCol, start), cb + offsetof(NCol, refs));
         }
     }
     h->nvec = off;
@@ -1318,11 +1460,9 @@ int mgx_nlte_iteration_stateq(mgx_nlte *h, const double *J, const double *lam, d
     if (int e = push_history(h, st)) return e;
     const double *old = h->ring[h->hist.back()];
     const size_t lds = point_lds(h, true);
-    if (int e = set_lds_limit((const void *)stateq_kernel<false>, lds)) return e;
-    hipLaunchKernelGGL(stateq_kernel<false>, dim3(h->P, h->nlspecs), dim3(NL_WAVE), lds, st,
-                       make_view(h), J, lam, old, h->cur, eps, kap, ic, Jlin, Jeff, h->part,
-                       GlobalIn{});
-    NL_TRY(hipGetLastError());
+    if (int e = launch_stateq<false>(h, lds, st, J, lam, old, h->cur, eps, kap, ic, Jlin, Jeff, h->part,
+                                     GlobalIn{}))
+        return e;
     if (int e = collect_conv(h, st)) return e;
     if (conv) std::memcpy(conv, h->conv.data(), sizeof(mgx_nlte_conv) * h->nlspecs);
     return MGX_OK;
@@ -1352,7 +1492,6 @@ int mgx_nlte_iteration_stateq_global(mgx_nlte *h, const double *J, uint32_t cap,
                        make_view(h), g, old, dx);
     NL_TRY(hipGetLastError());
     const size_t lds = point_lds(h, true);
-    if (int e = set_lds_limit((const void *)stateq_kernel<true>, lds)) return e;
     /* block-Jacobi sweeps until the largest change is at the rounding level of the point
        solves (below 1e-15 of the point's total, or no longer decreasing) */
     double prev = __builtin_inf();
@@ -1362,10 +1501,10 @@ int mgx_nlte_iteration_stateq_global(mgx_nlte *h, const double *J, uint32_t cap,
         g.x_it = xa;
         g.x_out = xb;
         NL_TRY(hipMemsetAsync(dmax, 0, sizeof(unsigned long long), st));
-        hipLaunchKernelGGL(stateq_kernel<true>, dim3(h->P, h->nlspecs), dim3(NL_WAVE), lds, st,
-                           make_view(h), J, nullptr, old, h->cur, eps, kap, ic,
-                           it == 0 ? Jlin : nullptr, it == 0 ? Jeff : nullptr, h->part, g);
-        NL_TRY(hipGetLastError());
+        if (int e = launch_stateq<true>(h, lds, st, J, (const double *)nullptr, (const double *)old, h->cur, eps,
+                                        kap, ic, it == 0 ? Jlin : (double *)nullptr,
+                                        it == 0 ? Jeff : (double *)nullptr, h->part, g))
+            return e;
         unsigned long long bits = 0;
         NL_TRY(hipMemcpyAsync(&bits, dmax, sizeof bits, hipMemcpyDeviceToHost, st));
         NL_TRY(hipStreamSynchronize(st));
