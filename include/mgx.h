@@ -344,7 +344,11 @@ int mgx_image_adjoint_width_device(const mgx_model *model_dev, const mgx_options
                                    const double *I_bar, double *d_eps, double *d_kap,
                                    double *d_inverse_width, void *stream);
 
-/* Frees the adjoint's device workspace (it is re-allocated on the next call). */
+/*
+ * Frees the adjoint's device workspace and the buffers that the solves keep between
+ * calls (packed tables, and at most 2 GiB of parts of a solve whose ray pairs are split
+ * over waves); they are re-allocated on the next call.  Waits for a call in progress.
+ */
 void mgx_release_workspace(void);
 
 /* ------------------------------------------------------------------------ */

@@ -351,7 +351,7 @@ struct GlobalIn {
  * scalar registers instead of LDS reads, and LDS keeps only the matrix itself for the residuals.
  * Each level's transitions come from its own list, four gathers at a time, instead of every
  * lane looking through all of them.  5832 points x 41 levels: 2.77 ms before (two matrices
- * in LDS, five waves per CU, 820 transitions looked through by every lane), 0.39 ms now; the
+ * in LDS, five waves per CU, 820 transitions looked through by every lane), 0.42 ms now; the
  * same results to the last bit.
  */
 template <bool GLOBAL, int NMAX>

@@ -3395,10 +3395,18 @@ MGX_SHARED(size_t g_prep_bytes[64], = {});
 } // namespace mgx_shared
 namespace {
 
+/* How a solve's ray pairs are split over waves, see ray_split below. */
+struct RaySplit {
+    uint32_t per, groups; /* ray pairs per group, groups */
+    size_t J_bytes;       /* the ray pairs' parts of J (0: from u) and of Lambda */
+    size_t bytes;         /* all parts (0: not split) */
+};
+
 /* the tables of model m in b: from the call workspace, or (persistent, for objects
-   that keep them, such as a batch) in allocations of their own */
+   that keep them, such as a batch) in allocations of their own.  A split whose parts find
+   no memory is given up (sp says so): the unsplit solve gives the same results. */
 int prepare(const mgx_model *m, const mgx_options *op, hipStream_t st, DevBuffers &b, KParams &kp,
-            bool persistent = false, size_t parts_bytes = 0)
+            bool persistent = false, RaySplit *sp = nullptr)
 {
     const size_t P = m->npoints, PL = (size_t)m->npoints * m->nlines;
     if (persistent) {
@@ -3410,9 +3418,9 @@ int prepare(const mgx_model *m, const mgx_options *op, hipStream_t st, DevBuffer
         return prepare_tables(m, op, st, b, kp);
     }
     const auto rnd = [](size_t n) { return (n + 255) & ~(size_t)255; };
-    const size_t need = rnd(PL * sizeof(double4)) + rnd(P * sizeof(PointRec)) +
-                        rnd(P * sizeof(PointIdx)) + rnd(4 * sizeof(uint32_t)) +
-                        rnd(sizeof(KParams)) + rnd(sizeof(ImageFrame)) + rnd(parts_bytes);
+    size_t need = rnd(PL * sizeof(double4)) + rnd(P * sizeof(PointRec)) +
+                  rnd(P * sizeof(PointIdx)) + rnd(4 * sizeof(uint32_t)) +
+                  rnd(sizeof(KParams)) + rnd(sizeof(ImageFrame)) + rnd(sp ? sp->bytes : 0);
     b.ws_lock = std::unique_lock<std::mutex>(g_prep_mutex);
     int dev = 0;
     HIP_TRY(hipGetDevice(&dev));
@@ -3422,7 +3430,13 @@ int prepare(const mgx_model *m, const mgx_options *op, hipStream_t st, DevBuffer
         if (g_prep[dev]) (void)hipFree(g_prep[dev]);
         g_prep[dev] = nullptr;
         g_prep_bytes[dev] = 0;
-        HIP_TRY(hipMalloc(&g_prep[dev], need));
+        if (sp && sp->bytes > 0 && hipMalloc(&g_prep[dev], need) != hipSuccess) {
+            (void)hipGetLastError();
+            g_prep[dev] = nullptr;
+            need -= rnd(sp->bytes);
+            *sp = RaySplit{m->hnrays, 1, 0, 0};
+        }
+        if (!g_prep[dev]) HIP_TRY(hipMalloc(&g_prep[dev], need));
         g_prep_bytes[dev] = need;
     }
     unsigned char *q = g_prep[dev];
@@ -4227,20 +4241,17 @@ namespace {
 /*
  * How a solve splits the ray pairs of an origin over waves.  One wave per origin
  * leaves the GPU idle when there are few origins (3072 waves are resident at once) and
- * ends with a long tail when there are not many more; kSplitWaves waves fill it about
- * five times over.  Splitting costs the ray pairs' contributions of J (unless u is
- * stored) and Lambda a trip through memory of their own, at most kSplitBytes; the sums
- * are the same to the last bit.  Measured: 250 shells, 100 ray pairs 39.8 -> 9.2 ms;
- * 10^3 wind, 6 pairs, three solves 2.2 -> 0.9 ms; from 16384 origins on nothing is split.
+ * ends with a long tail when there are not many more, the longer the more work each has;
+ * kSplitWaves waves keep it full to the end.  Splitting costs the ray pairs' contributions
+ * of J (unless u is stored) and Lambda a trip through memory of their own, at most
+ * kSplitBytes; the sums are the same to the last bit.  Measured, unsplit and split:
+ * 250 shells, 100 ray pairs 39.8 and 9.2 ms; 10^3 wind, 6 pairs, three solves 2.2 and
+ * 0.9 ms; 19^3, 6 pairs, blended lines 11.6 and 10.4 ms; 18^3, 24 pairs, 40 lines 43.0 and
+ * 35.6 ms (1.4 GiB of parts; 37.7 with 16384 waves, 36.3 with 32768, 35.6 with 131072).
+ * At 32^3 origins two groups measured 13.44 ms against 13.45: no split from there on.
  */
-constexpr uint32_t kSplitWaves = 16384;
-constexpr size_t kSplitBytes = (size_t)256 << 20;
-
-struct RaySplit {
-    uint32_t per, groups; /* ray pairs per group, groups */
-    size_t J_bytes;       /* the ray pairs' parts of J (0: from u) and of Lambda */
-    size_t bytes;         /* all parts (0: not split) */
-};
+constexpr uint32_t kSplitWaves = 65536, kSplitOrigins = 32768;
+constexpr size_t kSplitBytes = (size_t)2 << 30;
 
 size_t noalloc_scratch_bytes(const mgx_model *model)
 {
@@ -4255,7 +4266,7 @@ RaySplit ray_split(const mgx_model &m, bool with_J, bool with_u, bool with_lam, 
     RaySplit r{m.hnrays, 1, 0, 0};
     const uint64_t P = m.npoints;
     const uint64_t g = (kSplitWaves + P - 1) / P;
-    if (g < 2 || m.hnrays < 2) return r;
+    if (P >= kSplitOrigins || m.hnrays < 2) return r;
     const size_t PR = (size_t)P * m.hnrays * sizeof(double);
     const size_t J_bytes = with_J && !with_u ? PR * m.nfreqs : 0;
     const size_t bytes = J_bytes + (with_lam ? PR * m.nlines : 0);
@@ -4361,8 +4372,8 @@ int mgx_feautrier_forward_device(const mgx_model *model, const mgx_options *opts
     hipStream_t st = (hipStream_t)stream;
     DevBuffers b;
     KParams kp;
-    const RaySplit sp = ray_split(*model, true, u != nullptr, lambda_diag != nullptr, kSplitBytes);
-    if (int e = prepare(model, opts, st, b, kp, false, sp.bytes)) return e;
+    RaySplit sp = ray_split(*model, true, u != nullptr, lambda_diag != nullptr, kSplitBytes);
+    if (int e = prepare(model, opts, st, b, kp, false, &sp)) return e;
     return forward_launch(model, opts, u, J, lambda_diag, st, b, kp, sp);
 }
 
@@ -4391,8 +4402,8 @@ int mgx_feautrier_sparse_device(const mgx_model *model, const mgx_options *opts,
     }
     DevBuffers b;
     KParams kp;
-    const RaySplit sp = ray_split(*model, true, false, lambda_diag != nullptr, kSplitBytes);
-    if (int e = prepare(model, opts, st, b, kp, false, sp.bytes)) return e;
+    RaySplit sp = ray_split(*model, true, false, lambda_diag != nullptr, kSplitBytes);
+    if (int e = prepare(model, opts, st, b, kp, false, &sp)) return e;
     /* J of an origin stays in LDS; when it does not fit (long walks), its row of a
        scratch J, allocated by the launch that needs it */
     double *Jtmp = nullptr;
@@ -4433,7 +4444,7 @@ int mgx_feautrier_forward_noalloc(const mgx_model *model, const mgx_options *opt
     b.pts = reinterpret_cast<PointRec *>(take(P * sizeof(PointRec)));
     b.pidx = reinterpret_cast<PointIdx *>(take(P * sizeof(PointIdx)));
     b.lpack = reinterpret_cast<double4 *>(take(PL * sizeof(double4)));
-    const RaySplit sp = ray_split(*model, true, u != nullptr, lambda_diag != nullptr,
+    RaySplit sp = ray_split(*model, true, u != nullptr, lambda_diag != nullptr,
                                   (size_t)MGX_NOALLOC_SCRATCH_BYTES - off);
     b.parts = reinterpret_cast<double *>(take(sp.bytes));
     struct NoEvents {
@@ -4509,8 +4520,8 @@ int mgx_shortchar_order_0_device(const mgx_model *model, const mgx_options *opts
     hipStream_t st = (hipStream_t)stream;
     DevBuffers b;
     KParams kp;
-    const RaySplit sp = ray_split(*model, true, u != nullptr, lambda_diag != nullptr, kSplitBytes);
-    if (int e = prepare(model, opts, st, b, kp, false, sp.bytes)) return e;
+    RaySplit sp = ray_split(*model, true, u != nullptr, lambda_diag != nullptr, kSplitBytes);
+    if (int e = prepare(model, opts, st, b, kp, false, &sp)) return e;
     const ShortcharOut sc{I, v, min_dtau};
     return launch_with_capacity(st, b, kp, [&](size_t) {
         const dim3 grid(model->npoints, sp.groups), block(MGX_WAVE);
@@ -4559,7 +4570,7 @@ int mgx_feautrier_order_2_uv_device(const mgx_model *model, const mgx_options *o
     DevBuffers b;
     KParams kp;
     if (int e = prepare(model, opts, st, b, kp)) return e;
-    const RaySplit sp = ray_split(*model, false, true, false, 0); /* u and v are per ray pair */
+    RaySplit sp = ray_split(*model, false, true, false, 0); /* u and v are per ray pair */
     return launch_with_capacity(st, b, kp, [&](size_t) {
         const dim3 grid(model->npoints, sp.groups), block(MGX_WAVE);
         const size_t lds = solve_lds_bytes(kp.cap, kp.stage, model->nfreqs, model->nlines, false);
@@ -4805,6 +4816,17 @@ void mgx_release_workspace(void)
     }
     g_ws = nullptr;
     g_ws_bytes = 0;
+    std::lock_guard<std::mutex> prep_lock(g_prep_mutex); /* no call holds the buffers */
+    int dev = 0;
+    const bool back = hipGetDevice(&dev) == hipSuccess;
+    for (int d = 0; d < 64; d++) {
+        if (!g_prep[d]) continue;
+        if (hipSetDevice(d) == hipSuccess) (void)hipDeviceSynchronize();
+        (void)hipFree(g_prep[d]);
+        g_prep[d] = nullptr;
+        g_prep_bytes[d] = 0;
+    }
+    if (back) (void)hipSetDevice(dev);
 }
 
 #endif /* MGX_ADJOINT_TU */

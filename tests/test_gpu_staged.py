@@ -52,3 +52,21 @@ def test_interpolated_entries_across_chunks():
     m.params["max_interpolation_diff"] = 1.02
     print("[staged] interpolated chunks", flush=True)
     _check(m, m.options())
+
+
+@pytest.mark.parametrize("nrays", [12, 48])
+def test_ray_pair_parts_and_their_workspace(nrays):
+    """J from the ray pairs' parts and from the stored u, and once more after the kept
+    buffers were given back: the same bits"""
+    from magritte_amd import solver
+
+    print(f"[staged] parts of {nrays} rays", flush=True)
+    m = models.model_wind(n_edge=6, nrays=nrays, nquads=7)
+    d, op = solver.DeviceModel(m), m.options()
+    want = solver.feautrier_forward(d, op)
+    parts = solver.feautrier_forward(d, op, with_u=False)
+    _abi.lib().mgx_release_workspace()
+    again = solver.feautrier_forward(d, op, with_u=False)
+    for got in (parts, again):
+        for k in ("J", "lambda_diag"):
+            assert (got[k] == want[k]).all(), k
