@@ -3010,7 +3010,7 @@ __device__ inline CentreRow centre_row(const KParams &kp, uint32_t o, double fre
 template <int APPROX, int PREC, bool IW>
 __global__ __launch_bounds__(MGX_WAVE, IW ? 2 : MGX_J_ADJOINT_WAVES_PER_SIMD) void feautrier_adjoint_kernel(
     const KParams *__restrict__ kpp, const double *__restrict__ J_bar, double *g_eps,
-    double *g_kap, double *g_iw, double *scratch, uint32_t capE)
+    double *g_kap, double *g_iw, double *scratch, uint32_t capE, uint32_t per)
 {
     mgx_ref_tables_init();
     const KParams &kp = *kpp;
@@ -3018,6 +3018,7 @@ __global__ __launch_bounds__(MGX_WAVE, IW ? 2 : MGX_J_ADJOINT_WAVES_PER_SIMD) vo
     const mgx_model &m = kp.m;
     const uint32_t lane = threadIdx.x, grp = lane >> 5;
     const uint32_t cap = kp.cap;
+    const uint32_t groups = (m.hnrays + per - 1) / per;
     const uint32_t P = m.npoints, F = m.nfreqs, Q = m.nquads;
     GroupRay *g = reinterpret_cast<GroupRay *>(smem + group_lds_offset(cap, kp.stage)) + grp;
     StagedEntry *chunk = reinterpret_cast<StagedEntry *>(smem + stage_lds_offset(cap)) + grp * kp.stage;
@@ -3026,12 +3027,17 @@ __global__ __launch_bounds__(MGX_WAVE, IW ? 2 : MGX_J_ADJOINT_WAVES_PER_SIMD) vo
                              (size_t)blockIdx.x * 2 * capE * Tape::kRecord + 8 * lane;
     const GradOut out = {g_eps, g_kap, g_iw};
 
-    /* origins are handed out by an atomic counter (status word 3, cleared before
-       the launch), so the waves finish together however the origins' costs vary */
-    for (;;) {
-        uint32_t onext = 0;
-        if (lane == 0) onext = atomicAdd(&kp.status[3], 1u);
-        const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)onext, 0);
+    /* an origin's ray pairs, per at a time, are handed out by an atomic counter (status
+       word 3, cleared before the launch), so the waves finish together however the costs
+       vary; the first of a wave is its own number */
+    uint32_t item = blockIdx.x;
+    for (bool first = true;; first = false) {
+        if (!first) {
+            uint32_t next = 0;
+            if (lane == 0) next = gridDim.x + atomicAdd(&kp.status[3], 1u);
+            item = (uint32_t)__builtin_amdgcn_readlane((int)next, 0);
+        }
+        const uint32_t o = item / groups, rr0 = item % groups * per;
         if (o >= P) break;
         /* a buffer of this launch overflowed: the host clears the gradients and
            relaunches, so the remaining origins are skipped */
@@ -3039,7 +3045,8 @@ __global__ __launch_bounds__(MGX_WAVE, IW ? 2 : MGX_J_ADJOINT_WAVES_PER_SIMD) vo
                                                              __HIP_MEMORY_SCOPE_AGENT)) &
             (ERR_CAP | ERR_CAPE))
             return;
-        for (uint32_t rr = 0; rr < m.hnrays; rr++) {
+        const uint32_t rr1 = rr0 + per < m.hnrays ? rr0 + per : m.hnrays;
+        for (uint32_t rr = rr0; rr < rr1; rr++) {
             const uint32_t ar = gld(&m.antipod[rr]);
             uint32_t S;
             double shift0;
@@ -3807,13 +3814,23 @@ int run_J_adjoint_k(hipStream_t st, DevBuffers &b, KParams &kp, const double *J_
 {
     auto kern = feautrier_adjoint_kernel<A, PR, IW>;
     const uint32_t P = kp.m.npoints;
+    /* few origins leave the GPU idle (3072 waves are resident at 3 per SIMD) or end with a
+       long tail: their ray pairs go to several waves, into about kAdjointItems items.  Many
+       more would wait for the counter that hands them out, about 40 ns each.  Forward and
+       adjoint measured by whole origins, this way and by single pairs (6 pairs): 6^3 1060,
+       590 and 600 us; 11^3 1340, 970 and 1130; 21^3 with two lines 3120, 3080 and 5110;
+       22^3 9.54, 9.40 and 9.65 ms; 24^3 20.0, 19.8 and 19.7 ms */
+    constexpr uint32_t kAdjointItems = 16384;
+    const uint64_t want = (kAdjointItems + (uint64_t)P - 1) / P;
+    const uint32_t per = want >= kp.m.hnrays ? 1 : (uint32_t)((kp.m.hnrays + want - 1) / want);
+    const uint32_t items = P * ((kp.m.hnrays + per - 1) / per);
     return adjoint_launch(
         st, b, kp, walk_key(kp.m), d_eps, d_kap, d_iw, (size_t)P * kp.m.nlines, 2,
-        [&](size_t lds) { return persistent_waves(kern, lds, P); },
+        [&](size_t lds) { return persistent_waves(kern, lds, items); },
         [&](size_t lds, uint32_t grid, uint32_t capE) {
             timed(st, [&] {
                 hipLaunchKernelGGL(kern, dim3(grid), dim3(MGX_WAVE), lds, st, b.kp_dev, J_bar, d_eps,
-                                   d_kap, d_iw, g_ws, capE);
+                                   d_kap, d_iw, g_ws, capE, per);
             });
         });
 }
