@@ -2,19 +2,20 @@
  * gfx950 kernels of the plain-method Feautrier formal solver, and the C-ABI
  * entry points that launch them.
  *
- * Work decomposition (one 64-lane wavefront per origin point o):
- *   for each ray pair rr (sequential, so J and Lambda accumulate in the
- *   reference's order without atomics):
- *     1. walk the neighbour lists from o along ray rr and along its antipod.
- *        The 64 lanes evaluate the neighbours of the current point in
+ * Work decomposition (one 64-lane wavefront per origin point o, or per group of an
+ * origin's ray pairs, see ray_split):
+ *   for each ray pair rr of the wave, in the reference's order:
+ *     1. the half-waves walk the neighbour lists from o, one along ray rr and one along
+ *        its antipod.  The 32 lanes evaluate the neighbours of the current point in
  *        parallel and a lexicographic (d2, list index) arg-min selects the
  *        next point; that is the first-wins strict "<" of
  *        Geometry::get_next_general_geometry (geometry.tpp:14-44).  The walk
  *        (point, dZ, Doppler shift per step) is staged in LDS.
- *     2. lanes take the quadrature frequencies of up to two lines (32 lanes
- *        per line).  Each lane expands its line's interpolation points on the
- *        fly (set_data_for_line, solver.tpp:1057-1097) and solves the
- *        second-order Feautrier system of its frequency with a two-sided
+ *     2. each half-wave takes the quadrature frequencies of one line (32 lanes per
+ *        slot).  Its lanes first stage the entries of the half ray side by side in LDS
+ *        (interpolation points, set_data_for_line, solver.tpp:1057-1097; what the
+ *        segment is for the line's bins), kStage at a time; then each lane solves the
+ *        second-order Feautrier system of its frequency over them with a two-sided
  *        elimination: backward from the antipod-side boundary to the origin,
  *        forward from the rr-side boundary to the origin, then joined at the
  *        origin.  This gives u(o) and the Lambda diagonal with O(1) state per
@@ -22,7 +23,7 @@
  *        back substitution (solver.tpp:2194-2318), with the same source,
  *        optical-depth and boundary terms.
  *     3. u(rr,o,f) is stored coalesced, J(o,f) and Lambda(o,l) updated by the
- *        owning wave.
+ *        owning wave, or kept per ray pair and added up in their order.
  *
  * Numerics: FP64 throughout, no FMA contraction (-ffp-contract=off), and the
  * reference's float transcendentals (the C library's expf, expm1f, logf,
@@ -602,9 +603,8 @@ __device__ inline double interp_linear(double a, double b, double t)
     return (b - a) * t + a;
 }
 
-/* the powf path of interpolate_log, taken only by interpolated entries: out of line,
-   so that its registers do not count against the solve's loop (with the reference's
-   double-internal powf inline, the FP64 forward kernel spilled 40 VGPRs) */
+/* the powf path of interpolate_log, taken only by interpolated entries; inlined, as a call
+   from the solve's loop would keep the registers of its whole callee-saved range */
 template <int PREC>
 __device__ __forceinline__ double interp_log_pow(double a, double b, double t)
 {

@@ -70,3 +70,23 @@ def test_ray_pair_parts_and_their_workspace(nrays):
     for got in (parts, again):
         for k in ("J", "lambda_diag"):
             assert (got[k] == want[k]).all(), k
+
+
+@pytest.mark.parametrize("n_edge,nrays", [(3, 12), (15, 48), (26, 12)])
+def test_adjoint_ray_pair_items(n_edge, nrays):
+    """the J adjoint takes one ray pair per item, five with a remainder of four, or an
+    origin's six; the sums' order differs: 1e-9 relative, as the other gradient tests, and
+    1e-10 of the largest where contributions of both signs cancel"""
+    import torch
+
+    from magritte_amd import solver
+    from oracle import oracle
+
+    print(f"[staged] adjoint items {n_edge}^3 {nrays} rays", flush=True)
+    m = models.model_wind(n_edge=n_edge, nrays=nrays, nquads=7, nlev=2)
+    op = m.options()
+    J_bar = np.random.Generator(np.random.PCG64(7)).standard_normal((m.npoints, m.nfreqs))
+    got = solver.feautrier_adjoint(solver.DeviceModel(m), op, torch.from_numpy(J_bar))
+    for name, a, b in zip(("d_eps", "d_kap"), got, oracle.J_adjoint(m, op, J_bar)):
+        a, b = np.asarray(a.cpu()), np.asarray(b)
+        assert np.all(np.abs(a - b) <= 1e-9 * np.abs(b) + 1e-10 * np.abs(b).max()), name
