@@ -603,11 +603,19 @@ __device__ inline double interp_linear(double a, double b, double t)
     return (b - a) * t + a;
 }
 
-/* the powf path of interpolate_log, taken only by interpolated entries; inlined, as a call
-   from the solve's loop would keep the registers of its whole callee-saved range */
+/* the powf path of interpolate_log, taken only by interpolated entries.  The reference's
+   double-internal powf runs out of line: inlined at its dozen places it grew the FP64
+   kernels' code and SGPR spills (old imager, 32^3 wind 5.96 and 4.19 ms; forward 12.3 and
+   11.9; 24^3 gradient of J 19.8 and 19.1).  The hardware one is a few instructions. */
+__device__ __noinline__ double interp_log_pow_ref(double a, double b, double t)
+{
+    return a * (double)f_pow<MGX_PREC_FP64>((float)(b / a), (float)t);
+}
+
 template <int PREC>
 __device__ __forceinline__ double interp_log_pow(double a, double b, double t)
 {
+    if constexpr (PREC == MGX_PREC_FP64) return interp_log_pow_ref(a, b, t);
     return a * (double)f_pow<PREC>((float)(b / a), (float)t);
 }
 
