@@ -3,13 +3,15 @@
  * inside its anonymous namespace).
  *
  * What a segment depends on -- the line data interpolated at its two entries -- is the
- * same for every bin of the group.  So each bin forms the derivative with respect to the
- * logarithms of an entry's emissivity and opacity (E, K) and to its inverse width (W),
- * these are summed over the group, and only the sums are taken on to the two points the
- * entry is interpolated between: once per (line, entry), by the lanes of the group side
- * by side, whatever the number of bins.
+ * same for every bin of the group.  So each bin forms the derivative with respect to an
+ * entry's source, emissivity, opacity and inverse width (S, E, K, W), these are summed over
+ * the group, and only the sums are taken on to the two points the entry is interpolated
+ * between: once per (line, entry), by the lanes of the group side by side, whatever the
+ * number of bins.
  *   eps_i = eps_a^(1-t) eps_b^t (the same for kappa and for their quotient, the source),
- *   so d/d eps_a = (1 - t) E / eps_a, d/d eps_b = t E / eps_b; iw_i is linear in t.
+ *   so d eps_i / d eps_a = (1 - t) eps_i / eps_a, d eps_i / d eps_b = t eps_i / eps_b; iw_i
+ *   is linear in t.  An entry at a point (t = 0) has the point's own values: the factor is
+ *   one and no emissivity or opacity, which may be zero, is divided by.
  *
  * Before, a bin's reverse of an interpolated segment recomputed its erf and powf terms and
  * added to four points by itself, behind a call, and every walk step summed its points over
@@ -36,9 +38,10 @@ struct Tape {
     }
 };
 
-/* sums of a group's bins for one staged entry */
+/* sums of a group's bins for one line at a staged entry: the derivatives with respect to
+   its source (of line-integrated segments), emissivity and opacity there, and inverse width */
 struct EntryGrad {
-    double E, K, W;
+    double S, E, K, W;
 };
 
 /* where the gradients go; g_iw only in the IW instantiations */
@@ -51,25 +54,38 @@ __device__ __forceinline__ void grad_add(double *g, size_t i, double v)
     if (v != 0.0) unsafeAtomicAdd(&g[i], v);
 }
 
-/* takes the sums of line l at an entry on to its point and partner */
+/* takes the sums of line l at an entry, whose emissivity, opacity and source are eps, kap
+   and src (read where s has a derivative of them), on to its point and partner */
 template <bool IW>
 __device__ inline void entry_scatter(const KParams &kp, const GradOut &out, const StagedEntry *e, uint32_t l,
-                                     const EntryGrad &s)
+                                     double eps, double kap, double src, const EntryGrad &s)
 {
     const size_t L = kp.m.nlines, ia = (size_t)e->nr * L + l;
     const double t = e->fac;
     const double4 a = lp(kp, e->nr, l);
-    const double ta = (t == 1.0) ? 0.0 : 1.0 - t;
-    grad_add(out.eps, ia, ta * s.E / a.y);
-    grad_add(out.kap, ia, ta * s.K / a.z);
     if (IW) grad_add(out.iw, ia, (1.0 - t) * s.W);
-    if (t != 0.0) {
-        const size_t ib = (size_t)e->nri * L + l;
-        const double4 b = lp(kp, e->nri, l);
-        grad_add(out.eps, ib, t * s.E / b.y);
-        grad_add(out.kap, ib, t * s.K / b.z);
-        if (IW) grad_add(out.iw, ib, t * s.W);
+    if (t == 0.0) {
+        double de = s.E, dk = s.K;
+        if (s.S != 0.0) {
+            const double r = s.S / a.z;
+            de += r;
+            dk -= r * a.w;
+        }
+        grad_add(out.eps, ia, de);
+        grad_add(out.kap, ia, dk);
+        return;
     }
+    /* derivatives with respect to the logarithms */
+    const double Ss = s.S != 0.0 ? s.S * src : 0.0;
+    const double E = Ss + s.E * eps, K = s.K * kap - Ss;
+    const double ta = (t == 1.0) ? 0.0 : 1.0 - t;
+    grad_add(out.eps, ia, ta * E / a.y);
+    grad_add(out.kap, ia, ta * K / a.z);
+    const size_t ib = (size_t)e->nri * L + l;
+    const double4 b = lp(kp, e->nri, l);
+    grad_add(out.eps, ib, t * E / b.y);
+    grad_add(out.kap, ib, t * K / b.z);
+    if (IW) grad_add(out.iw, ib, t * s.W);
 }
 
 __device__ __forceinline__ double group_sum(double v)
@@ -82,10 +98,12 @@ template <bool IW>
 __device__ __forceinline__ bool group_total(EntryGrad &s)
 {
     const uint32_t grp = (threadIdx.x & (MGX_WAVE - 1)) >> 5;
-    const uint64_t b = __ballot(s.E != 0.0 || s.K != 0.0 || (IW && s.W != 0.0));
+    const uint64_t b_S = __ballot(s.S != 0.0), b_E = __ballot(s.E != 0.0), b_K = __ballot(s.K != 0.0);
+    const uint64_t b_W = IW ? __ballot(s.W != 0.0) : 0, b = b_S | b_E | b_K | b_W;
     if (b == 0) return false;
-    s.E = group_sum(s.E);
-    s.K = group_sum(s.K);
+    if (b_S) s.S = group_sum(s.S);
+    if (b_E) s.E = group_sum(s.E);
+    if (b_K) s.K = group_sum(s.K);
     if (IW) s.W = group_sum(s.W);
     return ((b >> (32 * grp)) & 0xffffffffull) != 0;
 }
@@ -118,10 +136,10 @@ __device__ __forceinline__ void line_bwd(const WindowLine &w, double f_o, double
                                          double ld_bar, double so, double si, EntryGrad &o, EntryGrad &i)
 {
     const double op_bar = 0.5 * dop * ld_bar;
-    o.E += so * w.src_o;
-    o.K += w.kap_o * op_bar - so * w.src_o;
-    i.E += si * w.src_i;
-    i.K += w.kap_i * op_bar - si * w.src_i;
+    o.S += so;
+    o.K += op_bar;
+    i.S += si;
+    i.K += op_bar;
     if (IW && ld_bar != 0.0) {
         const double wb = 0.5 * ld_bar * dtau_line_dw((w.iw_o + w.iw_i) / 2.0, (w.kap_o + w.kap_i) / 2.0, w.f,
                                                       f_o, f_i, dz);
@@ -160,11 +178,11 @@ __device__ __forceinline__ void window_bwd(const KParams &kp, const GroupRay *g,
     }
     window_lines_of<APPROX, PREC, ENTRY>(
         kp, g, lines, nw, eo, ei, f_o, f_i, mine, [&](const WindowLine *w, uint32_t l, bool in) {
-            EntryGrad o = {0.0, 0.0, 0.0}, i = {0.0, 0.0, 0.0};
+            EntryGrad o = {0.0, 0.0, 0.0, 0.0}, i = {0.0, 0.0, 0.0, 0.0};
             if (in && ENTRY) {
                 const double prof = gaussian<PREC>(w->iw_o, f_i - w->f);
-                i.E = sa * (prof * w->src_o);
-                i.K = sb * (prof * w->kap_o);
+                i.E = sa * prof;
+                i.K = sb * prof;
                 if (IW) i.W = gaussian_dw(w->iw_o, f_i - w->f) * (sa * w->src_o + sb * w->kap_o);
             } else if (in) {
                 double dop;
@@ -174,8 +192,13 @@ __device__ __forceinline__ void window_bwd(const KParams &kp, const GroupRay *g,
             }
             const bool any_o = ENTRY ? false : group_total<IW>(o);
             const bool any_i = group_total<IW>(i);
-            if (q == 0 && any_o) entry_scatter<IW>(kp, out, eo, l, o);
-            if (q == 0 && any_i) entry_scatter<IW>(kp, out, ei, l, i);
+            if (q == 0 && any_o) entry_scatter<IW>(kp, out, eo, l, 0.0, w->kap_o, w->src_o, o);
+            if (q == 0 && any_i) {
+                if (ENTRY) /* src_o is the emissivity */
+                    entry_scatter<IW>(kp, out, ei, l, w->src_o, w->kap_o, 0.0, i);
+                else
+                    entry_scatter<IW>(kp, out, ei, l, 0.0, w->kap_i, w->src_i, i);
+            }
         });
 }
 
@@ -221,7 +244,7 @@ struct RevCentre {
     bool centre_last;  /* rr-side half only: the centre is the system's last row */
 };
 
-/* adjoints an entry collects: of its own line's logarithms, and of emissivity and opacity
+/* adjoints an entry collects: of its own line's values, and of emissivity and opacity
    from the trapezoid segments on either side (values in eta, chi) */
 struct EntryBar {
     EntryGrad s;
@@ -245,14 +268,14 @@ __device__ __forceinline__ void reverse_half(const KParams &kp, unsigned char *s
     WindowLine *lines = reinterpret_cast<WindowLine *>(smem + lines_lds_offset(kp.cap, count)) +
                         ((threadIdx.x & (MGX_WAVE - 1)) >> 5) * nw;
     double u_in = rc.u, mu_in = rc.mu, lam_in = rc.lam, dbar = rc.dbar;
-    EntryBar in = {{0.0, 0.0, 0.0}, 0.0, 0.0, 0.0, 0.0, 0.0, false};
+    EntryBar in = {{0.0, 0.0, 0.0, 0.0}, 0.0, 0.0, 0.0, 0.0, 0.0, false};
     double Y = 0.0, X = 0.0, XI = 0.0, d = 0.0, gk = 0.0;
     bool first = true;
     for (uint32_t done = 0; done < nmax; done += count - 1) {
         /* entries k0 .. k0 + count - 1 of each group; the innermost one left is the last */
         const int k0 = (int)n_all - (int)done - (int)(count - 1);
         stage_chunk<APPROX, PREC>(kp, smem, g, k0, count, chunk);
-        if (q < count) sums[q] = EntryGrad{0.0, 0.0, 0.0};
+        if (q < count) sums[q] = EntryGrad{0.0, 0.0, 0.0, 0.0};
         __syncthreads();
         const uint32_t left = nmax - done, jmin = left < count - 1 ? count - left : 1;
         for (uint32_t j = count - 1; j >= jmin; j--) {
@@ -305,7 +328,7 @@ __device__ __forceinline__ void reverse_half(const KParams &kp, unsigned char *s
                     if (seg != SEG_EMPTY) dbar -= lam_k * bdy_row_dd(d, I_b, u_k, Din);
                 }
             }
-            EntryBar eb = {{0.0, 0.0, 0.0}, 0.0, 0.0, 0.0, 0.0, 0.0, false}; /* the outer entry */
+            EntryBar eb = {{0.0, 0.0, 0.0, 0.0}, 0.0, 0.0, 0.0, 0.0, 0.0, false}; /* the outer entry */
             const double so = backward ? (k == 1 ? lam_k : 0.0) : lam_k;
             const double si = backward ? lam_in : (k == (int)n && rc.centre_last ? rc.lam : 0.0);
             if (seg == SEG_LANE) {
@@ -350,8 +373,8 @@ __device__ __forceinline__ void reverse_half(const KParams &kp, unsigned char *s
                 const bool multi = here && e.have && !(e.phi == e.phi) && (e.eta_bar != 0.0 || e.chi_bar != 0.0);
                 if (own) {
                     /* eta = phi eps, chi = chi_min + phi kappa */
-                    e.s.E += e.eta_bar * e.eta;
-                    e.s.K += e.chi_bar * (e.phi * se->kap);
+                    e.s.E += e.eta_bar * e.phi;
+                    e.s.K += e.chi_bar * e.phi;
                     if (IW && e.phi != 0.0)
                         e.s.W += gaussian_dw(se->iw, freq * se->shift - bin.a_g) *
                                  (se->eps * e.eta_bar + se->kap * e.chi_bar);
@@ -362,7 +385,7 @@ __device__ __forceinline__ void reverse_half(const KParams &kp, unsigned char *s
                     window_bwd<APPROX, PREC, true, IW>(kp, g, lines, nw, se, se, f, f, multi, none, e.eta_bar,
                                                        e.chi_bar, 0.0, out);
                 }
-                EntryGrad t = here ? e.s : EntryGrad{0.0, 0.0, 0.0};
+                EntryGrad t = here ? e.s : EntryGrad{0.0, 0.0, 0.0, 0.0};
                 if (group_total<IW>(t) && q == 0) *sum = t;
             };
             finish(in, ei, &sums[j], on);
@@ -386,8 +409,9 @@ __device__ __forceinline__ void reverse_half(const KParams &kp, unsigned char *s
         const int ks = k0 + (int)q;
         if (q < count && ks >= 0 && (q > 0 || ks == 0) && ks <= (int)n_all) {
             const EntryGrad t = sums[q];
-            if (t.E != 0.0 || t.K != 0.0 || (IW && t.W != 0.0))
-                entry_scatter<IW>(kp, out, chunk + q, g->line, t);
+            const StagedEntry *se = chunk + q;
+            if (t.S != 0.0 || t.E != 0.0 || t.K != 0.0 || (IW && t.W != 0.0))
+                entry_scatter<IW>(kp, out, se, g->line, se->eps, se->kap, se->src, t);
         }
         __syncthreads();
     }

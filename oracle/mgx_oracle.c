@@ -292,12 +292,13 @@ static inline double interp_log(double a, double b, double t)
     return a * (double)O_POWF((float)(b / a), (float)t);
 }
 
-/* partial derivatives of interpolate_log(a, b, t) = a^(1-t) b^t (r its value) */
+/* partial derivatives of interpolate_log(a, b, t) = a^(1-t) b^t (r its value); at an end
+   it is that end's value, which may be zero */
 static inline void interp_log_partials(double a, double b, double t, double r, double *da,
                                        double *db)
 {
-    *da = (t == 1.0) ? 0.0 : (1.0 - t) * r / a;
-    *db = (t == 0.0) ? 0.0 : t * r / b;
+    *da = (t == 0.0) ? 1.0 : (t == 1.0) ? 0.0 : (1.0 - t) * r / a;
+    *db = (t == 0.0) ? 0.0 : (t == 1.0) ? 1.0 : t * r / b;
 }
 
 /* ------------------------------------------------------------------------- */

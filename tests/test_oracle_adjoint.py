@@ -148,3 +148,62 @@ def test_reference_powf_limits_finite_differences(wind6):
               for p, l in pts]
     assert max(errs_s) < 1e-6
     assert max(errs_r) > 10 * max(errs_s)
+
+
+def _no_interpolation(m, **kw):
+    op = m.options(**kw)
+    op.max_interpolation_diff = 1.0e30
+    return op
+
+
+@pytest.mark.parametrize("approx", [_abi.APPROX_CLOSE_LINES, _abi.APPROX_NONE, _abi.APPROX_ONE_LINE])
+@pytest.mark.parametrize("everywhere", [False, True])
+def test_gradient_at_zero_emissivity(wind6, approx, everywhere):
+    """J is linear in the emissivities (opacities and trace fixed): the gradient at zero
+    emissivity is the difference that a whole emissivity makes"""
+    op = _no_interpolation(wind6, approx=approx)
+    rng = np.random.default_rng(21)
+    Jb = rng.standard_normal((wind6.npoints, wind6.nfreqs))
+    eps = wind6.emissivity.copy()
+    try:
+        dark = np.arange(wind6.npoints) if everywhere else rng.choice(wind6.npoints, 20, replace=False)
+        wind6.emissivity[dark] = 0.0
+        de, dk = oracle.J_adjoint(wind6, op, Jb)
+        assert np.all(np.isfinite(de)) and np.all(np.isfinite(dk))
+        J0 = oracle.solve(wind6, op, with_u=False)[1]
+        for p in rng.choice(dark, 4, replace=False):
+            l = int(rng.integers(wind6.nlines))
+            wind6.emissivity[p, l] = eps[p, l]
+            diff = oracle.solve(wind6, op, with_u=False)[1] - J0
+            wind6.emissivity[p, l] = 0.0
+            want = float(np.sum(Jb * diff)) / eps[p, l]
+            # a difference of sums of J: 1e-13 of their size
+            assert abs(de[p, l] - want) <= 1e-9 * abs(want) + 1e-13 * np.sum(np.abs(Jb * J0)) / eps[p, l]
+    finally:
+        wind6.emissivity[:] = eps
+
+
+def test_gradient_at_zero_opacity():
+    """a model whose segments all take the trapezoid rule, some points without emissivity and
+    opacity: the opacity's gradient there against differences"""
+    m = models.model_wind(n_edge=6, seed=models.seed_for(1, 11), nlev=3)
+    m.params["max_width_fraction"] = 1.0e6
+    m.finalize()
+    op = _no_interpolation(m)
+    rng = np.random.default_rng(22)
+    Jb = rng.standard_normal((m.npoints, m.nfreqs))
+    kap = m.opacity.copy()
+    empty = rng.choice(m.npoints, 20, replace=False)
+    m.emissivity[empty] = 0.0
+    m.opacity[empty] = 0.0
+    de, dk = oracle.J_adjoint(m, op, Jb)
+    assert np.all(np.isfinite(de)) and np.all(np.isfinite(dk))
+    for p in empty[np.argsort(-np.abs(dk[empty, 0]))][:4]:
+        h = 1e-5 * kap[p, 0]
+        m.opacity[p, 0] = h
+        Jp = oracle.solve(m, op, with_u=False)[1]
+        m.opacity[p, 0] = -h
+        Jm = oracle.solve(m, op, with_u=False)[1]
+        m.opacity[p, 0] = 0.0
+        fd = float(np.sum(Jb * (Jp - Jm))) / (2 * h)
+        assert abs(dk[p, 0] - fd) < 1e-4 * abs(fd), (dk[p, 0], fd)
