@@ -1208,10 +1208,10 @@ __device__ __forceinline__ void staged_sweep(const KParams &kp, unsigned char *s
         for (uint32_t j = 1; j <= jmax; j++) {
             const StagedEntry *eo = chunk + j - 1, *ei = chunk + j;
             PointEC ec_in = {0.0, 0.0, false};
-            double dtau, S_out, S_in, dop;
+            double dtau, S_out, S_in, raw, dop;
             const bool on = k0 + j <= n;
             staged_segment<APPROX, PREC>(kp, g, lines, window_lines(count), bin, eo, ei, on, out, ec_out, ec_in, dtau,
-                                         S_out, S_in, dop);
+                                         S_out, S_in, raw, dop);
             if (!on) continue;
             if constexpr (METHOD == METHOD_TAU) {
                 sw.Y += dtau;
@@ -1270,7 +1270,7 @@ __device__ __forceinline__ void staged_sweep(const KParams &kp, unsigned char *s
                 *tape->at(k, 0) = sw.Y;
                 *tape->at(k, 1) = sw.X;
                 if ((ei->kind & SEG_MASK) != SEG_EMPTY) {
-                    *tape->at(k, 2) = dtau;
+                    *tape->at(k, 2) = raw;
                     *tape->at(k, 3) = dop;
                 }
             }

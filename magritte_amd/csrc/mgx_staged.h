@@ -508,16 +508,16 @@ __device__ __forceinline__ void staged_eta_chi(const KParams &kp, const GroupRay
  * solver.tpp:2140-2186).  Its value does not depend on which end is the current one.
  * ec_out / ec_in cache the ends' emissivity and opacity (ec_out from the segment
  * before, when that took the trapezoid rule too).  All lanes of the wave call this
- * together; those without a segment pass on = false.  dop is d depth / d mean opacity of a
- * segment with the own line alone, its lowest bit set when the depth was clamped (for the
- * adjoint's tape; it costs the other sweeps nothing).
+ * together; those without a segment pass on = false.  For the adjoint's tape (the other
+ * sweeps drop them): raw is the depth before a line-integrated one is clamped, dop
+ * d depth / d mean opacity of a segment with the own line alone.
  */
 template <int APPROX, int PREC>
 __device__ __forceinline__ void staged_segment(const KParams &kp, const GroupRay *g, WindowLine *lines, uint32_t nw,
                                                const BinLine &bin, const StagedEntry *eo,
                                                const StagedEntry *ei, bool on, OuterEnd &out, PointEC &ec_out,
                                                PointEC &ec_in, double &dtau, double &S_out, double &S_in,
-                                               double &dop)
+                                               double &raw, double &dop)
 {
     const uint32_t kind = ei->kind;
     const double dz = ei->dz;
@@ -528,7 +528,7 @@ __device__ __forceinline__ void staged_segment(const KParams &kp, const GroupRay
     in.f = bin.freq * ei->shift;
     const double bound = kp.op.min_opacity * dz;
     uint32_t seg = on ? kind & SEG_MASK : SEG_EMPTY;
-    dtau = bound;
+    dtau = raw = bound;
     dop = S_out = S_in = 0.0;
     if (seg == SEG_LANE) {
         const uint32_t w = lane_window<APPROX>(kp, g->ol, out.f, in.f, ei->ubm);
@@ -537,25 +537,22 @@ __device__ __forceinline__ void staged_segment(const KParams &kp, const GroupRay
     if (seg == SEG_SOLO) {
         const double d = line_depth<PREC>(out.iw, in.iw, out.kap, in.kap, out.f, in.f, bin.a_g, dz,
                                           kp.op.min_opacity, dop);
-        uint64_t bits = __builtin_bit_cast(uint64_t, dop) & ~1ull;
         S_out = out.src;
         S_in = in.src;
-        dtau = d;
+        dtau = raw = d;
         if (APPROX == MGX_APPROX_CLOSE_LINES && -bound < d && d < bound) {
             /* the clamped depth: the sources keep their share of the line's own */
             const double share = d * rcp(bound);
             dtau = bound;
             S_out *= share;
             S_in *= share;
-            bits |= 1;
         }
-        dop = __builtin_bit_cast(double, bits);
     }
     if (__ballot(seg >= SEG_LANE)) {
         if (__ballot(seg == SEG_LANE)) {
             const WindowSum v = window_sum<APPROX, PREC, false>(kp, g, lines, nw, eo, ei, out.f, in.f, seg == SEG_LANE);
             if (seg == SEG_LANE) {
-                double d = v.a;
+                double d = raw = v.a;
                 if (APPROX == MGX_APPROX_CLOSE_LINES && -bound < d) d = (bound < d) ? d : bound;
                 const double rd = rcp(d);
                 dtau = d;
@@ -571,7 +568,7 @@ __device__ __forceinline__ void staged_segment(const KParams &kp, const GroupRay
             ec_in.valid = true;
             S_out = ec_out.eta * rcp(ec_out.chi);
             S_in = ec_in.eta * rcp(ec_in.chi);
-            dtau = 0.5 * (ec_out.chi + ec_in.chi) * dz;
+            dtau = raw = 0.5 * (ec_out.chi + ec_in.chi) * dz;
         }
     }
     out = in;

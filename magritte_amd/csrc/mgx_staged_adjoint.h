@@ -22,8 +22,9 @@
  */
 
 /* Tape of one half ray: segment k (counted from the outer end) stores Y and X of the row
-   at its outer entry and, unless the segment is empty for every bin, its depth and, for a
-   line-integrated one, d depth / d mean opacity.  Lanes lie side by side within a word.
+   at its outer entry and, unless the segment is empty for every bin, its depth (before the
+   clamp of a line-integrated one) and d depth / d mean opacity of one with the own line
+   alone.  Lanes lie side by side within a word.
    The words are doubles in mixed precision too: the reverse forms u_k - u_{k+1} from Y and
    X, which cancels where u is smooth. */
 #define MGX_TAPE_WORDS 4
@@ -148,6 +149,13 @@ __device__ __forceinline__ void line_bwd(const WindowLine &w, double f_o, double
     }
 }
 
+/* whether a line-integrated depth is raised to the smallest one, as the forward sweep does */
+template <int APPROX>
+__device__ __forceinline__ bool depth_clamped(double raw, double bound)
+{
+    return APPROX == MGX_APPROX_CLOSE_LINES && -bound < raw && raw < bound;
+}
+
 /*
  * Reverse of window_sum: the lines of the bins' windows, in rounds of nw lines a group has
  * staged in LDS.  ENTRY false: the segment eo - ei with adjoints a_bar of its depth and
@@ -165,12 +173,9 @@ __device__ __forceinline__ void window_bwd(const KParams &kp, const GroupRay *g,
     double sa = a_bar, sb = b_bar, sc = c_bar;
     if (!ENTRY) {
         double d = v.a;
-        bool clamped = false;
-        if (APPROX == MGX_APPROX_CLOSE_LINES) {
-            const double bound = kp.op.min_opacity * ei->dz;
-            clamped = -bound < d && d < bound;
-            if (clamped) d = bound;
-        }
+        const double bound = kp.op.min_opacity * ei->dz;
+        const bool clamped = depth_clamped<APPROX>(d, bound);
+        if (clamped) d = bound;
         const double rd = rcp(d);
         sb = b_bar * rd;
         sc = c_bar * rd;
@@ -269,7 +274,7 @@ __device__ __forceinline__ void reverse_half(const KParams &kp, unsigned char *s
                         ((threadIdx.x & (MGX_WAVE - 1)) >> 5) * nw;
     double u_in = rc.u, mu_in = rc.mu, lam_in = rc.lam, dbar = rc.dbar;
     EntryBar in = {{0.0, 0.0, 0.0, 0.0}, 0.0, 0.0, 0.0, 0.0, 0.0, false};
-    double Y = 0.0, X = 0.0, XI = 0.0, d = 0.0, gk = 0.0;
+    double Y = 0.0, X = 0.0, XI = 0.0, raw = 0.0, gk = 0.0;
     bool first = true;
     for (uint32_t done = 0; done < nmax; done += count - 1) {
         /* entries k0 .. k0 + count - 1 of each group; the innermost one left is the last */
@@ -282,21 +287,21 @@ __device__ __forceinline__ void reverse_half(const KParams &kp, unsigned char *s
             const int k = k0 + (int)j; /* segment between entries k - 1 and k */
             const bool on = k >= 1 && n > 0;
             const StagedEntry *eo = chunk + j - 1, *ei = chunk + j;
-            const double dz = ei->dz, bound = kp.op.min_opacity * dz;
+            const double dz = ei->dz, bound = kp.op.min_opacity * dz, bound_n = kp.op.min_opacity * eo->dz;
             const uint32_t kind = on ? ei->kind : (uint32_t)SEG_EMPTY;
             uint32_t seg = kind & SEG_MASK;
             const uint32_t seg_n = on && k >= 2 ? eo->kind & SEG_MASK : (uint32_t)SEG_EMPTY;
             const double f_i = freq * ei->shift, f_o = freq * eo->shift;
-            double Yn = 0.0, Xn = 0.0, XIn = 0.0, dn = 0.0, gn = 0.0;
+            double Yn = 0.0, Xn = 0.0, XIn = 0.0, raw_n = 0.0, gn = 0.0;
             double u_k = 0.0, mu_k = 0.0, lam_k = 0.0, dbar_next = 0.0;
             if (on) {
                 if (first) {
                     Y = *tape.at(k - 1, 0);
                     X = *tape.at(k - 1, 1);
                     XI = rcp(1.0 + X);
-                    d = bound;
+                    raw = bound;
                     if (seg != SEG_EMPTY) {
-                        d = *tape.at(k - 1, 2);
+                        raw = *tape.at(k - 1, 2);
                         gk = *tape.at(k - 1, 3);
                     }
                     first = false;
@@ -304,16 +309,18 @@ __device__ __forceinline__ void reverse_half(const KParams &kp, unsigned char *s
                 if (k >= 2) {
                     Yn = *tape.at(k - 2, 0);
                     Xn = *tape.at(k - 2, 1);
-                    dn = kp.op.min_opacity * eo->dz;
+                    raw_n = bound_n;
                     if (seg_n != SEG_EMPTY) {
-                        dn = *tape.at(k - 2, 2);
+                        raw_n = *tape.at(k - 2, 2);
                         gn = *tape.at(k - 2, 3);
                     }
                 }
+                const double d = seg != SEG_TRAP && depth_clamped<APPROX>(raw, bound) ? bound : raw;
                 u_k = fma(XI, u_in, Y);
                 mu_k = XI * mu_in;
                 const double Din = fma(-X * XI, u_in, Y); /* u_k - u_in */
                 if (k >= 2) {
+                    const double dn = seg_n != SEG_TRAP && depth_clamped<APPROX>(raw_n, bound_n) ? bound_n : raw_n;
                     lam_k = 0.5 * (dn + d) * mu_k;
                     XIn = rcp(1.0 + Xn);
                     if (seg != SEG_EMPTY || seg_n != SEG_EMPTY) {
@@ -337,12 +344,12 @@ __device__ __forceinline__ void reverse_half(const KParams &kp, unsigned char *s
             }
             if (seg == SEG_SOLO) {
                 /* one line: unclamped, the segment's sources are the line's own and the adjoint
-                   of its depth is dbar (the source terms cancel exactly); clamped (the lowest
-                   bit of gk), the depth is the bound and the sources scale with the line's */
+                   of its depth is dbar (the source terms cancel exactly); clamped, the depth is
+                   the bound and the sources scale with the line's */
                 const WindowLine w = {bin.a_g, eo->iw, eo->kap, eo->src, ei->iw, ei->kap, ei->src, 0u, 0u};
                 double ld_bar = dbar, a = so, b = si;
-                if (__builtin_bit_cast(uint64_t, gk) & 1) {
-                    const double rb = rcp(bound), share = fma(0.5 * (w.kap_o + w.kap_i), gk, bound) * rb;
+                if (depth_clamped<APPROX>(raw, bound)) {
+                    const double rb = rcp(bound), share = raw * rb;
                     ld_bar = (so * w.src_o + si * w.src_i) * rb;
                     a *= share;
                     b *= share;
@@ -399,7 +406,7 @@ __device__ __forceinline__ void reverse_half(const KParams &kp, unsigned char *s
                 Y = Yn;
                 X = Xn;
                 XI = XIn;
-                d = dn;
+                raw = raw_n;
                 gk = gn;
             }
         }
