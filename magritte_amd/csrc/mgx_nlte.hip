@@ -351,7 +351,7 @@ struct GlobalIn {
  * scalar registers instead of LDS reads, and LDS keeps only the matrix itself for the residuals.
  * Each level's transitions come from its own list, four gathers at a time, instead of every
  * lane looking through all of them.  5832 points x 41 levels: 2.77 ms before (two matrices
- * in LDS, five waves per CU, 820 transitions looked through by every lane), 0.42 ms now; the
+ * in LDS, five waves per CU, 820 transitions looked through by every lane), 0.43 ms now; the
  * same results to the last bit.
  */
 template <bool GLOBAL, int NMAX>
@@ -546,18 +546,15 @@ __global__ __launch_bounds__(NL_WAVE) void stateq_kernel(NView v, const double *
         }
         row[NMAX - 1] = keep;
     }
-    const double rdiag = 1.0 / diag;
-    /* U x = b by columns from the last: lane c's x_c */
+    /* U x = b by columns from the last: lane c's x_c.  A division, not a product with the
+       pivot's reciprocal, which overflows for a pivot below 5.6e-309. */
     const auto back = [&](double b) {
         double x = 0.0;
 #pragma unroll
         for (int c = NMAX - 1; c >= 0; c--) {
             if ((uint32_t)c >= n) continue;
             const int pr = lane_of_step(my_step, c);
-            /* b / diag to the last bit: the quotient and one correction */
-            double q = b * rdiag;
-            q = fma(fma(-q, diag, b), rdiag, q);
-            if (diag == 0.0) q = 0.0;
+            const double q = diag != 0.0 ? b / diag : 0.0;
             const double xc = lane_value(q, pr);
             if ((int)lane == c) x = xc;
             if (r < n && my_step < c) b = fma(-row[c], xc, b);

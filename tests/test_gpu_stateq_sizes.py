@@ -44,3 +44,34 @@ def test_update_at_row_edges(nlev):
     assert np.all(np.isfinite(got))
     assert np.all(np.abs(got - ref) <= 1e-10 * np.abs(ref) + 1e-14 * ptot), float(
         np.max(np.abs(got - ref) / (np.abs(ref) + 1e-4 * ptot)))
+
+
+@pytest.mark.parametrize("nlev", [2, 5])
+def test_pivots_whose_reciprocal_overflows(nlev):
+    """Rates multiplied by one power of two have the same populations.  With some 1e-312 a
+    pivot's quotients are numbers where its reciprocal is not; such a rate has about 37 bits
+    (6e-12), a few of which are added up (1e-9).  The oracle's decomposition, as the
+    reference's, takes a row that small for a dependent one, so the other rates' update is
+    what it is compared with."""
+    import torch
+
+    from magritte_amd import solver
+
+    print(f"[stateq] {nlev} levels, rates of 1e-312", flush=True)
+    pops = []
+    for scale in (1.0, 2.0**-1013):
+        m = models.model_line_1d(npoints=7, nquads=3)
+        ld = models.linedata_linear_rotor(57.6e9, 0.11, nlev)
+        ld["colpar"] = [models.colpar_constant(ld, 0, 0.0)]
+        for k in ("A", "Bs", "Ba"):
+            ld[k] = ld[k] * scale
+        m.set_lines([ld], 3)
+        m.finalize()
+        lp = solver.LevelPopulations(solver.DeviceModel(m))
+        lp.set_lte()
+        nu = m.nu.reshape(m.npoints, m.nfreqs)
+        J = 2.0 * models.HH * nu**3 / models.CC_SQUARED / np.expm1(models.HH * nu / (models.KB * 15.0))
+        lp.stateq(torch.from_numpy(J).cuda(), torch.zeros((m.npoints, m.nlines), dtype=torch.float64).cuda())
+        pops.append(lp.populations()[0].cpu().numpy())
+    assert np.all(pops[0] > 0)
+    np.testing.assert_allclose(pops[1], pops[0], rtol=1e-9)
