@@ -1019,9 +1019,8 @@ __device__ inline double hi_advance(const KParams &kp, HalfIter &it, uint32_t l,
 #include "mgx_staged.h"
 
 /* LDS layout of the walk buffers of both half rays (point, length, shift per step)
-   plus 16 bytes a step for interpolation counts: four tables (2 lines x 2 halves)
-   of u16 in the tracing, imaging and adjoint kernels, two tables of u32 prefix sums
-   in the solves */
+   plus 8 bytes a step for interpolation counts: two tables of u32 prefix sums in the
+   staged sweeps, u16 counts in the old imager */
 __host__ __device__ inline size_t walk_lds_bytes(uint32_t cap)
 {
     return 8 * ((2 * (size_t)cap * 4 + 7) / 8) + 4 * (size_t)cap * 8 + 4 * (size_t)cap * 2;
@@ -1043,8 +1042,11 @@ __host__ __device__ inline size_t lines_lds_offset(uint32_t cap, uint32_t stage)
     return group_lds_offset(cap, stage) + 2 * sizeof(GroupRay);
 }
 
-/* lines a group takes side by side for windows with several lines */
-__host__ __device__ inline uint32_t window_lines(uint32_t stage) { return stage < kStage ? 1 : kWindowLines; }
+/* lines a group takes side by side for windows with several lines, beside stage entries */
+__host__ __device__ inline uint32_t window_lines(uint32_t stage)
+{
+    return stage - 2 < kWindowLines ? stage - 2 : kWindowLines;
+}
 
 __host__ __device__ inline size_t acc_lds_offset(uint32_t cap, uint32_t stage)
 {
@@ -1085,13 +1087,6 @@ inline bool j_in_lds(uint32_t cap, uint32_t stage, uint32_t F, uint32_t L)
 {
     const size_t share = (160 * 1024) / (4 * MGX_SOLVE_WAVES_PER_SIMD);
     return solve_lds_bytes(cap, stage, F, L, true) + kStaticLds <= share;
-}
-
-/* entries a group stages at a time: as many as its lanes can stage side by side; few
-   where the walk buffers of very long rays need the room */
-inline uint32_t stage_entries(uint32_t cap, uint32_t L)
-{
-    return solve_lds_bytes(cap, kStage, 0, L, false) + kStaticLds <= 80 * 1024 ? kStage : kStageMin;
 }
 
 /* J(o, f) += c for one ray pair: the first ray pair of a full pass stores (the sum
@@ -3543,6 +3538,26 @@ size_t lds_budget()
     return cached[dev];
 }
 
+/*
+ * Entries a group stages at a time beside walk buffers of cap steps, per_entry bytes a staged
+ * entry and tail bytes: as many as its lanes stage side by side while two workgroups fit a
+ * CU's LDS, which is up to about 1500 steps.  Beyond, the walk buffers alone decide whether
+ * one or two do, and the chunk takes what they leave of that share.  Chains of 1550, 1620,
+ * 2000 and 3000 points with five blended lines, forward: three entries and one window line at
+ * a time from 80 KiB on took 59, 62, 154 and 345 ms, this takes 35, 38, 89 and 200.
+ */
+uint32_t stage_entries(uint32_t cap, size_t tail, size_t per_entry = 0)
+{
+    const size_t limit = lds_budget() + kReservedLds, half = (160 * 1024) / 2;
+    const auto bytes = [&](uint32_t stage) {
+        return acc_lds_offset(cap, stage) + per_entry * stage + tail + kStaticLds;
+    };
+    const size_t room = bytes(kStageMin) <= half && half < limit ? half : limit;
+    uint32_t stage = kStage;
+    while (stage > kStageMin && bytes(stage) > room) stage--;
+    return stage;
+}
+
 /* the largest walk capacity whose buffers fit the LDS budget beside extra bytes */
 uint32_t max_walk_cap(size_t extra)
 {
@@ -3620,6 +3635,31 @@ uint32_t grown_cap(uint32_t cap, uint32_t need, uint32_t max_cap)
     return want > max_cap ? max_cap : want;
 }
 
+/* The walk capacity of a launch that walks the model's ray pairs from every origin, before
+   it: the longest half ray, by walk_max_kernel (its time is added to total_ms). */
+int pair_walk_cap(hipStream_t st, const DevBuffers &b, const KParams &kp, uint32_t max_cap, uint32_t &cap,
+                  double &total_ms)
+{
+    HIP_TRY(hipMemsetAsync(b.status, 0, 4 * sizeof(uint32_t), st));
+    HIP_TRY(hipMemcpyAsync(b.kp_dev, &kp, sizeof(KParams), hipMemcpyHostToDevice, st));
+    g_last_kernel_ms = 0.0;
+    timed(st, [&] {
+        hipLaunchKernelGGL(walk_max_kernel, dim3(kp.m.npoints, kp.m.hnrays), dim3(MGX_WAVE), 0, st, b.kp_dev,
+                           b.status + 3);
+    });
+    total_ms += g_last_kernel_ms;
+    HIP_TRY(hipGetLastError());
+    uint32_t h[4] = {0, 0, 0, 0};
+    HIP_TRY(hipMemcpyAsync(h, b.status, sizeof h, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    if (h[0] & ERR_NO_NEXT)
+        return mgx::fail(MGX_E_NO_NEXT, "a ray from an interior point found no valid next point");
+    if (h[3] > max_cap) return mgx::fail(MGX_E_RAY_LENGTH, "a ray needs more than %u walk steps", max_cap);
+    cap = (h[3] + 15) / 16 * 16;
+    cap = cap < 16 ? 16 : cap;
+    return MGX_OK;
+}
+
 /*
  * Launch loop of the solves: sets the LDS walk capacity, launches, and relaunches
  * with a larger capacity when a walk outgrew it.  With pair_walks (the launch walks
@@ -3643,30 +3683,13 @@ int launch_with_capacity(hipStream_t st, DevBuffers &b, KParams &kp, Launch laun
     if (hinted) {
         const bool have = cap_hint(key, cap);
         if (!have && pair_walks) {
-            HIP_TRY(hipMemsetAsync(b.status, 0, 4 * sizeof(uint32_t), st));
-            HIP_TRY(hipMemcpyAsync(b.kp_dev, &kp, sizeof(KParams), hipMemcpyHostToDevice, st));
-            g_last_kernel_ms = 0.0;
-            timed(st, [&] {
-                hipLaunchKernelGGL(walk_max_kernel, dim3(kp.m.npoints, kp.m.hnrays), dim3(MGX_WAVE), 0,
-                                   st, b.kp_dev, b.status + 3);
-            });
-            total_ms += g_last_kernel_ms;
-            HIP_TRY(hipGetLastError());
-            uint32_t h[4] = {0, 0, 0, 0};
-            HIP_TRY(hipMemcpyAsync(h, b.status, sizeof h, hipMemcpyDeviceToHost, st));
-            HIP_TRY(hipStreamSynchronize(st));
-            if (h[0] & ERR_NO_NEXT)
-                return mgx::fail(MGX_E_NO_NEXT, "a ray from an interior point found no valid next point");
-            if (h[3] > max_cap)
-                return mgx::fail(MGX_E_RAY_LENGTH, "a ray needs more than %u walk steps", max_cap);
-            cap = (h[3] + 15) / 16 * 16;
-            cap = cap < 16 ? 16 : cap;
+            if (int e = pair_walk_cap(st, b, kp, max_cap, cap, total_ms)) return e;
         }
         cap = cap > max_cap ? max_cap : cap;
     }
     for (;;) {
         kp.cap = cap;
-        kp.stage = stage_entries(cap, kp.m.nlines);
+        kp.stage = stage_entries(cap, 8 * (size_t)kp.m.nlines);
         kp.j_lds = j_in_lds(cap, kp.stage, kp.m.nfreqs, kp.m.nlines) ? 1 : 0;
         HIP_TRY(hipMemsetAsync(b.status, 0, 4 * sizeof(uint32_t), st));
         HIP_TRY(hipMemcpyAsync(b.kp_dev, &kp, sizeof(KParams), hipMemcpyHostToDevice, st));
@@ -3761,23 +3784,28 @@ uint32_t persistent_waves(K kernel, size_t lds, uint32_t work)
  * receives the dynamic LDS size; grid_of(lds) the persistent grid size.
  */
 template <typename Launch, typename Grid>
-int adjoint_launch(hipStream_t st, DevBuffers &b, KParams &kp, const WalkKey &key, double *d_eps,
+int adjoint_launch(hipStream_t st, DevBuffers &b, KParams &kp, const WalkKey &key, bool pair_walks, double *d_eps,
                    double *d_kap, double *d_iw, size_t PL, size_t per_wave_segments_factor,
                    Grid grid_of, Launch launch)
 {
     const uint32_t max_cap = max_walk_cap(8);
     uint32_t cap = 128;
-    (void)cap_hint(key, cap); /* the walks of the forward solve or image */
-    if (cap > max_cap) cap = max_cap;
     uint32_t capE = g_capE_hint;
     double total_ms = 0.0; /* kernel time summed over the launches */
     struct Report {
         double &t;
         ~Report() { g_last_kernel_ms = t; }
     } report{total_ms};
+    /* the walks of the forward solve or image, or else a length that a pass finds: a capacity
+       doubled until the walks fit would take LDS from the staged entries, also of the solves
+       that come after */
+    if (!cap_hint(key, cap) && pair_walks) {
+        if (int e = pair_walk_cap(st, b, kp, max_cap, cap, total_ms)) return e;
+    }
+    if (cap > max_cap) cap = max_cap;
     for (;;) {
         kp.cap = cap;
-        kp.stage = stage_entries(cap, kp.m.nlines);
+        kp.stage = stage_entries(cap, 0, 2 * sizeof(EntryGrad));
         const size_t lds = adjoint_lds_bytes(cap, kp.stage);
         const uint32_t grid = grid_of(lds);
         const size_t bytes = (size_t)grid * per_wave_segments_factor * capE * Tape::kRecord;
@@ -3833,7 +3861,7 @@ int run_J_adjoint_k(hipStream_t st, DevBuffers &b, KParams &kp, const double *J_
     const uint32_t per = want >= kp.m.hnrays ? 1 : (uint32_t)((kp.m.hnrays + want - 1) / want);
     const uint32_t items = P * ((kp.m.hnrays + per - 1) / per);
     return adjoint_launch(
-        st, b, kp, walk_key(kp.m), d_eps, d_kap, d_iw, (size_t)P * kp.m.nlines, 2,
+        st, b, kp, walk_key(kp.m), true, d_eps, d_kap, d_iw, (size_t)P * kp.m.nlines, 2,
         [&](size_t lds) { return persistent_waves(kern, lds, items); },
         [&](size_t lds, uint32_t grid, uint32_t capE) {
             timed(st, [&] {
@@ -3975,7 +4003,7 @@ uint32_t batch_grid(uint32_t wps, size_t lds)
     return persistent_waves(feautrier_batch_kernel<A, PR, 3>, lds, 0xffffffffu);
 }
 
-uint32_t batch_stage(const mgx_batch &B) { return stage_entries(B.cap, B.maxL); }
+uint32_t batch_stage(const mgx_batch &B) { return stage_entries(B.cap, 8 * (size_t)B.maxL); }
 
 bool batch_j_lds(const mgx_batch &B) { return j_in_lds(B.cap, batch_stage(B), B.maxF, B.maxL); }
 
@@ -4786,7 +4814,7 @@ static int image_adjoint_entry(const mgx_model *model, const mgx_options *opts,
     const WalkKey ikey = image_key(*model, raydir, nx, ny);
     auto run = [&](auto kern) {
         return adjoint_launch(
-            st, b, kp, ikey, d_eps, d_kap, d_iw, PL, 1,
+            st, b, kp, ikey, false, d_eps, d_kap, d_iw, PL, 1,
             [&](size_t lds) {
                 const uint32_t ppw = model->nfreqs <= 32 ? 2 : 1; /* pixels per wave */
                 return persistent_waves(kern, lds, (nx * ny + ppw - 1) / ppw);

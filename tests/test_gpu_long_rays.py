@@ -126,3 +126,34 @@ def test_interpolation_count_overflow_is_its_own_error():
         solver.feautrier_forward(dm, op)
     out = solver.feautrier_forward(dm, m.options())
     assert np.isfinite(out["J"].cpu().numpy()).all()
+
+
+@pytest.mark.parametrize("npoints,nlines", [(1508, 1), (1560, 3), (1640, 3), (2000, 5), (3340, 3), (3358, 17)])
+def test_blended_lines_on_long_chains(npoints, nlines):
+    """Where the walk buffers fill a half or all of a CU's LDS the sweeps stage fewer entries
+    and window lines at a time, at the last steps that are accepted three entries and one
+    line: forward (1e-10) and gradient of J (1e-9 relative, a tenth of that of the largest
+    where contributions of both signs cancel, as the other gradient tests)."""
+    import torch
+
+    from magritte_amd import solver
+    from oracle import oracle
+
+    print(f"[long rays] chain P={npoints}, {nlines} lines", flush=True)
+    m = models.model_line_1d(npoints=npoints, nquads=1)
+    if nlines > 1:
+        ld = models.linedata_blended(115.0e9, [1.5e-6 * (k + 1) for k in range(nlines - 1)], A=1.0e-7)
+        m.set_lines([ld], 1)
+        m.finalize()
+    op = m.options()
+    dm = solver.DeviceModel(m)
+    out = solver.feautrier_forward(dm, op, with_u=False)
+    _, J_r, lam_r = oracle.solve(m, op, with_u=False, nthreads=16)
+    assert _rel(out["J"].cpu().numpy(), J_r) < 1e-10
+    assert _rel(out["lambda_diag"].cpu().numpy(), lam_r) < 1e-10
+    Jb = np.random.default_rng(3).standard_normal((m.npoints, m.nfreqs))
+    got = solver.feautrier_adjoint(dm, op, torch.from_numpy(Jb))
+    for name, g, r in zip(("d_eps", "d_kap"), got, oracle.J_adjoint(m, op, Jb, nthreads=16)):
+        err = np.abs(g.cpu().numpy() - r) / (np.abs(r) + 0.1 * np.abs(r).max())
+        print(f"  {name} worst {err.max():.2e}", flush=True)
+        assert err.max() < 1e-9
