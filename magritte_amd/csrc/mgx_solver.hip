@@ -1166,9 +1166,9 @@ __device__ inline void ring_push(BandRing<NB> &r, double h, double g, uint32_t n
  * solver.tpp:1565-1757): I <- e^-dt I + expm1(-dt)/dt (S_c - S_n (1 + dt)) + S_c - S_n
  * per segment, from the outer entry (current) to the inner one (next) on both halves,
  * with dt = max(min_dtau, dtau) and the reference's float expf / expm1f; sw.Y carries
- * I and sw.prev_dtau the last dt.
+ * I and sw.prev_dtau the last dt.  WIDE: the bins of an image, see window_lines_of.
  */
-template <int APPROX, int PREC, int METHOD, int NB, bool TAPE = false>
+template <int APPROX, int PREC, int METHOD, int NB, bool TAPE = false, bool WIDE = false>
 __device__ __forceinline__ void staged_sweep(const KParams &kp, unsigned char *smem, const GroupRay *g,
                                              bool backward, double freq, bool active, StagedEntry *chunk,
                                              double min_dtau, Sweep &sw, BandRing<NB> &ring,
@@ -1205,7 +1205,7 @@ __device__ __forceinline__ void staged_sweep(const KParams &kp, unsigned char *s
             PointEC ec_in = {0.0, 0.0, false};
             double dtau, S_out, S_in, raw, dop;
             const bool on = k0 + j <= n;
-            staged_segment<APPROX, PREC>(kp, g, lines, window_lines(count), bin, eo, ei, on, out, ec_out, ec_in, dtau,
+            staged_segment<APPROX, PREC, WIDE>(kp, g, lines, window_lines(count), bin, eo, ei, on, out, ec_out, ec_in, dtau,
                                          S_out, S_in, raw, dop);
             if (!on) continue;
             if constexpr (METHOD == METHOD_TAU) {
@@ -2636,7 +2636,7 @@ __device__ bool image_pixels(const KParams &kp, const ImageFrame &fr, uint32_t p
         count_entries<true>(kp, smem, g);
         Sweep sw;
         BandRing<0> ring;
-        staged_sweep<APPROX, PREC, METHOD, 0>(kp, smem, g, false, freq, active, chunk, 0.0, sw, ring);
+        staged_sweep<APPROX, PREC, METHOD, 0, false, true>(kp, smem, g, false, freq, active, chunk, 0.0, sw, ring);
         if (!active) continue;
         double val;
         if constexpr (KIND == IMG_OPTICAL_DEPTH) {
@@ -3145,7 +3145,7 @@ __global__ __launch_bounds__(MGX_WAVE, IW ? 2 : MGX_J_ADJOINT_WAVES_PER_SIMD) vo
                     const Tape tape = {st_wave + (size_t)(back ? capE : 0) * Tape::kRecord, capE};
                     const RevCentre rc = {c.u, mu_c, lam_c, -lam_c * (back ? c.dd_bw : c.dd_fw),
                                           !back && S1 == 0};
-                    reverse_half<APPROX, PREC, IW>(kp, smem, g, back, freq, active, chunk, sums, tape,
+                    reverse_half<APPROX, PREC, IW, false>(kp, smem, g, back, freq, active, chunk, sums, tape,
                                                    pass == 1 ? I_b : I_f, rc, out);
                 }
             }
@@ -3215,13 +3215,13 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_IMAGE_ADJOINT_WAVES_PER_SIMD) void im
             Sweep fw;
             BandRing<0> ring;
             double I_f = 0.0;
-            staged_sweep<APPROX, PREC, METHOD_FEAUTRIER, 0, true>(kp, smem, g, false, freq, active, chunk, 0.0, fw,
-                                                                  ring, &tape, &I_f);
+            staged_sweep<APPROX, PREC, METHOD_FEAUTRIER, 0, true, true>(kp, smem, g, false, freq, active, chunk, 0.0,
+                                                                        fw, ring, &tape, &I_f);
             CentreRow c = {0.0, 0.0, 1.0, 0.0, 0.0};
             if (active) c = centre_row<PREC>(kp, w.ip, freq, w.shift_centre, true, false, fw, fw);
             const double lam_c = ubar * c.xc;
             const RevCentre rc = {c.u, ubar * c.xc * rcp(c.Dc), lam_c, -lam_c * c.dd_fw, true};
-            reverse_half<APPROX, PREC, IW>(kp, smem, g, false, freq, active, chunk, sums, tape, I_f, rc, out);
+            reverse_half<APPROX, PREC, IW, true>(kp, smem, g, false, freq, active, chunk, sums, tape, I_f, rc, out);
         }
     }
 }

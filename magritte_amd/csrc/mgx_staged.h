@@ -364,10 +364,36 @@ struct WindowSum {
     double a, b, c;
 };
 
+/* the lines at a segment's ends, or at an entry */
+template <int PREC, bool ENTRY>
+__device__ __forceinline__ void window_line(const KParams &kp, const StagedEntry *eo, const StagedEntry *ei,
+                                            double f, uint32_t l, WindowLine &w)
+{
+    w.f = f;
+    line_at<PREC, ENTRY>(kp, ENTRY ? ei : eo, l, w.iw_o, w.kap_o, w.src_o);
+    if (ENTRY) {
+        w.iw_i = w.kap_i = w.src_i = 0.0;
+    } else {
+        line_at<PREC, false>(kp, ei, l, w.iw_i, w.kap_i, w.src_i);
+    }
+    w.l = l;
+}
+
+/* a group whose bins' windows lie apart: their union is this many times a bin's own window,
+   in a list of more lines than two rounds.  64^2 images of a 7^3 wind, 31 bins over 2.2e-4 of
+   a line's frequency, lines 2e-6 apart, all bins together and each by itself: 20 lines 0.72
+   and 0.92 ms, 40 lines 1.29 and 1.11, 100 lines 2.60 and 1.16, 300 lines 3.9 and 1.5 (their
+   gradients 2.4 and 2.9, 5.1 and 3.6, 13.0 and 3.9, 18.5 and 5.0). */
+constexpr double kApart = 4.0;
+constexpr uint32_t kApartLines = 2 * kWindowLines;
+
 /* Stages the lines in the windows round by round and hands each to take(line, its index,
-   whether it is in the bin's window), in the sorted order; mine marks the bins that have a
-   window here.  All lanes of the wave call this together, and take too. */
-template <int APPROX, int PREC, bool ENTRY, typename Take>
+   whether it is in the bin's window, whether it is the same for all bins of the group), in the
+   sorted order; mine marks the bins that have a window here.  All lanes of the wave call this
+   together, and take too.  WIDE: the group's bins need not belong to one line.  Where their
+   windows lie apart, most lines of the union are in the windows of a few bins each, and every
+   bin takes its own window's lines at the same time instead. */
+template <int APPROX, int PREC, bool ENTRY, bool WIDE, typename Take>
 __device__ __forceinline__ void window_lines_of(const KParams &kp, const GroupRay *g, WindowLine *lines,
                                                 uint32_t nw, const StagedEntry *eo, const StagedEntry *ei,
                                                 double f_o, double f_i, bool mine, Take take)
@@ -396,11 +422,28 @@ __device__ __forceinline__ void window_lines_of(const KParams &kp, const GroupRa
             right_all = r1 + W1;
         }
     }
+    if constexpr (WIDE && APPROX == MGX_APPROX_CLOSE_LINES) {
+        if (m.nlines > kApartLines && __ballot(mine && right_all - left_all > kApart * (right - left))) {
+            uint32_t s = 0, end = 0;
+            if (mine) {
+                s = lower_bound_d(m.sorted_line, m.nlines, left);
+                end = upper_bound_d(m.sorted_line, m.nlines, right);
+            }
+#pragma unroll 1
+            for (; __ballot(s < end); s++) {
+                WindowLine w = {};
+                const bool here = s < end;
+                if (here)
+                    window_line<PREC, ENTRY>(kp, eo, ei, gld(&m.sorted_line[s]), gld(&m.sorted_line_map[s]), w);
+                take(&w, w.l, here, false);
+            }
+            return;
+        }
+    }
 #pragma unroll 1
     for (uint32_t s0 = 0; s0 < m.nlines; s0 += nw) {
         bool in = false;
         double f = 0.0;
-        uint32_t l = 0;
         if (any && q < nw && s0 + q < m.nlines) {
             f = APPROX == MGX_APPROX_CLOSE_LINES ? gld(&m.sorted_line[s0 + q]) : gld(&m.line[s0 + q]);
             in = !(f < left_all) && !(right_all < f);
@@ -409,16 +452,9 @@ __device__ __forceinline__ void window_lines_of(const KParams &kp, const GroupRa
         if (b == 0) continue;
         __syncthreads();
         if (in) {
-            l = APPROX == MGX_APPROX_CLOSE_LINES ? gld(&m.sorted_line_map[s0 + q]) : s0 + q;
             WindowLine w;
-            w.f = f;
-            line_at<PREC, ENTRY>(kp, ENTRY ? ei : eo, l, w.iw_o, w.kap_o, w.src_o);
-            if (ENTRY) {
-                w.iw_i = w.kap_i = w.src_i = 0.0;
-            } else {
-                line_at<PREC, false>(kp, ei, l, w.iw_i, w.kap_i, w.src_i);
-            }
-            w.l = l;
+            window_line<PREC, ENTRY>(kp, eo, ei, f,
+                                     APPROX == MGX_APPROX_CLOSE_LINES ? gld(&m.sorted_line_map[s0 + q]) : s0 + q, w);
             lines[q] = w;
         }
         __syncthreads();
@@ -430,20 +466,20 @@ __device__ __forceinline__ void window_lines_of(const KParams &kp, const GroupRa
             all &= all - 1;
             const WindowLine *w = lines + i;
             const bool here = mine && ((set >> i) & 1) != 0 && !(w->f < left) && !(right < w->f);
-            take(w, w->l, here);
+            take(w, w->l, here, true);
         }
     }
     __syncthreads();
 }
 
-template <int APPROX, int PREC, bool ENTRY>
+template <int APPROX, int PREC, bool ENTRY, bool WIDE>
 __device__ __forceinline__ WindowSum window_sum(const KParams &kp, const GroupRay *g, WindowLine *lines,
                                                 uint32_t nw, const StagedEntry *eo, const StagedEntry *ei,
                                                 double f_o, double f_i, bool mine)
 {
     WindowSum r = {0.0, ENTRY ? kp.op.min_opacity : 0.0, 0.0};
-    window_lines_of<APPROX, PREC, ENTRY>(
-        kp, g, lines, nw, eo, ei, f_o, f_i, mine, [&](const WindowLine *w, uint32_t, bool in) {
+    window_lines_of<APPROX, PREC, ENTRY, WIDE>(
+        kp, g, lines, nw, eo, ei, f_o, f_i, mine, [&](const WindowLine *w, uint32_t, bool in, bool) {
             if (!in) return;
             if (ENTRY) {
                 const double prof = gaussian<PREC>(w->iw_o, f_i - w->f);
@@ -475,7 +511,7 @@ struct BinLine {
 /* emissivity, opacity and own profile value of an entry at a bin's frequency; phi is
    NaN where several lines contribute, 0 where none does.  All lanes of the wave call
    this together; those that want a value pass need. */
-template <int APPROX, int PREC>
+template <int APPROX, int PREC, bool WIDE>
 __device__ __forceinline__ void staged_eta_chi(const KParams &kp, const GroupRay *g, WindowLine *lines, uint32_t nw,
                                                const BinLine &bin, const StagedEntry *e, bool need,
                                                double &eta, double &chi, double &phi)
@@ -494,7 +530,7 @@ __device__ __forceinline__ void staged_eta_chi(const KParams &kp, const GroupRay
         chi = kp.op.min_opacity + phi * e->kap;
     }
     if (__ballot(w == 2)) {
-        const WindowSum s = window_sum<APPROX, PREC, true>(kp, g, lines, nw, e, e, f, f, w == 2);
+        const WindowSum s = window_sum<APPROX, PREC, true, WIDE>(kp, g, lines, nw, e, e, f, f, w == 2);
         if (w == 2) {
             eta = s.a;
             chi = s.b;
@@ -512,7 +548,7 @@ __device__ __forceinline__ void staged_eta_chi(const KParams &kp, const GroupRay
  * sweeps drop them): raw is the depth before a line-integrated one is clamped, dop
  * d depth / d mean opacity of a segment with the own line alone.
  */
-template <int APPROX, int PREC>
+template <int APPROX, int PREC, bool WIDE>
 __device__ __forceinline__ void staged_segment(const KParams &kp, const GroupRay *g, WindowLine *lines, uint32_t nw,
                                                const BinLine &bin, const StagedEntry *eo,
                                                const StagedEntry *ei, bool on, OuterEnd &out, PointEC &ec_out,
@@ -550,7 +586,7 @@ __device__ __forceinline__ void staged_segment(const KParams &kp, const GroupRay
     }
     if (__ballot(seg >= SEG_LANE)) {
         if (__ballot(seg == SEG_LANE)) {
-            const WindowSum v = window_sum<APPROX, PREC, false>(kp, g, lines, nw, eo, ei, out.f, in.f, seg == SEG_LANE);
+            const WindowSum v = window_sum<APPROX, PREC, false, WIDE>(kp, g, lines, nw, eo, ei, out.f, in.f, seg == SEG_LANE);
             if (seg == SEG_LANE) {
                 double d = raw = v.a;
                 if (APPROX == MGX_APPROX_CLOSE_LINES && -bound < d) d = (bound < d) ? d : bound;
@@ -562,8 +598,8 @@ __device__ __forceinline__ void staged_segment(const KParams &kp, const GroupRay
         }
         double phi;
         const bool trap = seg == SEG_TRAP;
-        staged_eta_chi<APPROX, PREC>(kp, g, lines, nw, bin, eo, trap && !ec_out.valid, ec_out.eta, ec_out.chi, phi);
-        staged_eta_chi<APPROX, PREC>(kp, g, lines, nw, bin, ei, trap, ec_in.eta, ec_in.chi, phi);
+        staged_eta_chi<APPROX, PREC, WIDE>(kp, g, lines, nw, bin, eo, trap && !ec_out.valid, ec_out.eta, ec_out.chi, phi);
+        staged_eta_chi<APPROX, PREC, WIDE>(kp, g, lines, nw, bin, ei, trap, ec_in.eta, ec_in.chi, phi);
         if (trap) {
             ec_in.valid = true;
             S_out = ec_out.eta * rcp(ec_out.chi);

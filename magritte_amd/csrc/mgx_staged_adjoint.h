@@ -157,12 +157,12 @@ __device__ __forceinline__ bool depth_clamped(double raw, double bound)
 }
 
 /*
- * Reverse of window_sum: the lines of the bins' windows, in rounds of nw lines a group has
- * staged in LDS.  ENTRY false: the segment eo - ei with adjoints a_bar of its depth and
+ * Reverse of window_sum: the lines of the bins' windows, as window_lines_of hands them
+ * on.  ENTRY false: the segment eo - ei with adjoints a_bar of its depth and
  * b_bar, c_bar of its outer and inner source, and the window's sums v (depth unclamped);
  * ENTRY true: the entry ei with adjoints a_bar, b_bar of emissivity and opacity.
  */
-template <int APPROX, int PREC, bool ENTRY, bool IW>
+template <int APPROX, int PREC, bool ENTRY, bool IW, bool WIDE>
 __device__ __forceinline__ void window_bwd(const KParams &kp, const GroupRay *g, WindowLine *lines, uint32_t nw,
                                            const StagedEntry *eo, const StagedEntry *ei, double f_o, double f_i,
                                            bool mine, const WindowSum &v, double a_bar, double b_bar,
@@ -181,8 +181,8 @@ __device__ __forceinline__ void window_bwd(const KParams &kp, const GroupRay *g,
         sc = c_bar * rd;
         sa = clamped ? 0.0 : a_bar - sb * (v.b * rd) - sc * (v.c * rd);
     }
-    window_lines_of<APPROX, PREC, ENTRY>(
-        kp, g, lines, nw, eo, ei, f_o, f_i, mine, [&](const WindowLine *w, uint32_t l, bool in) {
+    window_lines_of<APPROX, PREC, ENTRY, WIDE>(
+        kp, g, lines, nw, eo, ei, f_o, f_i, mine, [&](const WindowLine *w, uint32_t l, bool in, bool shared) {
             EntryGrad o = {0.0, 0.0, 0.0, 0.0}, i = {0.0, 0.0, 0.0, 0.0};
             if (in && ENTRY) {
                 const double prof = gaussian<PREC>(w->iw_o, f_i - w->f);
@@ -195,10 +195,14 @@ __device__ __forceinline__ void window_bwd(const KParams &kp, const GroupRay *g,
                                                   kp.op.min_opacity, dop);
                 line_bwd<IW>(*w, f_o, f_i, ei->dz, dop, sa + sb * w->src_o + sc * w->src_i, sb * d, sc * d, o, i);
             }
-            const bool any_o = ENTRY ? false : group_total<IW>(o);
-            const bool any_i = group_total<IW>(i);
-            if (q == 0 && any_o) entry_scatter<IW>(kp, out, eo, l, 0.0, w->kap_o, w->src_o, o);
-            if (q == 0 && any_i) {
+            /* a line that the bins share goes to the points once, a bin's own by itself */
+            bool any_o = !ENTRY && in, any_i = in;
+            if (shared) {
+                any_o = !ENTRY && group_total<IW>(o) && q == 0;
+                any_i = group_total<IW>(i) && q == 0;
+            }
+            if (any_o) entry_scatter<IW>(kp, out, eo, l, 0.0, w->kap_o, w->src_o, o);
+            if (any_i) {
                 if (ENTRY) /* src_o is the emissivity */
                     entry_scatter<IW>(kp, out, ei, l, w->src_o, w->kap_o, 0.0, i);
                 else
@@ -257,7 +261,7 @@ struct EntryBar {
     bool have;
 };
 
-template <int APPROX, int PREC, bool IW>
+template <int APPROX, int PREC, bool IW, bool WIDE>
 __device__ __forceinline__ void reverse_half(const KParams &kp, unsigned char *smem, const GroupRay *g,
                                              bool backward, double freq, bool active, StagedEntry *chunk,
                                              EntryGrad *sums, const Tape &tape, double I_b,
@@ -359,12 +363,12 @@ __device__ __forceinline__ void reverse_half(const KParams &kp, unsigned char *s
             if (__ballot(seg >= SEG_LANE)) {
                 const bool gen = seg == SEG_LANE, trap = seg == SEG_TRAP;
                 if (__ballot(gen)) {
-                    const WindowSum v = window_sum<APPROX, PREC, false>(kp, g, lines, nw, eo, ei, f_o, f_i, gen);
-                    window_bwd<APPROX, PREC, false, IW>(kp, g, lines, nw, eo, ei, f_o, f_i, gen, v, dbar, so, si,
+                    const WindowSum v = window_sum<APPROX, PREC, false, WIDE>(kp, g, lines, nw, eo, ei, f_o, f_i, gen);
+                    window_bwd<APPROX, PREC, false, IW, WIDE>(kp, g, lines, nw, eo, ei, f_o, f_i, gen, v, dbar, so, si,
                                                         out);
                 }
-                staged_eta_chi<APPROX, PREC>(kp, g, lines, nw, bin, eo, trap, eb.eta, eb.chi, eb.phi);
-                staged_eta_chi<APPROX, PREC>(kp, g, lines, nw, bin, ei, trap && !in.have, in.eta, in.chi, in.phi);
+                staged_eta_chi<APPROX, PREC, WIDE>(kp, g, lines, nw, bin, eo, trap, eb.eta, eb.chi, eb.phi);
+                staged_eta_chi<APPROX, PREC, WIDE>(kp, g, lines, nw, bin, ei, trap && !in.have, in.eta, in.chi, in.phi);
                 if (trap) {
                     eb.have = in.have = true;
                     const double ro = rcp(eb.chi), ri = rcp(in.chi);
@@ -389,7 +393,7 @@ __device__ __forceinline__ void reverse_half(const KParams &kp, unsigned char *s
                 if (__ballot(multi)) {
                     const double f = freq * se->shift;
                     const WindowSum none = {0.0, 0.0, 0.0};
-                    window_bwd<APPROX, PREC, true, IW>(kp, g, lines, nw, se, se, f, f, multi, none, e.eta_bar,
+                    window_bwd<APPROX, PREC, true, IW, WIDE>(kp, g, lines, nw, se, se, f, f, multi, none, e.eta_bar,
                                                        e.chi_bar, 0.0, out);
                 }
                 EntryGrad t = here ? e.s : EntryGrad{0.0, 0.0, 0.0, 0.0};

@@ -90,3 +90,81 @@ def test_adjoint_ray_pair_items(n_edge, nrays):
     for name, a, b in zip(("d_eps", "d_kap"), got, oracle.J_adjoint(m, op, J_bar)):
         a, b = np.asarray(a.cpu()), np.asarray(b)
         assert np.all(np.abs(a - b) <= 1e-9 * np.abs(b) + 1e-10 * np.abs(b).max()), name
+
+
+@pytest.mark.parametrize("nlines,separation", [(63, 1.5e-6), (64, 1.5e-6), (65, 1.5e-6), (130, 1.0e-5),
+                                               (130, 1.0e-4)])
+def test_windows_in_long_lists(nlines, separation):
+    """lists around the length from which the windows' first line is searched for, windows
+    with many, a few and one of their lines"""
+    print(f"[staged] {nlines} lines {separation} apart", flush=True)
+    m = models.model_wind(n_edge=4, nrays=12, nquads=3, v_out=1.5e3)
+    m.set_lines([models.linedata_blended(115.0e9, [separation * (k + 1) for k in range(nlines - 1)], A=1.0e-7)], 3)
+    m.finalize()
+    _check(m, m.options())
+
+
+def _two_species(n_edge=5):
+    """blended lines of two species, the second one's below the first's: the lines are not in
+    ascending order"""
+    m = models.model_wind(n_edge=n_edge, nrays=12, nquads=5, v_out=1.5e3)
+    a = models.linedata_blended(115.0e9, [2.0e-6, 5.0e-6], A=1.0e-7, num=1)
+    b = models.linedata_blended(115.0e9 * (1 - 8.0e-6), [1.0e-6, 9.0e-6], A=1.0e-7, num=1)
+    m.set_lines([a, b], 5)
+    m.finalize()
+    assert np.any(np.diff(m.line) < 0)
+    return m
+
+
+@pytest.mark.parametrize("approx", [_abi.APPROX_NONE, _abi.APPROX_ONE_LINE, _abi.APPROX_CLOSE_LINES])
+def test_lines_out_of_order(approx):
+    import torch
+
+    from magritte_amd import solver
+    from oracle import oracle
+
+    print(f"[staged] two species, approx {approx}", flush=True)
+    m = _two_species()
+    op = m.options(approx=approx)
+    _check(m, op)
+    J_bar = np.random.Generator(np.random.PCG64(8)).standard_normal((m.npoints, m.nfreqs))
+    got = solver.feautrier_adjoint(solver.DeviceModel(m), op, torch.from_numpy(J_bar))
+    for name, a, b in zip(("d_eps", "d_kap"), got, oracle.J_adjoint(m, op, J_bar)):
+        a, b = np.asarray(a.cpu()), np.asarray(b)
+        assert np.all(np.abs(a - b) <= 1e-9 * np.abs(b) + 1e-10 * np.abs(b).max()), name
+
+
+@pytest.mark.parametrize("kind", ["apart", "close", "two species"])
+@pytest.mark.parametrize("nfreqs", [3, 31, 70])
+@pytest.mark.parametrize("approx", [_abi.APPROX_NONE, _abi.APPROX_CLOSE_LINES])
+def test_images_with_many_lines(kind, nfreqs, approx):
+    """image bins whose windows lie apart (each takes its own lines) or close together (they
+    share the group's): intensities, optical depths (1e-10) and gradients, the inverse
+    widths' too (bars of their tests)"""
+    import torch
+
+    from magritte_amd import solver
+    from oracle import oracle
+
+    print(f"[staged] image {kind} {nfreqs} bins approx {approx}", flush=True)
+    if kind == "two species":
+        m = _two_species(6)
+    else:
+        m = models.model_wind(n_edge=6, nrays=12, nquads=3, v_out=1.5e3)
+        m.set_lines([models.linedata_blended(115.0e9, [2.0e-6 * (k + 1) for k in range(79)], A=1.0e-7)], 3)
+        m.finalize()
+    half = 2.0e-6 if kind == "close" else 1.0e-4
+    fr = m.image_frequencies(m.line[0] * (1 + 8.0e-5 - half), m.line[0] * (1 + 8.0e-5 + half), nfreqs)
+    if kind == "two species":
+        fr = m.image_frequencies(m.line[0] * (1 - 1.0e-4), m.line[0] * (1 + 1.0e-4), nfreqs)
+    rd, op, d = np.array([0.3, -0.5, 0.81]), m.options(approx=approx), solver.DeviceModel(m)
+    for f_d, f_o in ((solver.image_new, oracle.image_new),
+                     (solver.image_optical_depth_new, oracle.image_optical_depth_new)):
+        got, want = f_d(d, op, rd, 9, 7, fr)[0].cpu().numpy(), f_o(m, op, rd, 9, 7, fr)[0]
+        assert np.max(np.abs(got - want) / np.maximum(np.abs(want), 1e-300)) < 1e-10
+    I_bar = np.random.Generator(np.random.PCG64(9)).standard_normal((63, nfreqs))
+    got = solver.image_adjoint(d, op, rd, 9, 7, fr, torch.from_numpy(I_bar), want_iw=True)
+    want = oracle.image_adjoint(m, op, rd, 9, 7, I_bar, fr, want_iw=True)
+    for name, a, b, rel in zip(("d_eps", "d_kap", "d_iw"), got, want, (1e-9, 1e-9, 1e-6)):
+        a, b = np.asarray(a.cpu()), np.asarray(b)
+        assert np.all(np.abs(a - b) <= rel * np.abs(b) + 0.1 * rel * np.abs(b).max()), name
