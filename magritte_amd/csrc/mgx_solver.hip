@@ -45,6 +45,7 @@
 
 #include "mgx.h"
 #include "mgx_constants.h"
+#include "mgx_call_buffer.h"
 #include "mgx_error.h"
 #include "mgx_fmath.h"
 #include "mgx_fmath_ref.h"
@@ -3428,27 +3429,26 @@ int prepare(const mgx_model *m, const mgx_options *op, hipStream_t st, DevBuffer
         return prepare_tables(m, op, st, b, kp);
     }
     const auto rnd = [](size_t n) { return (n + 255) & ~(size_t)255; };
-    size_t need = rnd(PL * sizeof(double4)) + rnd(P * sizeof(PointRec)) +
-                  rnd(P * sizeof(PointIdx)) + rnd(4 * sizeof(uint32_t)) +
-                  rnd(sizeof(KParams)) + rnd(sizeof(ImageFrame)) + rnd(sp ? sp->bytes : 0);
+    const size_t need = rnd(PL * sizeof(double4)) + rnd(P * sizeof(PointRec)) +
+                        rnd(P * sizeof(PointIdx)) + rnd(4 * sizeof(uint32_t)) +
+                        rnd(sizeof(KParams)) + rnd(sizeof(ImageFrame));
     b.ws_lock = std::unique_lock<std::mutex>(g_prep_mutex);
     int dev = 0;
     HIP_TRY(hipGetDevice(&dev));
     if (dev < 0 || dev >= 64) return mgx::fail(MGX_E_ARG, "device index %d out of range", dev);
-    if (g_prep_bytes[dev] < need) {
-        /* the previous holder has returned, so nothing uses the old buffer */
-        if (g_prep[dev]) (void)hipFree(g_prep[dev]);
-        g_prep[dev] = nullptr;
-        g_prep_bytes[dev] = 0;
-        if (sp && sp->bytes > 0 && hipMalloc(&g_prep[dev], need) != hipSuccess) {
+    /* the previous holder has returned, so nothing uses the old buffer */
+    const mgx::Held held = mgx::hold(
+        g_prep[dev], g_prep_bytes[dev], need, rnd(sp ? sp->bytes : 0),
+        [](size_t n) {
+            void *q = nullptr;
+            if (hipMalloc(&q, n) == hipSuccess) return static_cast<unsigned char *>(q);
             (void)hipGetLastError();
-            g_prep[dev] = nullptr;
-            need -= rnd(sp->bytes);
-            *sp = RaySplit{m->hnrays, 1, 0, 0};
-        }
-        if (!g_prep[dev]) HIP_TRY(hipMalloc(&g_prep[dev], need));
-        g_prep_bytes[dev] = need;
-    }
+            return static_cast<unsigned char *>(nullptr);
+        },
+        [](unsigned char *q) { (void)hipFree(q); });
+    if (held == mgx::Held::None)
+        return mgx::fail(MGX_E_HIP, "hipMalloc of %zu bytes for a call's tables: out of memory", need);
+    if (held == mgx::Held::Needed) *sp = RaySplit{m->hnrays, 1, 0, 0};
     unsigned char *q = g_prep[dev];
     b.owned = false;
     b.lpack = reinterpret_cast<double4 *>(q);
