@@ -20,6 +20,14 @@ def _require_gpu():
     return torch
 
 
+def release_workspace():
+    """Gives back the device memory that the library keeps between calls (the solves' tables
+    and ray pairs' parts, the adjoints' tape); the next call allocates what it needs again.
+    Waits for calls in progress."""
+    _require_gpu()
+    _abi.lib().mgx_release_workspace()
+
+
 class DeviceModel:
     """Model arrays resident on the GPU plus the mgx_model view of them."""
 

@@ -168,3 +168,26 @@ def test_images_with_many_lines(kind, nfreqs, approx):
     for name, a, b, rel in zip(("d_eps", "d_kap", "d_iw"), got, want, (1e-9, 1e-9, 1e-6)):
         a, b = np.asarray(a.cpu()), np.asarray(b)
         assert np.all(np.abs(a - b) <= rel * np.abs(b) + 0.1 * rel * np.abs(b).max()), name
+
+
+def test_workspace_is_given_back():
+    """200 MB of parts are kept after a solve and given back on request"""
+    import torch
+
+    from magritte_amd import solver
+
+    print("[staged] release", flush=True)
+    m = models.model_wind(n_edge=16, nrays=48, nquads=31)
+    d, op = solver.DeviceModel(m), m.options(precision=_abi.PREC_MIXED)
+    solver.release_workspace()
+    before = torch.cuda.mem_get_info()[0]
+    J = torch.empty((m.npoints, m.nfreqs), dtype=torch.float64, device="cuda")
+    out = {"u": None, "J": J, "lambda_diag": None}
+    solver.feautrier_forward(d, op, out=out)
+    parts = 8 * m.npoints * m.hnrays * m.nfreqs
+    assert before - torch.cuda.mem_get_info()[0] >= parts
+    solver.release_workspace()
+    assert before - torch.cuda.mem_get_info()[0] < parts / 4
+    want = J.clone()
+    solver.feautrier_forward(d, op, out=out)
+    assert (J == want).all()
