@@ -591,11 +591,7 @@ __device__ inline float f_pow(float x, float y)
    difference of two float erf values (compute_dtau_single_line), which cancels
    in the line wings, so a one-ulp change of either value moves u by up to
    ~1e-3 relative there */
-template <int PREC>
-__device__ inline float f_erf(float x, const double *)
-{
-    return mgx_ref_erff(x);
-}
+__device__ inline float f_erf(float x) { return mgx_ref_erff(x); }
 
 __device__ inline double interp_linear(double a, double b, double t)
 {
@@ -784,7 +780,7 @@ __device__ void eta_chi_interp(const KParams &kp, const OwnLine &ol, uint32_t p1
 /* compute_dtau_single_line (solver.tpp:2374-2455).  Everything up to the
    float conversions follows the reference's operation order. */
 template <int PREC>
-__device__ double dtau_single_line(const KParams &kp, const double *erf_tab, double4 c, double4 cI,
+__device__ double dtau_single_line(const KParams &kp, double4 c, double4 cI,
                                    double4 n, double4 nI, double linefreq, double curr_freq,
                                    double next_freq, double curr_interp, double next_interp,
                                    double dz)
@@ -804,14 +800,14 @@ __device__ double dtau_single_line(const KParams &kp, const double *erf_tab, dou
     const double curr_pos = (linefreq - curr_freq) * avg_iw;
     const double diff_pos = next_pos - curr_pos;
     const double avg_op = (op_n + op_c) / 2.0;
-    const float erf_diff = f_erf<PREC>((float)next_pos, erf_tab) - f_erf<PREC>((float)curr_pos, erf_tab);
+    const float erf_diff = f_erf((float)next_pos) - f_erf((float)curr_pos);
     const double erfterm = avg_op * (double)erf_diff * (0.5 * rcp(diff_pos));
     return dz * fma(avg_iw, erfterm, kp.op.min_opacity);
 }
 
 /* compute_S_dtau_line_integrated<approx> (solver.tpp:1879-2111) */
 template <int APPROX, int PREC>
-__device__ void S_dtau_line_integrated(const KParams &kp, const double *erf_tab, const OwnLine &ol,
+__device__ void S_dtau_line_integrated(const KParams &kp, const OwnLine &ol,
                                        uint32_t cp, uint32_t np, uint32_t cpi, uint32_t npi,
                                        uint32_t lineidx, double currfreq, double nextfreq,
                                        double curr_interp, double next_interp, double dZ,
@@ -822,7 +818,7 @@ __device__ void S_dtau_line_integrated(const KParams &kp, const double *erf_tab,
     if (APPROX == MGX_APPROX_ONE_LINE) {
         const double4 c = lp(kp, cp, lineidx), cI = lp(kp, cpi, lineidx);
         const double4 n = lp(kp, np, lineidx), nI = lp(kp, npi, lineidx);
-        dtau = dtau_single_line<PREC>(kp, erf_tab, c, cI, n, nI, m.line[lineidx], currfreq,
+        dtau = dtau_single_line<PREC>(kp, c, cI, n, nI, m.line[lineidx], currfreq,
                                       nextfreq, curr_interp, next_interp, dZ);
         Scurr = interp_log<PREC>(c.w, cI.w, curr_interp);
         Snext = interp_log<PREC>(n.w, nI.w, next_interp);
@@ -857,7 +853,7 @@ __device__ void S_dtau_line_integrated(const KParams &kp, const double *erf_tab,
         linefreq = gld(&m.line[l]);
         const double4 c = lp(kp, cp, l), cI = lp(kp, cpi, l);
         const double4 n = lp(kp, np, l), nI = lp(kp, npi, l);
-        const double line_dtau = dtau_single_line<PREC>(kp, erf_tab, c, cI, n, nI, linefreq,
+        const double line_dtau = dtau_single_line<PREC>(kp, c, cI, n, nI, linefreq,
                                                         currfreq, nextfreq, curr_interp,
                                                         next_interp, dZ);
         const double Sc = interp_log<PREC>(c.w, cI.w, curr_interp);
@@ -907,7 +903,7 @@ __device__ __forceinline__ double2 dsm_ub(const KParams &kp, uint32_t p)
 }
 
 template <int APPROX, int PREC>
-__device__ inline bool segment(const KParams &kp, const double *erf_tab, const OwnLine &ol,
+__device__ inline bool segment(const KParams &kp, const OwnLine &ol,
                                const Entry &cu, const Entry &nx, double dZ, double freq,
                                uint32_t line, PointEC &ec_cu, PointEC &ec_nx, double &dtau,
                                double &S_cu, double &S_nx)
@@ -920,7 +916,7 @@ __device__ inline bool segment(const KParams &kp, const double *erf_tab, const O
     const double dshift_max = (b < a) ? b : a;
     const double cf = freq * cu.shift, nf = freq * nx.shift;
     if (dshift_abs > dshift_max) {
-        S_dtau_line_integrated<APPROX, PREC>(kp, erf_tab, ol, cu.nr, nx.nr, cu.nri, nx.nri, line,
+        S_dtau_line_integrated<APPROX, PREC>(kp, ol, cu.nr, nx.nr, cu.nri, nx.nri, line,
                                              cf, nf, cu.ifac, nx.ifac, dZ, du_c.y, du_n.y, dtau,
                                              S_cu, S_nx);
         return false;
@@ -1390,7 +1386,7 @@ __device__ inline void lam_merge(const KParams &kp, const LamBands &lb, size_t p
 
 template <int APPROX, int PREC, int METHOD = METHOD_FEAUTRIER, int NB = 0>
 __device__ __forceinline__ int solve_origin(const KParams &kp, uint32_t o, uint32_t rr0,
-                                            uint32_t rr1, unsigned char *smem, const double *s_erf,
+                                            uint32_t rr1, unsigned char *smem,
                                             double *u, bool with_lam, double *s_J, double *Jrow,
                                             bool j_atomic, double *s_L, ShortcharOut sc = {},
                                             LamBands lb = {})
@@ -1769,7 +1765,6 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void feautrier_
     mgx_ref_tables_init();
     const KParams &kp = *kpp;
     extern __shared__ unsigned char smem[];
-    const double *s_erf = nullptr; /* erf needs no table */
     const mgx_model &m = kp.m;
     const uint32_t o = blockIdx.x;
     const uint32_t lane = threadIdx.x;
@@ -1789,7 +1784,7 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void feautrier_
     for (uint32_t rr = rr0; rr < rr1; rr += step) {
         const size_t row = split ? (size_t)rr * m.npoints + o : o;
         for (uint32_t i = lane; i < L + (s_J ? F : 0); i += MGX_WAVE) s_L[i] = 0.0;
-        if (solve_origin<APPROX, PREC>(kp, o, rr, rr + step, smem, s_erf, u, lam != nullptr, s_J,
+        if (solve_origin<APPROX, PREC>(kp, o, rr, rr + step, smem, u, lam != nullptr, s_J,
                                        s_J || !J ? nullptr : J + row * F, false, s_L))
             return;
         if (Jline) {
@@ -1850,7 +1845,6 @@ __global__ __launch_bounds__(MGX_WAVE, 2) void feautrier_bands_kernel(
     mgx_ref_tables_init();
     const KParams &kp = *kpp;
     extern __shared__ unsigned char smem[];
-    const double *s_erf = nullptr; /* erf needs no table */
     const mgx_model &m = kp.m;
     const uint32_t o = blockIdx.x;
     const uint32_t lane = threadIdx.x;
@@ -1867,7 +1861,7 @@ __global__ __launch_bounds__(MGX_WAVE, 2) void feautrier_bands_kernel(
     if (lane == 0)
         for (uint32_t l = 0; l < L; l++) lb.count[(size_t)o * L + l] = 0;
     if (solve_origin<APPROX, PREC, METHOD_FEAUTRIER, MGX_MAX_OFF_DIAG>(
-            kp, o, 0, m.hnrays, smem, s_erf, u, true, s_J, J + (size_t)o * F, false, s_L, {}, lb))
+            kp, o, 0, m.hnrays, smem, u, true, s_J, J + (size_t)o * F, false, s_L, {}, lb))
         return;
     if (s_J)
         for (uint32_t i = lane; i < F; i += MGX_WAVE) J[(size_t)o * F + i] = s_J[i];
@@ -1882,7 +1876,6 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void shortchar_
     mgx_ref_tables_init();
     const KParams &kp = *kpp;
     extern __shared__ unsigned char smem[];
-    const double *s_erf = nullptr; /* erf needs no table */
     const mgx_model &m = kp.m;
     const uint32_t o = blockIdx.x;
     const uint32_t lane = threadIdx.x;
@@ -1902,7 +1895,7 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void shortchar_
     for (uint32_t rr = rr0; rr < rr1; rr += step) {
         const size_t row = split ? (size_t)rr * m.npoints + o : o;
         for (uint32_t i = lane; i < L + (s_J ? F : 0); i += MGX_WAVE) s_L[i] = 0.0;
-        if (solve_origin<APPROX, PREC, METHOD_SHORTCHAR>(kp, o, rr, rr + step, smem, s_erf, u, lam != nullptr,
+        if (solve_origin<APPROX, PREC, METHOD_SHORTCHAR>(kp, o, rr, rr + step, smem, u, lam != nullptr,
                                                          s_J, s_J || !J ? nullptr : J + row * F, false, s_L,
                                                          sc))
             return;
@@ -1923,12 +1916,11 @@ __global__ __launch_bounds__(MGX_WAVE, MGX_SOLVE_WAVES_PER_SIMD) void feautrier_
     mgx_ref_tables_init();
     const KParams &kp = *kpp;
     extern __shared__ unsigned char smem[];
-    const double *s_erf = nullptr; /* erf needs no table */
     const uint32_t o = blockIdx.x;
     double *s_L = reinterpret_cast<double *>(smem + acc_lds_offset(kp.cap, kp.stage));
     ShortcharOut sc{nullptr, v, 0.0};
     const uint32_t rr0 = blockIdx.y * per, rr1 = rr0 + per < kp.m.hnrays ? rr0 + per : kp.m.hnrays;
-    solve_origin<APPROX, PREC, METHOD_UV>(kp, o, rr0, rr1, smem, s_erf, u, false, nullptr,
+    solve_origin<APPROX, PREC, METHOD_UV>(kp, o, rr0, rr1, smem, u, false, nullptr,
                                           nullptr, false, s_L, sc);
 }
 
@@ -1956,7 +1948,6 @@ __global__ __launch_bounds__(MGX_WAVE, WPS) void feautrier_batch_kernel(
 {
     mgx_ref_tables_init();
     extern __shared__ unsigned char smem[];
-    const double *s_erf = nullptr; /* erf needs no table */
     __shared__ uint32_t s_item;
     const uint32_t lane = threadIdx.x;
     for (;;) {
@@ -1975,7 +1966,7 @@ __global__ __launch_bounds__(MGX_WAVE, WPS) void feautrier_batch_kernel(
         double *Lm = lam ? lam[it.model] : nullptr;
         const size_t o = it.origin;
         const bool whole = it.rr0 == 0 && it.rr1 == kp.m.hnrays;
-        if (solve_origin<APPROX, PREC>(kp, it.origin, it.rr0, it.rr1, smem, s_erf, nullptr,
+        if (solve_origin<APPROX, PREC>(kp, it.origin, it.rr0, it.rr1, smem, nullptr,
                                        Lm != nullptr, s_J, Jm + o * F, !whole, s_L))
             return;
         __syncthreads();
@@ -2820,7 +2811,6 @@ __global__ __launch_bounds__(MGX_WAVE) void image_ray_kernel(const KParams *__re
     mgx_ref_tables_init();
     const KParams &kp = *kpp;
     extern __shared__ unsigned char smem[];
-    const double *s_erf = nullptr; /* erf needs no table */
     const mgx_model &m = kp.m;
     const uint32_t lane = threadIdx.x;
     const uint32_t F = m.nfreqs;
@@ -2873,7 +2863,7 @@ __global__ __launch_bounds__(MGX_WAVE) void image_ray_kernel(const KParams *__re
             auto cross = [&](const Entry &nx, double dz) {
                 PointEC ec_nx = {0.0, 0.0, false};
                 double dtau, S_cu, S_nx;
-                segment<APPROX, PREC>(kp, s_erf, ol, prev, nx, dz, freq, line, ec_prev, ec_nx,
+                segment<APPROX, PREC>(kp, ol, prev, nx, dz, freq, line, ec_prev, ec_nx,
                                       dtau, S_cu, S_nx);
                 if constexpr (KIND == IMG_OPTICAL_DEPTH)
                     tau += dtau;
