@@ -1072,8 +1072,8 @@ __host__ __device__ inline size_t solve_lds_bytes(uint32_t cap, uint32_t stage, 
 constexpr uint32_t kStageMin = 3;
 constexpr size_t kStaticLds = MGX_REF_LDS_TABLE_BYTES + 64;
 constexpr size_t kReservedLds = 2048;
-static_assert(kStaticLds + 2 * (kStageMin * (sizeof(StagedEntry) + sizeof(EntryGrad)) + sizeof(GroupRay) + sizeof(WindowLine)) +
-                      16 <= kReservedLds, "reserved LDS");
+static_assert(kStaticLds + 2 * (kStageMin * (sizeof(StagedEntry) + sizeof(EntryGrad)) + sizeof(GroupRay) +
+                                (kStageMin - 2) * sizeof(WindowLine)) + 16 <= kReservedLds, "reserved LDS");
 
 /* J stays in LDS while the whole LDS of a workgroup fits the share of a CU's
    160 KiB that the register-limited occupancy (MGX_SOLVE_WAVES_PER_SIMD waves on
@@ -1202,8 +1202,8 @@ __device__ __forceinline__ void staged_sweep(const KParams &kp, unsigned char *s
             PointEC ec_in = {0.0, 0.0, false};
             double dtau, S_out, S_in, raw, dop;
             const bool on = k0 + j <= n;
-            staged_segment<APPROX, PREC, WIDE>(kp, g, lines, window_lines(count), bin, eo, ei, on, out, ec_out, ec_in, dtau,
-                                         S_out, S_in, raw, dop);
+            staged_segment<APPROX, PREC, WIDE>(kp, g, lines, window_lines(count), bin, eo, ei, on, out, ec_out,
+                                               ec_in, dtau, S_out, S_in, raw, dop);
             if (!on) continue;
             if constexpr (METHOD == METHOD_TAU) {
                 sw.Y += dtau;
@@ -3322,7 +3322,8 @@ const uint32_t kMaxCap = 8192; /* walk steps per half ray: a ceiling above any L
 /*
  * State shared by the solver's two translation units: this file, and
  * mgx_adjoint.hip, which compiles it again with MGX_ADJOINT_TU for the adjoint
- * entry points (so that the two halves of the kernels compile side by side).  Kernel timing, the per-call workspace and the walk-capacity hints are
+ * entry points (so that the two halves of the kernels compile side by side).
+ * Kernel timing, the per-call workspace and the walk-capacity hints are
  * defined here and declared in the adjoint unit.
  */
 #ifdef MGX_ADJOINT_TU

@@ -302,10 +302,11 @@ __device__ inline void stage_chunk(const KParams &kp, unsigned char *smem, const
 }
 
 /*
- * Windows that hold several lines.  The lanes of a group take nw (kWindowLines, fewer
- * where LDS is short) lines of the sorted list side by side: those inside the union of the bins' windows have their data
- * gathered and interpolated at the segment's ends (or at one entry) by one lane each and
- * left in LDS, from where every bin adds up the lines of its own window, in order.
+ * Windows that hold several lines.  The lanes of a group take nw (kWindowLines, fewer where
+ * LDS is short) lines of the sorted list side by side: those inside the union of the bins'
+ * windows have their data gathered and interpolated at the segment's ends (or at one entry) by
+ * one lane each and left in LDS, from where every bin adds up the lines of its own window, in
+ * order.
  */
 constexpr uint32_t kWindowLines = 16;
 
