@@ -16,8 +16,8 @@
  * Before, a bin's reverse of an interpolated segment recomputed its erf and powf terms and
  * added to four points by itself, behind a call, and every walk step summed its points over
  * the group.  Measured, forward and backward: J of the 24^3 wind (16% of the entries
- * interpolated), FP64, 33.8 -> 20.1 ms; (log n, T) gradient of a 128^2 image of a clumpy 24^3
- * wind 4.8 -> 2.8 ms.  Four tape words instead of five, two for the half of the segments that
+ * interpolated), FP64, 33.6 -> 19.0 ms; (log n, T) gradient of a 128^2 image of a clumpy 24^3
+ * wind 4.2 -> 2.5 ms.  Four tape words instead of five, two for the half of the segments that
  * no line reaches; the tape and the reverse's own arithmetic bind what is left.
  */
 

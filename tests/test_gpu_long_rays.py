@@ -1,10 +1,11 @@
 """Rays longer than the kernels' first walk buffer.
 
 The reference sizes its scratch with a tracing pass; the solves here size the
-LDS walk buffer from a walk-only pass (the longest half ray of the model) and
-the imager and adjoints start at 128 steps and relaunch with twice the buffer
-when a walk does not fit, up to what the device's LDS per workgroup holds
-(160 KiB on gfx950: about 3360 steps), then fail with MGX_E_RAY_LENGTH.  On a
+LDS walk buffer from a walk-only pass (the longest half ray of the model), as
+does the adjoint of J where no solve came before, and the imager and its adjoint
+start at 128 steps and relaunch with what a walk that does not fit needs, up to
+what the device's LDS per workgroup holds (160 KiB on gfx950: about 3360 steps),
+then fail with MGX_E_RAY_LENGTH.  On a
 1D chain of 1000 points the half rays from the ends have 999 steps: the forward
 solve (u, J and Lambda within 1e-10 of the oracle) and the adjoint (whose
 per-wave tape also grows) must come out as on short rays, and so must the
