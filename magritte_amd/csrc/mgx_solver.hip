@@ -3843,13 +3843,23 @@ int run_J_adjoint_k(hipStream_t st, DevBuffers &b, KParams &kp, const double *J_
     const uint32_t P = kp.m.npoints;
     /* few origins leave the GPU idle (3072 waves are resident at 3 per SIMD) or end with a
        long tail: their ray pairs go to several waves, into about kAdjointItems items.  Many
-       more would wait for the counter that hands them out, about 40 ns each.  Forward and
+       more would wait for the counter that hands them out, 40 to 60 ns each.  Forward and
        adjoint measured by whole origins, this way and by single pairs (6 pairs): 6^3 1060,
        590 and 600 us; 11^3 1340, 970 and 1130; 21^3 with two lines 3120, 3080 and 5110;
-       22^3 9.54, 9.40 and 9.65 ms; 24^3 20.0, 19.8 and 19.7 ms */
-    constexpr uint32_t kAdjointItems = 16384;
+       22^3 9.54, 9.40 and 9.65 ms; 24^3 20.0, 19.8 and 19.7 ms.  Items of a line or two wait
+       even then, where there are more than resident waves; they take the pairs of
+       kAdjointSlots line slots.  The adjoint by single pairs, by two, three and six, us: 12^3
+       with one line 626, 365, 298 and 364, with two lines 709, 444, 385 and 550, four 803, 636,
+       629 and 954, nine 1245, 1235, 1318 and 2085; 20^3 with one line 3077, 1776, 1397 and 1332 */
+    constexpr uint32_t kAdjointItems = 16384, kAdjointWaves = 3072, kAdjointSlots = 5;
+    const uint32_t R = kp.m.hnrays;
     const uint64_t want = (kAdjointItems + (uint64_t)P - 1) / P;
-    const uint32_t per = want >= kp.m.hnrays ? 1 : (uint32_t)((kp.m.hnrays + want - 1) / want);
+    uint32_t per = want >= R ? 1 : (uint32_t)((R + want - 1) / want);
+    const uint32_t light = (kAdjointSlots + kp.nslots - 1) / kp.nslots;
+    if ((uint64_t)P * R > kAdjointWaves && per < light) {
+        const uint32_t groups = (R + light - 1) / light;
+        per = (R + groups - 1) / groups;
+    }
     const uint32_t items = P * ((kp.m.hnrays + per - 1) / per);
     return adjoint_launch(
         st, b, kp, walk_key(kp.m), true, d_eps, d_kap, d_iw, (size_t)P * kp.m.nlines, 2,

@@ -72,10 +72,10 @@ def test_ray_pair_parts_and_their_workspace(nrays):
             assert (got[k] == want[k]).all(), k
 
 
-@pytest.mark.parametrize("n_edge,nrays", [(3, 12), (15, 48), (26, 12)])
+@pytest.mark.parametrize("n_edge,nrays", [(3, 12), (12, 12), (15, 48), (26, 12)])
 def test_adjoint_ray_pair_items(n_edge, nrays):
-    """the J adjoint takes one ray pair per item, five with a remainder of four, or an
-    origin's six; the sums' order differs: 1e-9 relative, as the other gradient tests, and
+    """the J adjoint takes one ray pair per item, half an origin's of one line, five with a
+    remainder of four, or an origin's six; the sums' order differs: 1e-9 relative, as the other gradient tests, and
     1e-10 of the largest where contributions of both signs cancel"""
     import torch
 
